@@ -1050,6 +1050,25 @@ static uint32_t half_weight(float w) {
 // contiguous eighth per XCD (band 0).
 constexpr uint32_t kTraceBandRows = 1;
 
+// Wavefronts that share a 64-pixel block's cones (k_trace), for a launch of `blocks` such
+// blocks. With few blocks a third wavefront shortens the launch, until the specular cone
+// alone sets its length (room, 9 + 1 cones, FP16 x-pair: 96 x 54 pixels 104 us with one, 60
+// with two, 47 with three, 48 with five; 640 x 360 147 / 125 / 116; 1280 x 720 359 / 344 /
+// 345). With many, two suffice and the third only costs its setup (4 + 1 cones at 1080p,
+// FP32: 481 us with two, 530 with three). But a block's results take 1 KB of LDS per
+// diffuse cone, and seven wavefronts a SIMD must fit beside them: two a block up to 10
+// cones, four beyond (16 + 1 cones at 1080p, FP32: 1.71 ms with two, 1.37 with three, 1.29
+// with four). Sorted pixels take four too: their footprints are scattered, and the fewer
+// blocks a CU holds the more of them its L1 keeps (a frame of 16 scenes in Morton order,
+// FP16: 3.69 ms with two, 3.63 with three, 3.54 with four; 3.61 with a wavefront each).
+constexpr size_t kManyTraceBlocks = 12000;
+// From here a launch fills the chip (k_trace's registers: trace_waves).
+constexpr size_t kFullTraceBlocks = 5000;
+uint32_t trace_wavefronts(size_t blocks, uint32_t cones, uint32_t diffuse, bool sorted) {
+  const uint32_t w = sorted || diffuse > 10 ? 4u : blocks < kManyTraceBlocks ? 3u : 2u;
+  return std::max(1u, std::min(w, cones));
+}
+
 // March schedule of a cone whose sample distances do not depend on the pixel (a fixed
 // aperture): the per-pixel recurrence of the cone march evaluated once, in FP32 -- diameter
 // d = max(h, 2 t tan), level max(0, log2(d / h)), next t = t + step d -- while
@@ -1100,6 +1119,9 @@ int trace_batch(vgi_context* ctx, const vgi_trace_item* items, uint32_t count, v
     size_t o_params, o_blocks, o_seg, o_sched, nblocks, entries, nsched;
     bool buffer_path;
     uint32_t band;  // work items an XCD takes in a row (k_trace's block order)
+    uint32_t waves, max_diffuse;
+    size_t items;   // screen tiles
+    bool full;
   };
   // per item: its parameters and the schedules of its fixed-aperture cones
   std::vector<TraceParams> tp(count);
@@ -1109,28 +1131,34 @@ int trace_batch(vgi_context* ctx, const vgi_trace_item* items, uint32_t count, v
     if (tp[i].num_diffuse > 0) march_schedule(tp[i], tp[i].tan_d, sched[2 * i]);
     if (tp[i].specular && !tp[i].rough) march_schedule(tp[i], tp[i].tan_s, sched[2 * i + 1]);
   }
+  const uint32_t sub_shift = ilog2((tn.tile_w / 8) * (tn.tile_h / 8));  // 8x8 blocks per tile
   std::vector<Launch> launches;
   Carve cv;
   size_t max_entries = 0;
   for (uint32_t p = 0; p < kPrecisions; p++) {
     if (group[p].empty()) continue;
-    Launch L{p, (uint32_t)group[p].size(), 0, 0, 0, 0, 0, 0, 0, tn.address_mode == VGI_ADDRESS_AUTO, 0};
-    // bands of kTraceBandRows rows of the first item's tiles
-    L.band = morton ? 0u : kTraceBandRows * (uint32_t)ceil_div(items[group[p][0]].gbuffer.width, tn.tile_w);
+    Launch L{p, (uint32_t)group[p].size(), 0, 0, 0, 0, 0, 0, 0, tn.address_mode == VGI_ADDRESS_AUTO, 0, 0, 0, 0, false};
+    uint32_t cones = 0;
     for (uint32_t i : group[p]) {
       L.nsched += sched[2 * i].size() + sched[2 * i + 1].size();
       const vgi_gbuffer& gb = items[i].gbuffer;
+      L.max_diffuse = std::max(L.max_diffuse, tp[i].num_diffuse);
+      cones = std::max(cones, tp[i].num_diffuse + (tp[i].specular && tp[i].out_s ? 1u : 0u));
       if (morton) L.entries += align_up((size_t)gb.width * gb.height, kSortBlock);
-      else L.nblocks += (size_t)ceil_div(gb.width, tn.tile_w) * ceil_div(gb.height, tn.tile_h);
+      else L.items += (size_t)tp[i].tiles_x * tp[i].tiles_y;
       for (uint32_t k = 0; k < items[i].scene->grid.levels; k++)
         // buffer gathers: unsigned 32-bit byte offsets and a 32-bit record count
         L.buffer_path = L.buffer_path && items[i].scene->level_bytes[k] < 0xFFFFFFF0ull;
     }
-    if (morton) L.nblocks = L.entries / kSortBlock;
+    L.nblocks = morton ? L.entries / 64 : L.items << sub_shift;
+    // bands of kTraceBandRows rows of the first item's tiles
+    L.band = morton ? 0u : kTraceBandRows * (tp[group[p][0]].tiles_x << sub_shift);
+    L.waves = trace_wavefronts(L.nblocks, cones, L.max_diffuse, morton);
+    L.full = L.nblocks >= kFullTraceBlocks;
     if (L.nblocks >= (1ull << 31) || L.entries >= (1ull << 32))
       return fail(VGI_E_RANGE, "trace batch too large (%zu workgroups)", L.nblocks);
     L.o_params = cv.take((size_t)L.nscenes * sizeof(TraceParams));
-    L.o_blocks = cv.take(!morton && L.nscenes > 1 ? L.nblocks * sizeof(uint2) : 0);
+    L.o_blocks = cv.take(!morton && L.nscenes > 1 ? L.items * sizeof(uint2) : 0);
     L.o_seg = cv.take(morton ? ((size_t)L.nscenes + 1) * sizeof(uint32_t) : 0);
     L.o_sched = cv.take(L.nsched * sizeof(SchedEntry));
     max_entries = std::max(max_entries, L.entries);
@@ -1197,6 +1225,10 @@ int trace_batch(vgi_context* ctx, const vgi_trace_item* items, uint32_t count, v
     B.prec = L.prec;
     B.nscenes = L.nscenes;
     B.band = L.band;
+    B.sub_shift = sub_shift;
+    B.waves = L.waves;
+    B.full = L.full ? 1u : 0u;
+    B.max_diffuse = L.max_diffuse;
     if (morton && L.entries > 0) {
       unsigned long long* keys = (unsigned long long*)w->sort_keys;
       uint32_t* pix = (uint32_t*)w->sort_pix;

@@ -9,11 +9,11 @@
 // two adjacent levels), front-to-back compositing C += (1-a) c, a += (1-a) alpha,
 // step t += step_factor * d, stop at max_distance, alpha >= cutoff or the grid boundary.
 //
-// Schedule: a workgroup is one screen tile (8x8, 16x16 or 32x8 pixels; each wavefront an
-// 8x8 block) of one scene of the batch; tiles are dealt to the XCDs in bands of one tile
-// row (neighbouring tiles share that XCD's L2, and every XCD works across the whole
-// screen), and every lane of a wavefront marches the same cone index at the same time,
-// so directions stay coherent across the wavefront.
+// Schedule: a workgroup is one 8x8 pixel block of one scene of the batch; its wavefronts
+// share the block's cones, each marching one cone of all 64 pixels at a time, so directions
+// stay coherent across a wavefront. Blocks follow the screen tiles (8x8, 16x16 or 32x8
+// pixels), which are dealt to the XCDs in bands of one tile row (neighbouring tiles share
+// that XCD's L2, and every XCD works across the whole screen).
 //
 // Gather: a quadrilinear sample is 16 weighted texels, sum_i w_i c_i with the level blend
 // folded into the weights, accumulated in FP32 (FP16 texels feed v_fma_mix directly; no
@@ -31,7 +31,7 @@
 // Morton order (for G-buffers that are not spatially coherent, e.g. points sampled on
 // triangles): k_morton_keys keys every pixel by (scene << 32 | 30-bit Morton code of its
 // position quantized to 1024^3 over the grid), one radix sort orders the batch, and a
-// workgroup then takes 256 consecutive sorted pixels of one scene, so the cones of a
+// workgroup then takes 64 consecutive sorted pixels of one scene, so the cones of a
 // wavefront start close together and share cache lines. Every pixel's result is the
 // same in either order.
 #include <rocprim/device/device_radix_sort.hpp>
@@ -320,23 +320,29 @@ __device__ __forceinline__ void gather_uniform(const TraceParams& P, uint32_t k,
     }
     const __amdgpu_buffer_rsrc_t r =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(L.ptr), 0, (int)L.bytes32, 0x00020000);  // unsigned field
+    // every load is issued before the first is waited for (left to itself the scheduler pairs
+    // them with their uses to save registers, four round trips instead of one)
+    constexpr int kRowLoads = PREC == VGI_PREC_FP32 ? 2 : 1;
+    vgi_u32x4 v[4 * kRowLoads];
+  #pragma unroll
+    for (int q = 0; q < 4 * kRowLoads; q++) {
+      const auto e = __builtin_amdgcn_raw_buffer_load_b128(r, off + 16u * (q % kRowLoads), soff[q / kRowLoads], 0);
+      v[q] = vgi_u32x4{e[0], e[1], e[2], e[3]};
+    }
+    __builtin_amdgcn_sched_barrier(0);
   #pragma unroll
     for (int q = 0; q < 4; q++) {
       const float wz = q < 2 ? f.wz0 : f.wz1;
       if constexpr (PREC == VGI_PREC_FP32) {
-        const auto a = __builtin_amdgcn_raw_buffer_load_b128(r, off, soff[q], 0);
-        const auto b = __builtin_amdgcn_raw_buffer_load_b128(r, off + 16, soff[q], 0);
-        const uint32_t a0 = a[0], a1 = a[1], a2 = a[2], a3 = a[3];
-        const uint32_t b0 = b[0], b1 = b[1], b2 = b[2], b3 = b[3];
-        Acc<VGI_PREC_FP32>::add(acc, wxy[q][0] * wz, a0, a1, a2, a3);
-        Acc<VGI_PREC_FP32>::add(acc, wxy[q][1] * wz, b0, b1, b2, b3);
-        abits |= a3 | b3;
+        const vgi_u32x4 a = v[2 * q], b = v[2 * q + 1];
+        Acc<VGI_PREC_FP32>::add(acc, wxy[q][0] * wz, a[0], a[1], a[2], a[3]);
+        Acc<VGI_PREC_FP32>::add(acc, wxy[q][1] * wz, b[0], b[1], b[2], b[3]);
+        abits |= a[3] | b[3];
       } else {
-        const auto a = __builtin_amdgcn_raw_buffer_load_b128(r, off, soff[q], 0);
-        const uint32_t a0 = a[0], a1 = a[1], a2 = a[2], a3 = a[3];
-        Acc<PREC>::add(acc, wxy[q][0] * wz, a0, a1);
-        Acc<PREC>::add(acc, wxy[q][1] * wz, a2, a3);
-        abits |= (a1 | a3) & 0xFFFF0000u;  // opacity is the high half
+        const vgi_u32x4 a = v[q];
+        Acc<PREC>::add(acc, wxy[q][0] * wz, a[0], a[1]);
+        Acc<PREC>::add(acc, wxy[q][1] * wz, a[2], a[3]);
+        abits |= (a[1] | a[3]) & 0xFFFF0000u;  // opacity is the high half
       }
     }
   }
@@ -410,7 +416,7 @@ __device__ __forceinline__ bool inside_grid(float ux, float uy, float uz, float 
 
 // cone origin in level-0 voxel units, with -0.0 made +0.0 (inside_grid relies on it)
 __device__ __forceinline__ float cone_origin(float o, float origin, float inv_h) {
-  return (o - origin) * inv_h + 0.0f;
+  return fmaf(o - origin, inv_h, 0.0f);
 }
 
 // One fixed-aperture cone: its samples (distance, levels, level weights) come from the
@@ -461,6 +467,34 @@ __device__ __forceinline__ float4 cone_march_fixed(const TraceParams& P, const S
   return make_float4(cr, cg, cb, a);
 }
 
+// One sample at a per-lane level lvl (top: the top level's number).
+template <int PREC, bool BUF>
+__device__ __forceinline__ void lane_sample(const TraceParams& P, float ux, float uy, float uz, float lvl, float top,
+                                            float4& s, uint32_t& count) {
+  uint32_t abits = 0;
+  if (lvl >= top) {
+    if constexpr (BUF) gather_uniform<PREC, true>(P, P.levels - 1, ux, uy, uz, 1.0f, kHalfOne, s, abits);
+    else gather_lane<PREC, true>(P, P.levels - 1, ux, uy, uz, 1.0f, kHalfOne, s, abits);
+    count += 1;
+  } else {
+    const float fl = floorf(lvl);
+    const float fr = lvl - fl, gr = 1.0f - fr;
+    const uint32_t l0 = (uint32_t)fl;
+    const uint32_t hfr = half_weight(fr), hgr = half_weight(gr);  // used by the FP16 x-pair form
+    // per-lane schedules usually still agree on the level across the wavefront: then the
+    // level's descriptor and pitches are scalars
+    const uint32_t lu = __builtin_amdgcn_readfirstlane(l0);
+    if (BUF && __all(l0 == lu)) {
+      gather_uniform<PREC, true>(P, lu + 1, ux, uy, uz, fr, hfr, s, abits);
+      if (abits || !skip_fine_ok<PREC>(lu)) gather_uniform<PREC, false>(P, lu, ux, uy, uz, gr, hgr, s, abits);
+    } else {
+      gather_lane<PREC, true>(P, l0 + 1, ux, uy, uz, fr, hfr, s, abits);
+      if (abits || !skip_fine_ok<PREC>(l0)) gather_lane<PREC, false>(P, l0, ux, uy, uz, gr, hgr, s, abits);
+    }
+    count += 2;
+  }
+}
+
 // One cone with a per-pixel aperture (the roughness-driven specular cone), or any cone when
 // a level is too large for 32-bit buffer offsets (BUF false: every gather then uses 64-bit
 // addresses): sample diameter d(t) = max(h, 2 t tan), level log2(d / h), step
@@ -487,184 +521,235 @@ __device__ __forceinline__ float4 cone_march_lane(const TraceParams& P, float ox
     const float diam = fmaxf(h, 2.0f * t * tan_half);
     const float lvl = fmaxf(0.0f, __log2f(diam * inv_h));
     float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-    uint32_t abits = 0;
-    if (lvl >= top) {
-      if constexpr (BUF) gather_uniform<PREC, true>(P, P.levels - 1, ux, uy, uz, 1.0f, kHalfOne, s, abits);
-      else gather_lane<PREC, true>(P, P.levels - 1, ux, uy, uz, 1.0f, kHalfOne, s, abits);
-      count += 1;
-    } else {
-      const float fl = floorf(lvl);
-      const float fr = lvl - fl, gr = 1.0f - fr;
-      const uint32_t l0 = (uint32_t)fl;
-      const uint32_t hfr = half_weight(fr), hgr = half_weight(gr);  // used by the FP16 x-pair form
-      // per-lane schedules usually still agree on the level across the wavefront: then the
-      // level's descriptor and pitches are scalars
-      const uint32_t lu = __builtin_amdgcn_readfirstlane(l0);
-      if (BUF && __all(l0 == lu)) {
-        gather_uniform<PREC, true>(P, lu + 1, ux, uy, uz, fr, hfr, s, abits);
-        if (abits || !skip_fine_ok<PREC>(lu)) gather_uniform<PREC, false>(P, lu, ux, uy, uz, gr, hgr, s, abits);
-      } else {
-        gather_lane<PREC, true>(P, l0 + 1, ux, uy, uz, fr, hfr, s, abits);
-        if (abits || !skip_fine_ok<PREC>(l0)) gather_lane<PREC, false>(P, l0, ux, uy, uz, gr, hgr, s, abits);
-      }
-      count += 2;
-    }
+    lane_sample<PREC, BUF>(P, ux, uy, uz, lvl, top, s, count);
     composite(s, cr, cg, cb, a);
     if (a >= cutoff) break;
-    t = t + step * diam;
+    t = fmaf(step, diam, t);
   }
   return make_float4(cr, cg, cb, a);
 }
 
-template <int PREC, bool BUF, bool SORTED>
-__global__ __launch_bounds__(256) void k_trace(TraceBatch Bt, const TraceParams* __restrict__ scenes,
-                                               const uint2* __restrict__ blocks,
-                                               const unsigned long long* __restrict__ skeys,
-                                               const uint32_t* __restrict__ spix) {
-  // XCD-aware order: block b runs on XCD b % 8. The batch's work list (tiles of one scene
-  // are consecutive, row-major; sorted runs are consecutive in Morton order) is dealt to
-  // the XCDs in bands of Bt.band consecutive items, XCD x taking bands x, x + 8, ...:
-  // neighbouring items share that XCD's L2, and every XCD draws from the whole list, so
-  // they finish together (one contiguous eighth each left the room's frame with XCD
-  // workloads 20% apart). The items after the last whole round of bands are split into
-  // eight contiguous parts.
-  const uint32_t b = blockIdx.x;
+// Work item of workgroup b in the XCD-aware order: block b runs on XCD b % 8. The batch's
+// work list (tiles of one scene are consecutive, row-major; sorted runs are consecutive in
+// Morton order) is dealt to the XCDs in bands of Bt.band consecutive items, XCD x taking
+// bands x, x + 8, ...: neighbouring items share that XCD's L2, and every XCD draws from the
+// whole list, so they finish together (one contiguous eighth each left the room's frame
+// with XCD workloads 20% apart). The items after the last whole round of bands are split
+// into eight contiguous parts.
+__device__ __forceinline__ uint32_t work_index(const TraceBatch& Bt, uint32_t b) {
   const uint32_t xcd = b & 7u;
   const uint32_t per = Bt.band * 8u, rounds = Bt.band ? Bt.nblocks / per : 0u;
-  uint32_t idx;
   if (b < rounds * per) {
     const uint32_t slot = b >> 3;
-    idx = ((slot / Bt.band) * 8u + xcd) * Bt.band + slot % Bt.band;
-  } else {
-    const uint32_t r = b - rounds * per, n = Bt.nblocks - rounds * per;  // r % 8 == xcd
-    const uint32_t full = n >> 3, rem = n & 7u;
-    idx = rounds * per + xcd * full + (xcd < rem ? xcd : rem) + (r >> 3);
+    return ((slot / Bt.band) * 8u + xcd) * Bt.band + slot % Bt.band;
   }
-  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t r = b - rounds * per, n = Bt.nblocks - rounds * per;  // r % 8 == xcd
+  const uint32_t full = n >> 3, rem = n & 7u;
+  return rounds * per + xcd * full + (xcd < rem ? xcd : rem) + (r >> 3);
+}
+
+// A pixel's cone origin, normal and the quotient of its tangent frame (Duff et al. 2017:
+// ab = -1 / (sign(nz) + nz)), held in LDS for the whole block (word i of lane l at 64 i + l):
+// in registers they would be live across every march.
+enum { kOx, kOy, kOz, kNx, kNy, kNz, kAb, kFrameWords };
+
+// The per-pixel arithmetic below is written with its fused multiply-adds spelled out and
+// contraction off: what the compiler fuses by itself depends on the block that a product
+// lands in, and the outputs' bits must not.
+
+// Writes pixel p's frame to f; false (no cones, outputs zero) for a zero normal.
+__device__ __forceinline__ bool make_frame(const TraceParams& P, size_t p, float* f) {
+#pragma clang fp contract(off)
+  const float px = gld(P.pos + p * 3), py = gld(P.pos + p * 3 + 1), pz = gld(P.pos + p * 3 + 2);
+  const float Nx = gld(P.nrm + p * 3), Ny = gld(P.nrm + p * 3 + 1), Nz = gld(P.nrm + p * 3 + 2);
+  const float len2 = fmaf(Nz, Nz, fmaf(Nx, Nx, Ny * Ny));
+  if (!(len2 > 0.f)) return false;
+  const float inv = 1.0f / __builtin_sqrtf(len2);
+  const float nx = Nx * inv, ny = Ny * inv, nz = Nz * inv;
+  const float off = P.normal_off * P.h;
+  const float sign = copysignf(1.0f, nz);
+  f[64 * kOx] = fmaf(nx, off, px), f[64 * kOy] = fmaf(ny, off, py), f[64 * kOz] = fmaf(nz, off, pz);
+  f[64 * kNx] = nx, f[64 * kNy] = ny, f[64 * kNz] = nz;
+  f[64 * kAb] = -1.0f / (sign + nz);
+  return true;
+}
+
+template <int PREC, bool BUF>
+__device__ __forceinline__ float4 march_diffuse(const TraceParams& P, const float* f, uint32_t c, uint32_t& count) {
+#pragma clang fp contract(off)
+  const float lx = P.dirs[c][0], ly = P.dirs[c][1], lz = P.dirs[c][2];
+  const float nx = f[64 * kNx], ny = f[64 * kNy], nz = f[64 * kNz], ab = f[64 * kAb];
+  // tangent (t0, t1, t2), bitangent (bb, b1, -ny)
+  const float sign = copysignf(1.0f, nz);
+  const float bb = nx * ny * ab;
+  const float t0 = fmaf(sign * nx * nx, ab, 1.0f), t1 = sign * bb, t2 = -sign * nx;
+  const float b1 = fmaf(ny * ny, ab, sign);
+  const float dx = fmaf(nx, lz, fmaf(t0, lx, bb * ly));
+  const float dy = fmaf(ny, lz, fmaf(t1, lx, b1 * ly));
+  const float dz = fmaf(nz, lz, fmaf(t2, lx, -ny * ly));
+  const float ox = f[64 * kOx], oy = f[64 * kOy], oz = f[64 * kOz];
+  return BUF ? cone_march_fixed<PREC>(P, P.sched[0], P.sched_len[0], ox, oy, oz, dx, dy, dz, count)
+             : cone_march_lane<PREC, BUF>(P, ox, oy, oz, dx, dy, dz, P.tan_d, count);
+}
+
+template <int PREC, bool BUF>
+__device__ __forceinline__ float4 march_specular(const TraceParams& P, const float* f, size_t p, uint32_t& count) {
+#pragma clang fp contract(off)
+  const float px = gld(P.pos + p * 3), py = gld(P.pos + p * 3 + 1), pz = gld(P.pos + p * 3 + 2);
+  const float nx = f[64 * kNx], ny = f[64 * kNy], nz = f[64 * kNz];
+  const float vx = P.eye[0] - px, vy = P.eye[1] - py, vz = P.eye[2] - pz;
+  const float vl2 = fmaf(vz, vz, fmaf(vx, vx, vy * vy));
+  const float vi = vl2 > 0.f ? 1.0f / __builtin_sqrtf(vl2) : 0.f;
+  const float ix = -vx * vi, iy = -vy * vi, iz = -vz * vi;
+  const float dn2 = 2.0f * fmaf(nz, iz, fmaf(nx, ix, ny * iy));
+  const float rx = fmaf(-dn2, nx, ix), ry = fmaf(-dn2, ny, iy), rz = fmaf(-dn2, nz, iz);
+  const float ox = f[64 * kOx], oy = f[64 * kOy], oz = f[64 * kOz];
+  if (P.rough) {
+    const float th = fminf(fmaxf(gld(P.rough + p), 0.0087f), 1.0f);
+    return cone_march_lane<PREC, BUF>(P, ox, oy, oz, rx, ry, rz, th, count);
+  }
+  return BUF ? cone_march_fixed<PREC>(P, P.sched[1], P.sched_len[1], ox, oy, oz, rx, ry, rz, count)
+             : cone_march_lane<PREC, BUF>(P, ox, oy, oz, rx, ry, rz, P.tan_s, count);
+}
+
+__device__ __forceinline__ void store_out(float4* out, float4 v) {
+  gst4(out, make_uint4(__builtin_bit_cast(uint32_t, v.x), __builtin_bit_cast(uint32_t, v.y),
+                       __builtin_bit_cast(uint32_t, v.z), __builtin_bit_cast(uint32_t, v.w)));
+}
+
+// Adds the workgroup's gathers to the counter: one global atomic per workgroup (all add to
+// one address).
+__device__ __forceinline__ void add_count(unsigned long long* counter, uint32_t count) {
+  __shared__ unsigned long long s_count[kMaxTraceWaves];
+  unsigned long long c = count;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
+  if ((threadIdx.x & 63u) == 0) s_count[threadIdx.x >> 6] = c;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    unsigned long long t = 0;
+    for (uint32_t i = 0; i < (blockDim.x >> 6); i++) t += s_count[i];
+    atomicAdd(counter, t);
+  }
+}
+
+// Registers: the march is bound by VALU issue and hides its loads behind other wavefronts.
+// With the block's frames in LDS every form but FP32 fits seven wavefronts a SIMD as it is;
+// FP32, whose footprint takes 32 registers, does so with six values in scratch, which pays
+// once a launch fills the chip (room, 1080p: 794 us against 892 with four wavefronts; 860 x
+// 480 228 / 239) and not before (640 x 360: 172 / 164; 96 x 54: 77 / 60). Eight wavefronts
+// split the footprint's loads into several round trips (incoherent G-buffers 15% slower).
+constexpr int trace_waves(int prec, bool full) { return prec == VGI_PREC_FP32 && !full ? 4 : 7; }
+
+// The cones of 64 pixels (an 8x8 block, or 64 sorted ones) shared by the wavefronts of one
+// workgroup: a wavefront takes the next cone of the whole block (the specular one first, it
+// marches farthest) until none is left; the diffuse results meet in LDS and are summed in
+// cone order, so an output does not depend on who marched what. One wavefront per block,
+// marching every cone in turn, takes as long as the block's longest pixels however small the
+// launch (96 x 54 pixels, 9 + 1 cones: 104 us, 47 with three wavefronts), and of a large
+// launch keeps twice the blocks resident per CU, whose footprints share its L1 (1280 x 720:
+// FP32 439 -> 388 us, FP16 436 -> 410, BF16 470 -> 427, FP16 x-pair 364 -> 341).
+template <int PREC, bool BUF, bool SORTED, bool FULL>
+__global__ __launch_bounds__(64 * kMaxTraceWaves) __attribute__((amdgpu_waves_per_eu(trace_waves(PREC, FULL))))
+void k_trace(TraceBatch Bt, const TraceParams* __restrict__ scenes, const uint2* __restrict__ blocks,
+             const unsigned long long* __restrict__ skeys, const uint32_t* __restrict__ spix) {
+  extern __shared__ float4 s_cone[];  // diffuse cone c of lane l at 64 c + l
+  __shared__ float s_frame[64 * kFrameWords];
+  __shared__ uint32_t s_next;
+  __shared__ uint64_t s_cones;  // the block's pixels that have cones
+  const uint32_t idx = work_index(Bt, blockIdx.x);
+  const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t nwaves = blockDim.x >> 6;
+  if (threadIdx.x == 0) s_next = nwaves;
   uint32_t scene;
   size_t p;
   bool active;
   if constexpr (SORTED) {
-    const size_t e = (size_t)idx * kSortBlock + threadIdx.x;
-    scene = (uint32_t)(skeys[(size_t)idx * kSortBlock] >> 32);  // a run never spans two scenes
+    const size_t e = (size_t)idx * 64u + lane;
+    scene = (uint32_t)(skeys[(size_t)idx * 64u] >> 32);  // a scene's entries are a multiple of 64
     const uint32_t q = gld(spix + e);
     active = q != kNoPixel;
     p = q;
   } else {
-    const uint2 st = Bt.nscenes == 1 ? make_uint2(0u, idx) : blocks[idx];
+    // a tile's 8x8 blocks are consecutive work items
+    const uint32_t sub = idx & ((1u << Bt.sub_shift) - 1u), item = idx >> Bt.sub_shift;
+    const uint2 st = Bt.nscenes == 1 ? make_uint2(0u, item) : blocks[item];
     scene = st.x;
     const TraceParams& T = scenes[scene];
-    const uint32_t tile = st.y;
-    const uint32_t tx = tile % T.tiles_x, ty = tile / T.tiles_x;
-    const uint32_t wave = threadIdx.x >> 6;
-    const uint32_t wpr = Bt.tile_w >> 3;  // 8x8 wave blocks per tile row
-    const uint32_t px = tx * Bt.tile_w + (wave % wpr) * 8 + (lane & 7u);
-    const uint32_t py = ty * Bt.tile_h + (wave / wpr) * 8 + (lane >> 3);
+    const uint32_t tx = st.y % T.tiles_x, ty = st.y / T.tiles_x;
+    const uint32_t bw = Bt.tile_w >> 3;  // 1, 2 or 4 blocks per tile row
+    const uint32_t px = tx * Bt.tile_w + (sub & (bw - 1u)) * 8u + (lane & 7u);
+    const uint32_t py = ty * Bt.tile_h + (sub / bw) * 8u + (lane >> 3);
     active = px < T.width && py < T.height;
     p = (size_t)py * T.width + px;
   }
   const TraceParams& P = scenes[scene];
   uint32_t count = 0;
-  if (active) {
-    const float Px = gld(P.pos + p * 3), Py = gld(P.pos + p * 3 + 1), Pz = gld(P.pos + p * 3 + 2);
-    const float Nx = gld(P.nrm + p * 3), Ny = gld(P.nrm + p * 3 + 1), Nz = gld(P.nrm + p * 3 + 2);
-    const float len2 = (Nx * Nx + Ny * Ny) + Nz * Nz;
-    float4 od = make_float4(0.f, 0.f, 0.f, 0.f), os = make_float4(0.f, 0.f, 0.f, 0.f);
-    if (len2 > 0.f) {
-      const float inv = 1.0f / __builtin_sqrtf(len2);
-      const float nx = Nx * inv, ny = Ny * inv, nz = Nz * inv;
-      const float off = P.normal_off * P.h;
-      const float ox = Px + nx * off, oy = Py + ny * off, oz = Pz + nz * off;
-      // orthonormal basis (Duff et al. 2017)
-      const float sign = copysignf(1.0f, nz);
-      const float ab = -1.0f / (sign + nz);
-      const float bb = nx * ny * ab;
-      const float t0 = 1.0f + sign * nx * nx * ab, t1 = sign * bb, t2 = -sign * nx;
-      const float b0 = bb, b1 = sign + ny * ny * ab, b2 = -ny;
-      float ar = 0.f, ag = 0.f, abl = 0.f, aa = 0.f;
+  const float* frame = s_frame + lane;
+  if (wave == 0) {
+    const uint64_t m = __ballot(active && make_frame(P, p, s_frame + lane));
+    if (lane == 0) s_cones = m;
+  }
+  const bool spec = P.out_s && P.specular;
+  const uint32_t ntask = P.num_diffuse + (spec ? 1u : 0u);
+  __syncthreads();
+  const bool cones = (s_cones >> lane) & 1u;
+  for (uint32_t k = wave; k < ntask;) {
+    const uint32_t c = spec ? k - 1u : k;  // diffuse cone, or all ones for the specular cone
+    if (cones) {
+      if (c == ~0u) store_out(P.out_s + p, march_specular<PREC, BUF>(P, frame, p, count));
+      else s_cone[64u * c + lane] = march_diffuse<PREC, BUF>(P, frame, c, count);
+    }
+    uint32_t next = 0;
+    if (lane == 0) next = atomicAdd(&s_next, 1u);
+    k = __builtin_amdgcn_readfirstlane(next);
+  }
+  __syncthreads();
+  if (wave == 0 && active) {
+    float4 od = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (cones) {
+      float4 s = od;
       for (uint32_t c = 0; c < P.num_diffuse; c++) {
-        const float lx = P.dirs[c][0], ly = P.dirs[c][1], lz = P.dirs[c][2];
-        const float dx = (t0 * lx + b0 * ly) + nx * lz;
-        const float dy = (t1 * lx + b1 * ly) + ny * lz;
-        const float dz = (t2 * lx + b2 * ly) + nz * lz;
-        const float4 r = BUF ? cone_march_fixed<PREC>(P, P.sched[0], P.sched_len[0], ox, oy, oz, dx, dy, dz, count)
-                             : cone_march_lane<PREC, BUF>(P, ox, oy, oz, dx, dy, dz, P.tan_d, count);
+        const float4 r = s_cone[64u * c + lane];
         const float wc = P.w[c];
-        ar = fmaf(wc, r.x, ar);
-        ag = fmaf(wc, r.y, ag);
-        abl = fmaf(wc, r.z, abl);
-        aa = fmaf(wc, r.w, aa);
+        s.x = fmaf(wc, r.x, s.x);
+        s.y = fmaf(wc, r.y, s.y);
+        s.z = fmaf(wc, r.z, s.z);
+        s.w = fmaf(wc, r.w, s.w);
       }
-      od = make_float4(ar, ag, abl, 1.0f - aa);
-      if (P.out_s && P.specular) {
-        const float vx = P.eye[0] - Px, vy = P.eye[1] - Py, vz = P.eye[2] - Pz;
-        const float vl2 = (vx * vx + vy * vy) + vz * vz;
-        const float vi = vl2 > 0.f ? 1.0f / __builtin_sqrtf(vl2) : 0.f;
-        const float ix = -vx * vi, iy = -vy * vi, iz = -vz * vi;
-        const float dn = (nx * ix + ny * iy) + nz * iz;
-        const float rx = ix - 2.0f * dn * nx, ry = iy - 2.0f * dn * ny, rz = iz - 2.0f * dn * nz;
-        if (P.rough) {
-          const float th = fminf(fmaxf(gld(P.rough + p), 0.0087f), 1.0f);
-          os = cone_march_lane<PREC, BUF>(P, ox, oy, oz, rx, ry, rz, th, count);
-        } else {
-          os = BUF ? cone_march_fixed<PREC>(P, P.sched[1], P.sched_len[1], ox, oy, oz, rx, ry, rz, count)
-                   : cone_march_lane<PREC, BUF>(P, ox, oy, oz, rx, ry, rz, P.tan_s, count);
-        }
-      }
+      od = make_float4(s.x, s.y, s.z, 1.0f - s.w);
     }
-    gst4(P.out_d + p, make_uint4(__builtin_bit_cast(uint32_t, od.x), __builtin_bit_cast(uint32_t, od.y),
-                                 __builtin_bit_cast(uint32_t, od.z), __builtin_bit_cast(uint32_t, od.w)));
-    if (P.out_s)
-      gst4(P.out_s + p, make_uint4(__builtin_bit_cast(uint32_t, os.x), __builtin_bit_cast(uint32_t, os.y),
-                                   __builtin_bit_cast(uint32_t, os.z), __builtin_bit_cast(uint32_t, os.w)));
+    store_out(P.out_d + p, od);
+    if (P.out_s && !(cones && spec)) store_out(P.out_s + p, make_float4(0.f, 0.f, 0.f, 0.f));
   }
-  if (Bt.counter) {  // one global atomic per workgroup (all add to one address)
-    __shared__ unsigned long long s_count[4];
-    unsigned long long c = count;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
-    if (lane == 0) s_count[threadIdx.x >> 6] = c;
-    __syncthreads();
-    if (threadIdx.x == 0) {  // workgroups of 64 (8x8 tiles) or 256 threads
-      unsigned long long t = 0;
-      for (uint32_t i = 0; i < (blockDim.x >> 6); i++) t += s_count[i];
-      atomicAdd(Bt.counter, t);
-    }
-  }
+  if (Bt.counter) add_count(Bt.counter, count);
 }
 
 template <int PREC, bool SORTED>
-static void launch_trace_prec(const TraceBatch& B, bool buffer_path, dim3 grid, dim3 block, hipStream_t s) {
-  if (buffer_path)
-    hipLaunchKernelGGL((k_trace<PREC, true, SORTED>), grid, block, 0, s, B, B.scenes, B.blocks, B.skeys, B.spix);
-  else
-    hipLaunchKernelGGL((k_trace<PREC, false, SORTED>), grid, block, 0, s, B, B.scenes, B.blocks, B.skeys, B.spix);
+static void launch_trace_prec(const TraceBatch& B, bool buffer_path, hipStream_t s) {
+  const dim3 grid(B.nblocks), block(64u * B.waves);
+  const uint32_t lds = B.max_diffuse * 64u * (uint32_t)sizeof(float4);
+#define VGI_LAUNCH(BUF, FULL) \
+  hipLaunchKernelGGL((k_trace<PREC, BUF, SORTED, FULL>), grid, block, lds, s, B, B.scenes, B.blocks, B.skeys, B.spix)
+  if (!buffer_path) VGI_LAUNCH(false, false);
+  else if (PREC == VGI_PREC_FP32 && B.full) VGI_LAUNCH(true, PREC == VGI_PREC_FP32);  // (other forms: one variant)
+  else VGI_LAUNCH(true, false);
+#undef VGI_LAUNCH
 }
 
 hipError_t launch_trace(const TraceBatch& B, bool buffer_path, hipStream_t s) {
   if (B.nblocks == 0) return hipSuccess;
   const bool sorted = B.skeys != nullptr;
-  const dim3 block(sorted ? kSortBlock : B.tile_w * B.tile_h), grid(B.nblocks);
+#define VGI_LAUNCH(PREC) \
+  (sorted ? launch_trace_prec<PREC, true>(B, buffer_path, s) : launch_trace_prec<PREC, false>(B, buffer_path, s))
   switch (B.prec) {
-    case VGI_PREC_FP32:
-      if (sorted) launch_trace_prec<VGI_PREC_FP32, true>(B, buffer_path, grid, block, s);
-      else launch_trace_prec<VGI_PREC_FP32, false>(B, buffer_path, grid, block, s);
-      break;
-    case VGI_PREC_FP16:
-      if (sorted) launch_trace_prec<VGI_PREC_FP16, true>(B, buffer_path, grid, block, s);
-      else launch_trace_prec<VGI_PREC_FP16, false>(B, buffer_path, grid, block, s);
-      break;
-    case VGI_PREC_BF16:
-      if (sorted) launch_trace_prec<VGI_PREC_BF16, true>(B, buffer_path, grid, block, s);
-      else launch_trace_prec<VGI_PREC_BF16, false>(B, buffer_path, grid, block, s);
-      break;
-    case VGI_PREC_FP16X2:
-      if (sorted) launch_trace_prec<VGI_PREC_FP16X2, true>(B, buffer_path, grid, block, s);
-      else launch_trace_prec<VGI_PREC_FP16X2, false>(B, buffer_path, grid, block, s);
-      break;
-    default:
-      return hipErrorInvalidValue;
+    case VGI_PREC_FP32: VGI_LAUNCH(VGI_PREC_FP32); break;
+    case VGI_PREC_FP16: VGI_LAUNCH(VGI_PREC_FP16); break;
+    case VGI_PREC_BF16: VGI_LAUNCH(VGI_PREC_BF16); break;
+    case VGI_PREC_FP16X2: VGI_LAUNCH(VGI_PREC_FP16X2); break;
+    default: return hipErrorInvalidValue;
   }
+#undef VGI_LAUNCH
   return hipGetLastError();
 }
 

@@ -266,7 +266,7 @@ struct TraceParams {
 
 struct TraceBatch {
   const TraceParams* scenes;
-  const uint2* blocks;            // (scene, tile) per workgroup (screen-tile order, > 1 scene)
+  const uint2* blocks;            // (scene, tile) per screen tile (screen-tile order, > 1 scene)
   unsigned long long* counter;    // trilinear gathers (may be null)
   // Morton order (null in screen-tile order): the batch's pixels sorted by
   // (scene << 32 | Morton code of the position); scene s owns entries [seg[s], seg[s+1]),
@@ -278,11 +278,16 @@ struct TraceBatch {
   uint32_t tile_w, tile_h;
   uint32_t prec;
   uint32_t nscenes;
-  uint32_t band;  // work items (tiles or sorted runs) an XCD takes in a row before the next XCD's
+  uint32_t band;  // work items (64-pixel blocks) an XCD takes in a row before the next XCD's
+  uint32_t sub_shift;    // log2 of the 8x8 blocks in a screen tile
+  uint32_t waves;        // wavefronts that share a 64-pixel block's cones
+  uint32_t full;         // the launch has wavefronts to fill every SIMD (trace_waves)
+  uint32_t max_diffuse;  // most diffuse cones of the launch's items (the LDS it takes)
 };
 
 constexpr uint32_t kNoPixel = 0xFFFFFFFFu;
-constexpr uint32_t kSortBlock = 256;  // sorted pixels per workgroup
+constexpr uint32_t kSortBlock = 256;  // a scene's sorted entries are padded to a multiple of this
+constexpr uint32_t kMaxTraceWaves = 4;
 
 // Texel bytes per precision.
 inline uint32_t texel_bytes(uint32_t prec) { return (prec == VGI_PREC_FP32 || prec == VGI_PREC_FP16X2) ? 16u : 8u; }

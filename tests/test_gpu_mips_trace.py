@@ -505,3 +505,57 @@ def test_shadowed_and_plain_scenes_in_one_batch(ctx, soup):
     finally:
         a.release()
         b.release()
+
+
+@pytest.mark.parametrize("prec", ["fp32", "fp16x2"])
+def test_trace_is_independent_of_launch_size(ctx, soup, prec):
+    """Launches of few, many and very many 8x8 blocks share a block's cones among other
+    numbers of wavefronts (and FP32 has a register variant for each side): the first rows of
+    a large G-buffer, traced by themselves, give the same bits. 728 x 728 pixels (8281
+    blocks) are past the line where FP32 changes its variant, 888 x 888 (12321) past the one
+    where two wavefronts share a block."""
+    vgi = _vgi()
+    w = soup["w"]
+    f = Frame(ctx, w, prec)
+    rng = np.random.default_rng(9)
+    pick = rng.integers(0, w.num_pixels, 888 * 888)
+    pos, nrm = w.gb_pos[pick].copy(), w.gb_nrm[pick].copy()
+    nrm[rng.random(len(pick)) < 0.02] = 0.0  # pixels without a surface
+
+    def trace(n, width, height):
+        gb = vgi.GBufferData(ctx, pos[:n], nrm[:n], width, height)
+        od = vgi.DeviceArray.empty(ctx, (n, 4), np.float32)
+        osp = vgi.DeviceArray.empty(ctx, (n, 4), np.float32)
+        f.scene.trace(gb, vgi.make_cones(**w.cones), od, osp)
+        return od.numpy(), osp.numpy()
+
+    d0, s0 = trace(72 * 9, 72, 9)
+    for side in (728, 888):
+        print(f"case trace {prec} {side}x{side}", flush=True)
+        d, s = trace(side * side, side, side)
+        assert np.array_equal(d[:len(d0)], d0) and np.array_equal(s[:len(s0)], s0)
+    f.release()
+
+
+@pytest.mark.parametrize("num_diffuse,specular", [(0, True), (1, False), (1, True), (10, True), (11, True), (32, True)])
+def test_cone_counts_vs_fp64(ctx, soup, num_diffuse, specular):
+    """Every split of a block's cones: fewer cones than wavefronts, the counts either side of
+    the change from three wavefronts to four, the most cones; a G-buffer of odd size."""
+    vgi = _vgi()
+    w = soup["w"]
+    print(f"case cones {num_diffuse}+{int(specular)}", flush=True)
+    f = Frame(ctx, w, "fp32")
+    n = 61 * 13
+    cones = dict(w.cones, num_diffuse=num_diffuse, specular=specular)
+    gb = vgi.GBufferData(ctx, w.gb_pos[:n], w.gb_nrm[:n], 61, 13)
+    od = vgi.DeviceArray.empty(ctx, (n, 4), np.float32)
+    osp = vgi.DeviceArray.empty(ctx, (n, 4), np.float32)
+    f.scene.trace(gb, vgi.make_cones(**cones), od, osp)
+    acc, _ = orc.voxelize(w.positions, w.grid, albedo=w.albedo)
+    lv64 = orc.inject_mips(acc, w.grid, w.lights, f64=True)
+    d64, s64, _ = orc.trace(lv64, w.grid, w.gb_pos[:n], w.gb_nrm[:n], cones, f64=True)
+    d, s = od.numpy(), osp.numpy()
+    for got, ref in ((d, d64), (s, s64)):
+        norm = np.linalg.norm(ref)
+        assert np.linalg.norm(got - ref) <= 1e-3 * norm if norm else not got.any()
+    f.release()
