@@ -29,6 +29,7 @@
 #include <memory>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "gltf.hpp"
@@ -91,17 +92,18 @@ int grow_bytes(void** p, size_t* cap, size_t need, const char* what) {
   return VGI_OK;
 }
 
-// Pinned staging for descriptor tables: a ring of slots per stream. A slot's host half is
-// reused once the copy that read it has completed (its event); its device half is reused
-// four calls later on the same stream, when the kernels that read it have run.
-constexpr int kSlots = 4;
+// Pinned staging for descriptor tables: a ring of slots per stream. A kernel copies a
+// slot's host half to its device half and flags what it has read (StageArgs); the host half
+// is reused once every workgroup of that copy has, its device half when the slot's turn
+// comes again on the same stream, after the kernels that read it.
+constexpr int kSlots = 12;  // four frames of three calls
 struct Slot {
   uint8_t* h = nullptr;
   uint8_t* d = nullptr;
   size_t cap = 0;
-  hipEvent_t done = nullptr;
-  bool pending = false;
-  uint64_t gen = 0;  // changes whenever the slot is taken for new contents
+  uint32_t* flags = nullptr;  // pinned, kStageBlocks words
+  uint32_t blocks = 0;        // workgroups of the copy last enqueued
+  uint64_t gen = 0;           // changes whenever the slot is taken for new contents
 };
 
 // Call sites whose descriptor uploads are reused while unchanged.
@@ -224,10 +226,12 @@ struct vgi_scene {
   uint32_t* live = nullptr;  // per 16^3 tile of level 0: a word, then 8 row words (the mip kernel's skip state)
   size_t live_bytes = 0;
   uint32_t alloc_levels = 0, alloc_n = 0, alloc_prec = 0;
-  // the injecting launch's tile-list counts are zero once the work queued so far has run
-  // (the tile state was just cleared, or the last ordered build's later launch zeroed
-  // them); otherwise the next ordered build clears them first
+  // The injecting launch's tile list has two pairs of counts, used in turn by the ordered
+  // builds: a build's list goes with one pair, which is zero, and its injecting launch zeroes
+  // the other for the next build. tile_counts_zero is false while that is not known (a call
+  // that failed in between); the next ordered build then clears both.
   bool tile_counts_zero = false;
+  uint32_t tile_pair = 0;
   bool has_voxels = false, has_mips = false;
   uint64_t tris_in = 0;
   // the last voxelize call's statistics: written by the device into the pinned record after
@@ -261,7 +265,7 @@ void free_workspace(vgi_workspace* w) {
   for (Slot& s : w->slot) {
     if (s.d) (void)hipFree(s.d);
     if (s.h) (void)hipHostFree(s.h);
-    if (s.done) (void)hipEventDestroy(s.done);
+    if (s.flags) (void)hipHostFree(s.flags);
   }
   if (w->hist) (void)hipHostFree(w->hist);
 }
@@ -276,10 +280,13 @@ vgi_workspace* workspace(vgi_context* ctx, hipStream_t st) {
   auto w = std::make_unique<vgi_workspace>();
   w->stream = st;
   for (Slot& s : w->slot)
-    if (hipEventCreateWithFlags(&s.done, hipEventDisableTiming) != hipSuccess) {
+    if (hipHostMalloc((void**)&s.flags, kStageBlocks * sizeof(uint32_t), hipHostMallocCoherent) != hipSuccess) {
       (void)hipGetLastError();
+      s.flags = nullptr;
       free_workspace(w.get());
       return nullptr;
+    } else {
+      std::memset(s.flags, 0, kStageBlocks * sizeof(uint32_t));
     }
   vgi_workspace* raw = w.get();
   ctx->ws.emplace(st, std::move(w));
@@ -291,15 +298,36 @@ vgi_tuning tuning_of(vgi_context* ctx) {
   return ctx->tuning;
 }
 
+// Whether the copy last enqueued from a slot has read its host half.
+bool slot_read(const Slot& s) {
+  for (uint32_t b = 0; b < s.blocks; b++)
+    if (__atomic_load_n(&s.flags[b], __ATOMIC_ACQUIRE) != (uint32_t)s.gen) return false;
+  return true;
+}
+
+// Waits until it has. The stream is asked now and then, so that a wait ends with an error
+// where the copy can no longer run (and never outlasts the stream's work).
+int wait_slot(vgi_workspace* w, const Slot& s) {
+  for (uint32_t spin = 1; !slot_read(s); spin++) {
+    if (spin % 1024u != 0u) {
+      std::this_thread::yield();
+      continue;
+    }
+    const hipError_t e = hipStreamQuery(w->stream);
+    if (e == hipErrorNotReady) continue;
+    HIP_TRY(e);
+    if (!slot_read(s)) return fail(VGI_E_HIP, "a descriptor copy did not run");
+  }
+  return VGI_OK;
+}
+
 // Takes the next staging slot with room for `bytes`; waits for the copy that last used it.
 int acquire_slot(vgi_workspace* w, size_t bytes, Slot** out) {
   Slot& s = w->slot[w->next];
+  TRY(wait_slot(w, s));
   w->next = (w->next + 1) % kSlots;
+  s.blocks = 0;
   s.gen = ++w->slot_gen;  // invalidates any reuse entry for this slot's old contents
-  if (s.pending) {
-    HIP_TRY(hipEventSynchronize(s.done));
-    s.pending = false;
-  }
   if (s.cap < bytes) {
     HIP_TRY(hipStreamSynchronize(w->stream));  // the device half may still be read
     if (s.d) (void)hipFree(s.d);
@@ -309,7 +337,7 @@ int acquire_slot(vgi_workspace* w, size_t bytes, Slot** out) {
     s.cap = 0;
     const size_t cap = std::max<size_t>(align_up(bytes + bytes / 2, 4096), 65536);
     if (hipMalloc((void**)&s.d, cap) != hipSuccess ||
-        hipHostMalloc((void**)&s.h, cap, hipHostMallocDefault) != hipSuccess) {
+        hipHostMalloc((void**)&s.h, cap, hipHostMallocCoherent) != hipSuccess) {
       (void)hipGetLastError();
       return fail(VGI_E_NOMEM, "staging allocation of %zu bytes failed", cap);
     }
@@ -319,21 +347,27 @@ int acquire_slot(vgi_workspace* w, size_t bytes, Slot** out) {
   return VGI_OK;
 }
 
-int upload(vgi_workspace* w, Slot* s, size_t offset, size_t bytes) {
-  if (bytes) HIP_TRY(hipMemcpyAsync(s->d + offset, s->h + offset, bytes, hipMemcpyHostToDevice, w->stream));
-  HIP_TRY(hipEventRecord(s->done, w->stream));
-  s->pending = true;
-  return VGI_OK;
+// The copy of a slot's first `bytes` bytes, for the kernel that will do it.
+StageArgs stage_args(const Slot& s, size_t bytes) {
+  StageArgs a{};
+  a.dst = s.d;
+  a.src = s.h;
+  a.flags = s.flags;
+  a.words = (uint32_t)((bytes + 15) / 16);
+  a.blocks = std::min<uint32_t>((a.words + 255) / 256, kStageBlocks);
+  a.gen = (uint32_t)s.gen;
+  return a;
 }
 
 // A call's descriptor tables: fill(h, d) writes them into host memory h for a device copy
-// at d (tables may point into themselves). If the site's last upload is still held (its
-// slot not taken since) and the new bytes equal it, that device copy is used as it is and
-// nothing is copied -- a repeated frame over unchanged scenes, lights and G-buffers uploads
-// nothing. Otherwise a slot is taken and the tables are uploaded. Equal bytes mean the
-// device already holds exactly what the upload would write, so reuse cannot change results.
-template <class F>
-int stage_descriptors(vgi_workspace* w, UploadSite site, size_t bytes, F&& fill, Slot** out) {
+// at d (tables may point into themselves). If the site's last copy is still held (its slot
+// not taken since) and the new bytes equal it, that device copy is used as it is and nothing
+// is copied -- a repeated frame over unchanged scenes, lights and G-buffers copies nothing.
+// Otherwise a slot is taken and launch(args) enqueues the kernel that copies it. Equal bytes
+// mean the device already holds exactly what the copy would write, so reuse cannot change
+// results. launch is called either way, with no blocks where nothing is to be copied.
+template <class F, class L>
+int stage_descriptors(vgi_workspace* w, UploadSite site, size_t bytes, F&& fill, L&& launch, Slot** out) {
   UploadCache& c = w->cache[site];
   if (c.slot >= 0 && c.bytes == bytes && w->slot[c.slot].gen == c.gen) {
     Slot& s = w->slot[c.slot];
@@ -341,14 +375,19 @@ int stage_descriptors(vgi_workspace* w, UploadSite site, size_t bytes, F&& fill,
     fill(w->staging.data(), s.d);
     if (std::memcmp(w->staging.data(), s.h, bytes) == 0) {
       *out = &s;
-      return VGI_OK;
+      return launch(s, StageArgs{});
     }
   }
   Slot* sl = nullptr;
   TRY(acquire_slot(w, bytes, &sl));
   std::memset(sl->h, 0, bytes);
   fill(sl->h, sl->d);
-  TRY(upload(w, sl, 0, bytes));
+  const StageArgs a = stage_args(*sl, bytes);
+  if (const int rc = launch(*sl, a)) {  // the copy may or may not be queued
+    (void)hipStreamSynchronize(w->stream);
+    return rc;
+  }
+  sl->blocks = a.blocks;
   c.slot = (int)(sl - w->slot);
   c.gen = sl->gen;
   c.bytes = bytes;
@@ -513,15 +552,15 @@ struct VoxPlan {
 // persistent for the
 // large triangles and the split bins, whose counts only the device knows; k_voxelize takes
 // one work unit per workgroup up to grid_blocks and loops over the rest.
-int launch_voxelize_kernels(vgi_context* ctx, const VoxBatch& B, uint32_t* zb, size_t zeroed_bytes, void* scan_tmp,
-                            size_t scan_tmp_bytes, size_t nblk_t, size_t nblk_b, uint32_t ts, uint32_t grid_blocks,
+int launch_voxelize_kernels(vgi_context* ctx, const VoxBatch& B, const StageArgs& stage, uint32_t* zb,
+                            size_t zeroed_bytes, size_t nblk_t, size_t nblk_b, uint32_t ts, uint32_t grid_blocks,
                             uint32_t big_blocks, uint32_t zero_blocks, vgi_scene* const* scenes, uint32_t count,
                             hipStream_t st, bool prof) {
-  const uint32_t cus = (uint32_t)ctx->num_cus;
-  const uint32_t persistent = cus * 4;
+  const uint32_t persistent = (uint32_t)ctx->num_cus * 4;
   if (prof) HIP_TRY(hipEventRecord(ctx->ev[0], st));
-  // bin_small, bin_big, big_cursor, the per-scene counters and the overflow word start at zero
-  HIP_TRY(launch_fill_u32(zb, 0u, zeroed_bytes / 4, st));
+  // bin_small, bin_big, big_cursor, the per-scene counters and the overflow word start at
+  // zero; the same launch brings the call's descriptors to the device
+  HIP_TRY(launch_begin(stage, zb, zeroed_bytes / 4, st));
   HIP_TRY(launch_setup(B, (uint32_t)nblk_t, st));
   HIP_TRY(launch_big_count(B, persistent, st));
   if (prof) HIP_TRY(hipEventRecord(ctx->ev[1], st));
@@ -531,7 +570,6 @@ int launch_voxelize_kernels(vgi_context* ctx, const VoxBatch& B, uint32_t* zb, s
   HIP_TRY(launch_scatter(B, (uint32_t)nblk_b, (uint32_t)nblk_t, big_blocks, zero_blocks, st));
   if (prof) HIP_TRY(hipEventRecord(ctx->ev[3], st));
   HIP_TRY(launch_voxelize(B, ts, grid_blocks, st));
-  HIP_TRY(launch_voxelize_fallback(B, cus, st));
   if (prof) {
     HIP_TRY(hipEventRecord(ctx->ev[4], st));
     ctx->ev_vox = true;
@@ -702,13 +740,7 @@ int voxelize_batch(vgi_context* ctx, const vgi_voxelize_item* items, uint32_t co
     }
   }
   };
-  Slot* sl = nullptr;
-  TRY(stage_descriptors(w, kSiteVoxelize, cv.off, fill, &sl));
-
   VoxBatch B{};
-  B.scenes = (const VoxScene*)(sl->d + o_scenes);
-  B.tri_blocks = multi ? (const uint2*)(sl->d + o_tblk) : nullptr;
-  B.bin_blocks = multi ? (const uint2*)(sl->d + o_bblk) : nullptr;
   B.scan_all = (unsigned long long*)w->scan_all;
   B.scan_flags = (uint32_t*)((uint8_t*)w->zeroed + flags_off);
   B.scan_vals = (unsigned long long*)w->scan_tmp;
@@ -737,8 +769,15 @@ int voxelize_batch(vgi_context* ctx, const vgi_voxelize_item* items, uint32_t co
       (uint32_t)std::min<uint64_t>(cus * 4, w->hist_big ? (w->hist_big + w->hist_big / 4 + 3) / 4 + 1 : cus);
   const uint32_t zero_blocks = (uint32_t)std::min<uint64_t>(
       std::min<uint64_t>(cus * 4, total_bins), w->hist_split ? w->hist_split + w->hist_split / 4 + 1 : cus / 4);
-  TRY(launch_voxelize_kernels(ctx, B, zb, zeroed_need, w->scan_tmp, w->scan_tmp_bytes, nblk_t, nblk_b, ts,
-                              grid_blocks, big_blocks, zero_blocks, scs.data(), count, st, ctx->profiling != 0));
+  auto launch = [&](const Slot& sl, const StageArgs& stage) -> int {
+    B.scenes = (const VoxScene*)(sl.d + o_scenes);
+    B.tri_blocks = multi ? (const uint2*)(sl.d + o_tblk) : nullptr;
+    B.bin_blocks = multi ? (const uint2*)(sl.d + o_bblk) : nullptr;
+    return launch_voxelize_kernels(ctx, B, stage, zb, zeroed_need, nblk_t, nblk_b, ts, grid_blocks, big_blocks,
+                                   zero_blocks, scs.data(), count, st, ctx->profiling != 0);
+  };
+  Slot* sl = nullptr;
+  TRY(stage_descriptors(w, kSiteVoxelize, cv.off, fill, launch, &sl));
   for (uint32_t i = 0; i < count; i++) {
     vgi_scene* s = plan[i].s;
     s->grid = items[i].grid;
@@ -786,6 +825,7 @@ int scene_levels(vgi_scene* s, uint32_t precision, hipStream_t st) {
     s->live_bytes = bytes;
     HIP_TRY(launch_fill_u32(s->live, 0u, bytes / 4, st));
     s->tile_counts_zero = true;
+    s->tile_pair = 0;
   }
   for (uint32_t k = 0; k < g.levels; k++) {
     const size_t p = (size_t)(g.n >> k) + 2;
@@ -907,42 +947,52 @@ int mips_batch(vgi_context* ctx, const vgi_mips_item* items, uint32_t count, uin
       boff += v.size();
     }
   };
-  Slot* sl = nullptr;
-  TRY(stage_descriptors(w, kSiteMips, cv.off, fill, &sl));
   const bool prof = ctx->profiling != 0;
-  if (prof) HIP_TRY(hipEventRecord(ctx->ev[5], st));
-  size_t off = 0;
-  uint32_t* list_counts = nullptr;  // an ordered build's tile-list counts
-  for (size_t j = 0; j < stages.size(); j++) {
-    MipBatch B{};
-    B.scenes = (const MipScene*)(sl->d + o_scenes);
-    B.blocks = table ? (const MipBlock*)(sl->d + o_blocks) + off : nullptr;
-    B.lut = ctx->d_lut;
-    B.src = stages[j][0].src;  // one scene: every block of the stage shares src and nout
-    B.nout = stages[j][0].nout;
-    B.shadow = shadow;
-    // (not for a one-level chain: its launch writes every texel of every tile and keeps no
-    // tile words, so every tile is visited; not with visibility walks, whose cost does not
-    // follow the pair count: the room's shadowed builds were 3-5% slower in list order)
-    B.ordered = j == 0 && !table && stages[0][0].nout > 0 && !shadow;
-    if (B.ordered) {  // the injecting launch's tile list, dense tiles first
-      vgi_scene* sc = items[0].scene;
-      const vgi_grid& g = sc->grid;
-      const size_t tpa = g.n / std::min<uint32_t>(g.n, 16u), ntl = tpa * tpa * tpa;
-      list_counts = sc->live + 10 * ntl;
-      if (!sc->tile_counts_zero) HIP_TRY(launch_fill_u32(list_counts, 0u, 2, st));
-      sc->tile_counts_zero = false;
-      HIP_TRY(launch_tiles(B, (uint32_t)ntl, st));
+  auto launch = [&](const Slot& sl, const StageArgs& stage) -> int {
+    if (prof) HIP_TRY(hipEventRecord(ctx->ev[5], st));
+    size_t off = 0;
+    for (size_t j = 0; j < stages.size(); j++) {
+      MipBatch B{};
+      B.scenes = (const MipScene*)(sl.d + o_scenes);
+      B.blocks = table ? (const MipBlock*)(sl.d + o_blocks) + off : nullptr;
+      B.lut = ctx->d_lut;
+      B.src = stages[j][0].src;  // one scene: every block of the stage shares src and nout
+      B.nout = stages[j][0].nout;
+      B.shadow = shadow;
+      // (not for a one-level chain: its launch writes every texel of every tile and keeps no
+      // tile words, so every tile is visited; not with visibility walks, whose cost does not
+      // follow the pair count: the room's shadowed builds were 3-5% slower in list order)
+      const bool ordered = j == 0 && !table && stages[0][0].nout > 0 && !shadow;
+      if (ordered) {  // the injecting launch's tile list, dense tiles first; the descriptors with it
+        vgi_scene* sc = items[0].scene;
+        const vgi_grid& g = sc->grid;
+        const size_t tpa = g.n / std::min<uint32_t>(g.n, 16u), ntl = tpa * tpa * tpa;
+        uint32_t* counts = sc->live + 10 * ntl;
+        if (!sc->tile_counts_zero) HIP_TRY(launch_fill_u32(counts, 0u, 4, st));
+        sc->tile_counts_zero = false;
+        B.counts = counts + 2 * sc->tile_pair;
+        B.clear_counts = counts + 2 * (sc->tile_pair ^ 1u);
+        const TileArgs t{(const unsigned long long*)sc->bin_packed, sc->live, sc->live + 9 * ntl, B.counts, g.n,
+                         sc->bin_shift, sc->nbins_axis};
+        HIP_TRY(launch_tiles(t, stage, (uint32_t)ntl, st));
+      } else if (j == 0) {
+        HIP_TRY(launch_stage(stage, st));
+      }
+      HIP_TRY(launch_mips(B, precision, j == 0, (uint32_t)stages[j].size(), st));
+      if (B.counts) {
+        items[0].scene->tile_counts_zero = true;
+        items[0].scene->tile_pair ^= 1u;
+      }
+      off += stages[j].size();
     }
-    B.clear_counts = j == 1 ? list_counts : nullptr;  // the next build then needs no clearing launch
-    HIP_TRY(launch_mips(B, precision, j == 0, (uint32_t)stages[j].size(), st));
-    if (B.clear_counts) items[0].scene->tile_counts_zero = true;
-    off += stages[j].size();
-  }
-  if (prof) {
-    HIP_TRY(hipEventRecord(ctx->ev[6], st));
-    ctx->ev_mips = true;
-  }
+    if (prof) {
+      HIP_TRY(hipEventRecord(ctx->ev[6], st));
+      ctx->ev_mips = true;
+    }
+    return VGI_OK;
+  };
+  Slot* sl = nullptr;
+  TRY(stage_descriptors(w, kSiteMips, cv.off, fill, launch, &sl));
   for (uint32_t i = 0; i < count; i++) {
     items[i].scene->prec = precision;
     items[i].scene->has_mips = true;
@@ -1208,44 +1258,48 @@ int trace_batch(vgi_context* ctx, const vgi_trace_item* items, uint32_t count, v
     if (morton) hs[L.nscenes] = (uint32_t)e;
   }
   };
-  TRY(stage_descriptors(w, kSiteTrace, cv.off, fill, &sl));
-  const bool prof = ctx->profiling != 0;
-  if (prof) {
-    HIP_TRY(launch_fill_u32((uint32_t*)ctx->d_counter, 0u, 2, st));
-    HIP_TRY(hipEventRecord(ctx->ev[7], st));
-  }
-  for (const Launch& L : launches) {
-    TraceBatch B{};
-    B.scenes = (const TraceParams*)(sl->d + L.o_params);
-    B.blocks = !morton && L.nscenes > 1 ? (const uint2*)(sl->d + L.o_blocks) : nullptr;
-    B.counter = prof ? ctx->d_counter : nullptr;
-    B.nblocks = (uint32_t)L.nblocks;
-    B.tile_w = tn.tile_w;
-    B.tile_h = tn.tile_h;
-    B.prec = L.prec;
-    B.nscenes = L.nscenes;
-    B.band = L.band;
-    B.sub_shift = sub_shift;
-    B.waves = L.waves;
-    B.full = L.full ? 1u : 0u;
-    B.max_diffuse = L.max_diffuse;
-    if (morton && L.entries > 0) {
-      unsigned long long* keys = (unsigned long long*)w->sort_keys;
-      uint32_t* pix = (uint32_t*)w->sort_pix;
-      B.seg = (const uint32_t*)(sl->d + L.o_seg);
-      HIP_TRY(launch_morton_keys(B, keys, pix, (uint32_t)L.entries, st));
-      const int end_bit = 32 + (int)ilog2(std::max<uint32_t>(L.nscenes - 1, 1)) + 1;
-      HIP_TRY(sort_pixels(w->sort_tmp, &w->sort_tmp_bytes, keys, keys + max_entries, pix, pix + max_entries,
-                          (uint32_t)L.entries, std::min(end_bit, 64), st));
-      B.skeys = keys + max_entries;
-      B.spix = pix + max_entries;
+  auto launch = [&](const Slot& sl, const StageArgs& stage) -> int {
+    HIP_TRY(launch_stage(stage, st));
+    const bool prof = ctx->profiling != 0;
+    if (prof) {
+      HIP_TRY(launch_fill_u32((uint32_t*)ctx->d_counter, 0u, 2, st));
+      HIP_TRY(hipEventRecord(ctx->ev[7], st));
     }
-    HIP_TRY(launch_trace(B, L.buffer_path, st));
-  }
-  if (prof) {
-    HIP_TRY(hipEventRecord(ctx->ev[8], st));
-    ctx->ev_trace = true;
-  }
+    for (const Launch& L : launches) {
+      TraceBatch B{};
+      B.scenes = (const TraceParams*)(sl.d + L.o_params);
+      B.blocks = !morton && L.nscenes > 1 ? (const uint2*)(sl.d + L.o_blocks) : nullptr;
+      B.counter = prof ? ctx->d_counter : nullptr;
+      B.nblocks = (uint32_t)L.nblocks;
+      B.tile_w = tn.tile_w;
+      B.tile_h = tn.tile_h;
+      B.prec = L.prec;
+      B.nscenes = L.nscenes;
+      B.band = L.band;
+      B.sub_shift = sub_shift;
+      B.waves = L.waves;
+      B.full = L.full ? 1u : 0u;
+      B.max_diffuse = L.max_diffuse;
+      if (morton && L.entries > 0) {
+        unsigned long long* keys = (unsigned long long*)w->sort_keys;
+        uint32_t* pix = (uint32_t*)w->sort_pix;
+        B.seg = (const uint32_t*)(sl.d + L.o_seg);
+        HIP_TRY(launch_morton_keys(B, keys, pix, (uint32_t)L.entries, st));
+        const int end_bit = 32 + (int)ilog2(std::max<uint32_t>(L.nscenes - 1, 1)) + 1;
+        HIP_TRY(sort_pixels(w->sort_tmp, &w->sort_tmp_bytes, keys, keys + max_entries, pix, pix + max_entries,
+                            (uint32_t)L.entries, std::min(end_bit, 64), st));
+        B.skeys = keys + max_entries;
+        B.spix = pix + max_entries;
+      }
+      HIP_TRY(launch_trace(B, L.buffer_path, st));
+    }
+    if (prof) {
+      HIP_TRY(hipEventRecord(ctx->ev[8], st));
+      ctx->ev_trace = true;
+    }
+    return VGI_OK;
+  };
+  TRY(stage_descriptors(w, kSiteTrace, cv.off, fill, launch, &sl));
   return VGI_OK;
 }
 
@@ -1638,7 +1692,7 @@ int vgi_voxelize_noalloc(vgi_context* ctx, vgi_scene* sc, const vgi_mesh* meshes
   B.textured = textured ? 1u : 0u;
   const uint32_t grid_blocks = (uint32_t)std::min<uint64_t>((uint64_t)ctx->num_cus * 8, work_cap64);
   const uint32_t cus = (uint32_t)ctx->num_cus;
-  TRY(launch_voxelize_kernels(ctx, B, zb, zeroed_bytes, base + o_stmp, scan_need, ceil_div(ntri, kBlockTris),
+  TRY(launch_voxelize_kernels(ctx, B, StageArgs{}, zb, zeroed_bytes, ceil_div(ntri, kBlockTris),
                               ceil_div(nbins, kBlockBins), ts, grid_blocks, cus,
                               (uint32_t)std::min<uint64_t>(cus / 4, nbins), &sc, 1, st, false));
   sc->grid = *grid;

@@ -330,25 +330,26 @@ template <int PREC, bool SRC_ACC, bool SHADOW>
 __global__ __launch_bounds__(1024) void k_mips(const MipScene* __restrict__ scenes,
                                                const MipBlock* __restrict__ blocks,
                                                const float* __restrict__ lut, uint32_t src1, uint32_t nout1,
-                                               uint32_t ordered, uint32_t* __restrict__ clear_counts) {
+                                               const uint32_t* __restrict__ counts,
+                                               uint32_t* __restrict__ clear_counts) {
   using TX = Texel<PREC>;
   constexpr uint32_t kThreads = mips_threads(PREC, SRC_ACC, SHADOW);
   __shared__ float4 s_a[512];
   __shared__ float4 s_b[64];
   const MipBlock blk = blocks ? blocks[blockIdx.x] : MipBlock{0u, blockIdx.x, src1, nout1};
   const MipScene& P = scenes[blk.scene];
-  // a later launch of an ordered build: the injecting launch, the list's only reader, has
-  // completed, so the counts are zeroed here for the next build's k_tiles
-  if (!SRC_ACC && clear_counts && blockIdx.x == 0 && threadIdx.x < 2) gst(clear_counts + threadIdx.x, 0u);
+  // the other pair of list counts, zeroed for the next build's k_tiles (its last reader, the
+  // injecting launch before this one, has completed)
+  if (SRC_ACC && clear_counts && blockIdx.x == 0 && threadIdx.x < 2) gst(clear_counts + threadIdx.x, 0u);
   const uint32_t src = blk.src, nout = blk.nout;
   const uint32_t ns = P.nk[src];
   const uint32_t S = ns < 16u ? ns : 16u;  // source tile edge (a power of two)
   const uint32_t tpa = ns / S;             // tiles per axis
   uint32_t tile = blk.tile;
-  if (SRC_ACC && ordered) {  // block b takes the b-th tile of k_tiles' list; unlisted tiles keep their zeros
+  if (SRC_ACC && counts) {  // block b takes the b-th tile of k_tiles' list; unlisted tiles keep their zeros
     const uint32_t ntl = tpa * tpa * tpa, b = blockIdx.x;
     // (clamped: a list never holds more than ntl tiles)
-    const uint32_t nd = min(gld(P.order + ntl), ntl), nl = min(gld(P.order + ntl + 1), ntl - nd);
+    const uint32_t nd = min(gld(counts), ntl), nl = min(gld(counts + 1), ntl - nd);
     if (b >= nd + nl) return;  // uniform
     tile = gld(P.order + (b < nd ? b : ntl - 1u - (b - nd)));
   }
@@ -526,30 +527,33 @@ static void launch_mips_prec(const MipBatch& B, bool from_acc, dim3 g, hipStream
   const dim3 b(mips_threads(PREC, from_acc, from_acc && B.shadow));
   if (!from_acc)
     hipLaunchKernelGGL((k_mips<PREC, false, false>), g, b, 0, s, B.scenes, B.blocks, B.lut, B.src, B.nout,
-                       (uint32_t)B.ordered, B.clear_counts);
+                       (const uint32_t*)nullptr, (uint32_t*)nullptr);
   else if (B.shadow)
     hipLaunchKernelGGL((k_mips<PREC, true, true>), g, b, 0, s, B.scenes, B.blocks, B.lut, B.src, B.nout,
-                       (uint32_t)B.ordered, (uint32_t*)nullptr);
+                       B.counts, B.clear_counts);
   else
     hipLaunchKernelGGL((k_mips<PREC, true, false>), g, b, 0, s, B.scenes, B.blocks, B.lut, B.src, B.nout,
-                       (uint32_t)B.ordered, (uint32_t*)nullptr);
+                       B.counts, B.clear_counts);
 }
 
 // The injecting launch's tiles for one scene, densest first: a tile is listed when its bins
 // hold pairs (it may hold voxels) or its stored texels are not all zero (it must be
 // cleared); tiles whose bins hold at least kDenseTilePairs pairs go to the front of the
-// list, the others to the back, with one atomic per wavefront and class on the two counts
-// after the list (cleared before the launch). Unlisted tiles hold no voxel and only zeros,
+// list, the others to the back, with one atomic per wavefront and class on the list's two
+// counts (zero before the launch). Unlisted tiles hold no voxel and only zeros,
 // and are left as they are. A dense tile's inject sets the injecting launch's length (on
 // the room, about 3200 occupied voxels against a median of 430), so those start first,
 // and empty tiles no longer take a workgroup slot each. A tile's bins' pair count follows
 // its occupied voxel count closely (correlation 0.96 on the room); 384 pairs marks about
 // the densest third of the room's occupied tiles.
 constexpr uint32_t kDenseTilePairs = 384;
-__global__ __launch_bounds__(256) void k_tiles(const MipScene* __restrict__ scenes) {
-  const MipScene& P = scenes[0];
-  const uint32_t ns = P.nk[0], S = ns < 16u ? ns : 16u, tpa = ns / S, ntl = tpa * tpa * tpa;
-  const uint32_t t = blockIdx.x * 256u + threadIdx.x;
+__global__ __launch_bounds__(256) void k_tiles(TileArgs P, StageArgs stage) {
+  if (blockIdx.x < stage.blocks) {  // the tables that the build's other kernels read
+    stage_block(stage, blockIdx.x);
+    return;
+  }
+  const uint32_t ns = P.n, S = ns < 16u ? ns : 16u, tpa = ns / S, ntl = tpa * tpa * tpa;
+  const uint32_t t = (blockIdx.x - stage.blocks) * 256u + threadIdx.x;
   uint32_t dense = 0, other = 0;
   if (t < ntl) {
     const uint32_t tx = t % tpa, ty = (t / tpa) % tpa, tz = t / (tpa * tpa);
@@ -582,8 +586,8 @@ __global__ __launch_bounds__(256) void k_tiles(const MipScene* __restrict__ scen
   const uint64_t below = (1ull << lane) - 1ull;
   uint32_t dbase = 0, obase = 0;
   if (lane == 0) {
-    if (dm) dbase = gatomic_add(P.order + ntl, (uint32_t)__popcll(dm));
-    if (om) obase = gatomic_add(P.order + ntl + 1, (uint32_t)__popcll(om));
+    if (dm) dbase = gatomic_add(P.counts, (uint32_t)__popcll(dm));
+    if (om) obase = gatomic_add(P.counts + 1, (uint32_t)__popcll(om));
   }
   dbase = __shfl(dbase, 0);
   obase = __shfl(obase, 0);
@@ -591,8 +595,8 @@ __global__ __launch_bounds__(256) void k_tiles(const MipScene* __restrict__ scen
   if (other) gst(P.order + ntl - 1u - (obase + (uint32_t)__popcll(om & below)), t);
 }
 
-hipError_t launch_tiles(const MipBatch& B, uint32_t ntiles, hipStream_t s) {
-  hipLaunchKernelGGL(k_tiles, dim3((ntiles + 255) / 256), dim3(256), 0, s, B.scenes);
+hipError_t launch_tiles(const TileArgs& t, const StageArgs& a, uint32_t ntiles, hipStream_t s) {
+  hipLaunchKernelGGL(k_tiles, dim3(a.blocks + (ntiles + 255) / 256), dim3(256), 0, s, t, a);
   return hipGetLastError();
 }
 

@@ -132,6 +132,21 @@ struct NoAllocDesc {
   MeshDev meshes[VGI_NOALLOC_MAX_MESHES];
 };
 
+// A call's descriptor tables on their way to the device: workgroup b of `blocks` copies its
+// share from pinned host memory and then stores `gen` to flags[b] (pinned), which tells the
+// host that it has read it. Folded into a call's first kernel where that one does not read
+// the tables itself. A copy command and the event behind it held the stream about 9.5 us,
+// three times a frame; the copying workgroups add about 1 us to a kernel that runs anyway.
+struct StageArgs {
+  void* dst;
+  const void* src;   // 16-byte words
+  uint32_t* flags;
+  uint32_t words;
+  uint32_t blocks;   // 0: nothing to copy
+  uint32_t gen;
+};
+constexpr uint32_t kStageBlocks = 16;
+
 struct VoxBatch {
   const VoxScene* scenes;
   const uint2* tri_blocks;          // (scene, first triangle) per setup/emit workgroup
@@ -182,8 +197,7 @@ struct MipScene {
   uint32_t* live;  // per 16^3 tile of level 0: 1 while the tile's stored texels are not all zero;
                    // after the tiles' words, 8 words per tile: bit (ly + 16 lz) while that
                    // x-row's stored level-0 texels are not all zero
-  uint32_t* order; // the injecting launch's tiles, dense ones first (one word per tile), then
-                   // the dense and other tiles' counts (k_tiles)
+  uint32_t* order; // the injecting launch's tiles, dense ones first (one word per tile; k_tiles)
   void* level[VGI_MAX_LEVELS];
   uint32_t nk[VGI_MAX_LEVELS];
   uint32_t n;
@@ -201,6 +215,15 @@ struct MipBlock {
   uint32_t scene, tile, src, nout;
 };
 
+// What k_tiles needs of its scene, by value: its launch brings the tables to the device.
+struct TileArgs {
+  const unsigned long long* bin_packed;
+  const uint32_t* live;
+  uint32_t* order;
+  uint32_t* counts;
+  uint32_t n, bin_shift, nbins_axis;
+};
+
 struct MipBatch {
   const MipScene* scenes;
   const MipBlock* blocks;  // per workgroup; null for one scene: then block b is tile b of
@@ -208,9 +231,10 @@ struct MipBatch {
   const float* lut;        // 256 entries: (i/255)^2.2
   uint32_t src, nout;
   bool shadow;             // some light of the batch casts shadows (the injecting launch walks)
-  bool ordered;            // one scene, injecting launch: block b takes the listed tile b
-  uint32_t* clear_counts;  // a later launch of an ordered build: the list's two counts, which
-                           // its first workgroup zeroes for the next build (else null)
+  // an ordered build's injecting launch (one scene): block b takes the listed tile b; the
+  // list's two counts (dense and other tiles), and the next build's pair, which it zeroes
+  uint32_t* counts;
+  uint32_t* clear_counts;
 };
 
 // One scene of a trace batch (device memory).
@@ -379,6 +403,14 @@ __device__ __forceinline__ void gatomic_or(uint32_t* p, uint32_t v) {
   __hip_atomic_fetch_or((VGI_GLOBAL uint32_t*)p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Workgroup b (256 threads) of a descriptor copy.
+__device__ __forceinline__ void stage_block(const StageArgs& a, uint32_t b) {
+  for (uint32_t i = b * 256u + threadIdx.x; i < a.words; i += a.blocks * 256u)
+    gst4((uint4*)a.dst + i, gld4((const uint4*)a.src + i));
+  __syncthreads();  // a word is stored once its load has returned: the host's copy is read
+  if (threadIdx.x == 0) __hip_atomic_store(a.flags + b, a.gen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // FP32 -> FP16 bits, round to nearest even. The value is rounded to FP32 first, then to
 // FP16: without the register barrier the backend may fuse a preceding multiply into the
 // conversion (v_fma_mixlo_f16), which rounds once and differs from the two roundings by
@@ -401,6 +433,9 @@ int check_request_input(const vgi_mesh* meshes, uint32_t num_meshes, const vgi_g
 
 // ---- launchers (each returns hipError_t) ----
 hipError_t launch_fill_u32(uint32_t* p, uint32_t value, size_t count, hipStream_t s);
+hipError_t launch_stage(const StageArgs& a, hipStream_t s);
+// Zeroes `words` words at zb and copies a call's descriptor tables, in one launch.
+hipError_t launch_begin(const StageArgs& a, uint32_t* zb, size_t words, hipStream_t s);
 hipError_t launch_copy(void* dst, const void* src, size_t bytes, hipStream_t s);
 hipError_t launch_setup(const VoxBatch& B, uint32_t blocks, hipStream_t s);
 hipError_t launch_big_count(const VoxBatch& B, uint32_t blocks, hipStream_t s);
@@ -410,9 +445,8 @@ hipError_t launch_stage_desc(const NoAllocDesc& d, NoAllocDesc* dst, hipStream_t
 hipError_t launch_scatter(const VoxBatch& B, uint32_t nblk_b, uint32_t nblk_t, uint32_t big_blocks,
                           uint32_t zero_blocks, hipStream_t s);
 hipError_t launch_voxelize(const VoxBatch& B, uint32_t tile, uint32_t grid_blocks, hipStream_t s);
-hipError_t launch_voxelize_fallback(const VoxBatch& B, uint32_t grid_blocks, hipStream_t s);
 hipError_t launch_mips(const MipBatch& B, uint32_t prec, bool from_acc, uint32_t blocks, hipStream_t s);
-hipError_t launch_tiles(const MipBatch& B, uint32_t ntiles, hipStream_t s);
+hipError_t launch_tiles(const TileArgs& t, const StageArgs& a, uint32_t ntiles, hipStream_t s);
 hipError_t launch_trace(const TraceBatch& B, bool buffer_path, hipStream_t s);
 // Morton keys of every pixel of a batch (entries seg[0]..seg[nscenes], padding included).
 hipError_t launch_morton_keys(const TraceBatch& B, unsigned long long* keys, uint32_t* pix, uint32_t entries,

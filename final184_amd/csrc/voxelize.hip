@@ -41,16 +41,16 @@
 //                   flush every tile. Flush: occupancy mask + the records of occupied
 //                   voxels, by plain stores for bins of one unit (most bins: a unit is up
 //                   to kUnitItems chunks) and by 64-bit integer atomics otherwise.
-//   7 k_voxelize_fallback  only when the overflow word is set (k_scatter then cleared every
-//                   bin with pairs instead of scattering): one wavefront per triangle tests
-//                   every voxel of its box and adds its increments by 64-bit atomics. The
-//                   voxel set and the sums are the same; it is slower, and the host grows the
-//                   pair list for the calls that follow.
+//   7 fallback pass  k_voxelize's other branch, taken when the overflow word is set (k_scatter
+//                   then cleared every bin with pairs instead of scattering): one wavefront
+//                   per triangle tests every voxel of its box and adds its increments by
+//                   64-bit atomics. The voxel set and the sums are the same; it is slower, and
+//                   the host grows the pair list for the calls that follow.
 //
 // All coverage decisions are exact integer arithmetic on snapped vertices, so the
 // voxel set and the integer sums do not depend on order, rounding or thread mapping.
+#include <algorithm>
 #include <cstddef>
-
 
 #include "vgi_internal.hpp"
 
@@ -73,6 +73,30 @@ hipError_t launch_fill_u32(uint32_t* p, uint32_t value, size_t count, hipStream_
   size_t blocks = (count + 255) / 256;
   if (blocks > 4096) blocks = 4096;
   hipLaunchKernelGGL(k_fill_u32, dim3((unsigned)blocks), dim3(256), 0, s, p, value, count);
+  return hipGetLastError();
+}
+
+__global__ __launch_bounds__(256) void k_stage(StageArgs a) { stage_block(a, blockIdx.x); }
+
+hipError_t launch_stage(const StageArgs& a, hipStream_t s) {
+  if (a.blocks == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_stage, dim3(a.blocks), dim3(256), 0, s, a);
+  return hipGetLastError();
+}
+
+__global__ __launch_bounds__(256) void k_begin(StageArgs a, uint32_t* __restrict__ zb, size_t quads) {
+  if (blockIdx.x < a.blocks) {
+    stage_block(a, blockIdx.x);
+    return;
+  }
+  const size_t stride = (size_t)(gridDim.x - a.blocks) * 256u;
+  for (size_t i = (size_t)(blockIdx.x - a.blocks) * 256u + threadIdx.x; i < quads; i += stride)
+    gst4((uint4*)zb + i, make_uint4(0, 0, 0, 0));
+}
+
+hipError_t launch_begin(const StageArgs& a, uint32_t* zb, size_t words, hipStream_t s) {
+  const size_t blocks = std::min<size_t>((words / 4 + 255) / 256, 2048);
+  hipLaunchKernelGGL(k_begin, dim3((unsigned)(a.blocks + blocks)), dim3(256), 0, s, a, zb, words / 4);
   return hipGetLastError();
 }
 
@@ -1144,16 +1168,76 @@ struct TileLayout {
   static constexpr int ENTRIES = (TS - 1) * (1 + PY + PZ) + 1;
 };
 
+// The overflow path, taken by the whole launch when k_scatter set the overflow word (and
+// cleared every bin with pairs). Wavefront w of the launch takes triangles w, w + nwaves, ...
+// of every scene; its lanes walk the triangle's voxel box, keep the voxels the exact
+// closed-box test accepts (the same test as the bin pass, at voxel size) and add the
+// triangle's increments: R, G, B and the count, then the three biased normal components, as
+// four 64-bit atomics (exact with fewer than 2^21 triangles per voxel: no 32-bit word's total
+// reaches 2^32), and set the voxel's occupancy bit. Integer sums do not depend on order, so
+// the accumulator is the same as the binned path's.
+template <bool TEX>
+__device__ __forceinline__ void fallback_pass(const VoxBatch& B, const VoxScene* __restrict__ scenes) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6), nwaves = gridDim.x * (blockDim.x >> 6);
+  for (uint32_t sc = 0; sc < B.nscenes; sc++) {
+    const VoxScene& P = scenes[sc];
+    const uint32_t nbr = P.n >> 3;
+    for (uint32_t t = wave; t < P.ntri; t += nwaves) {
+      const TriRec R = gld_rec(P.tris + t);
+      if (!tri_ok(R)) continue;
+      int64_t q[3][3], N[3];
+      load_q(R, q, N);
+      const int nx = R.hi[0] - R.lo[0] + 1, ny = R.hi[1] - R.lo[1] + 1, nz = R.hi[2] - R.lo[2] + 1;
+      const uint32_t r = R.rgb & 0xFFu, g = (R.rgb >> 8) & 0xFFu, b = (R.rgb >> 16) & 0xFFu;
+      unsigned long long i0 = (unsigned long long)r | ((unsigned long long)g << 32);
+      unsigned long long i1 = (unsigned long long)b | (1ull << 32);
+      TexCoef X;
+      X.textured = 0;
+      if constexpr (TEX) load_texcoef(P, t, X);
+      const unsigned long long i2 = (unsigned long long)(uint32_t)(R.nq[0] + kNormalBias) |
+                                    ((unsigned long long)(uint32_t)(R.nq[1] + kNormalBias) << 32);
+      const unsigned long long i3 = (unsigned long long)(uint32_t)(R.nq[2] + kNormalBias);
+      const uint32_t total = (uint32_t)nx * (uint32_t)ny * (uint32_t)nz;
+      for (uint32_t j = lane; j < total; j += 64) {
+        const int x = R.lo[0] + (int)(j % (uint32_t)nx), y = R.lo[1] + (int)((j / (uint32_t)nx) % (uint32_t)ny),
+                  z = R.lo[2] + (int)(j / ((uint32_t)nx * (uint32_t)ny));
+        const int32_t bb[3] = {x << VGI_FIXED_BITS, y << VGI_FIXED_BITS, z << VGI_FIXED_BITS};
+        if (!sat_box(q, N, bb, VGI_FIXED_BITS)) continue;
+        if constexpr (TEX) {
+          if (X.textured) {
+            int64_t e[3];
+            voxel_bary(q, N, R.axis, x, y, z, e);
+            uint32_t rgb;
+            if (!tex_albedo(X, e[0], e[1], e[2], rgb)) continue;  // discarded: nothing, not even the bit
+            i0 = (unsigned long long)(rgb & 0xFFu) | ((unsigned long long)((rgb >> 8) & 0xFFu) << 32);
+            i1 = (unsigned long long)((rgb >> 16) & 0xFFu) | (1ull << 32);
+          }
+        }
+        const uint32_t brick = ((uint32_t)x >> 3) + nbr * (((uint32_t)y >> 3) + nbr * ((uint32_t)z >> 3));
+        const uint32_t l = ((uint32_t)x & 7u) + 8u * ((uint32_t)y & 7u) + 64u * ((uint32_t)z & 7u);
+        unsigned long long* d64 = (unsigned long long*)(P.acc + ((size_t)brick * 512u + l) * kAccWords);
+        gatomic_add(d64 + 0, i0);
+        gatomic_add(d64 + 1, i1);
+        gatomic_add(d64 + 2, i2);
+        gatomic_add(d64 + 3, i3);
+        gatomic_or(P.mask + (size_t)brick * 16u + (l >> 5), 1u << (l & 31u));
+      }
+    }
+  }
+}
+
 // Registers: the 8^3 tile's unit accumulators (14 per thread) are held at 6 waves per SIMD
 // (80 VGPRs; 6 resident workgroups per CU, as many as LDS allows at 25.5 KB each), which
-// spills one 64-bit value per thread to scratch, reloaded at the flush. The kernel is
+// keeps the binned path in registers (only the fallback pass spills: as a launch of its own
+// it cost every call about 3 us to find nothing to do). The kernel is
 // latency-bound (dependent loads and barriers per chunk), so resident workgroups count:
 // 6 instead of 5 took the room's launch from 80 to 75 us.
 // TEX: the batch has a textured mesh; each triangle's texture inputs sit beside its
 // coefficients and a textured triangle samples its albedo per column (kept apart so that
 // untextured batches run the kernel without the sampler's registers and LDS).
 template <int TS, bool TEX>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TS == 8 && !TEX ? 6 : 1)))
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(TS == 8 ? (TEX ? 5 : 6) : 1)))
 void k_voxelize(VoxBatch Bt, const VoxScene* __restrict__ scenes) {
   constexpr int TV = TS * TS * TS;
   constexpr int NBK = TS / 8;  // 8^3 accumulator bricks per tile edge
@@ -1167,7 +1251,10 @@ void k_voxelize(VoxBatch Bt, const VoxScene* __restrict__ scenes) {
 
   const uint32_t tid = threadIdx.x;
   const uint32_t lane = tid & 63u;
-  if (gld(Bt.overflow) != 0u) return;  // the per-triangle kernel voxelizes this call
+  if (gld(Bt.overflow) != 0u) {  // uniform over the launch
+    fallback_pass<TEX>(Bt, scenes);
+    return;
+  }
   // the batch's work units, from the scan (the launch is sized from earlier calls: normally
   // one unit per workgroup, and workgroups take further units in turn when it falls short)
   const uint32_t nwork = (uint32_t)(gld(Bt.scan_all + Bt.total_bins) >> 32);
@@ -1352,79 +1439,5 @@ hipError_t launch_voxelize(const VoxBatch& B, uint32_t tile, uint32_t grid_block
   return hipGetLastError();
 }
 
-
-// ---------------------------------------------------------------------------
-// 7 overflow path: per-triangle voxelize with global atomics
-// ---------------------------------------------------------------------------
-
-// Runs only when k_scatter set the overflow word (and cleared every bin with pairs). A kernel of its own: inlined into k_voxelize it would spill that kernel's
-// registers, called from it the call would cut its occupancy. Wavefront w of the launch
-// takes triangles w, w + nwaves, ... of every scene; its
-// lanes walk the triangle's voxel box, keep the voxels the exact closed-box test accepts
-// (the same test as the bin pass, at voxel size) and add the triangle's increments: R, G,
-// B and the count, then the three biased normal components, as four 64-bit atomics (exact
-// with fewer than 2^21 triangles per voxel: no 32-bit word's total reaches 2^32), and set
-// the voxel's occupancy bit. Integer sums do not depend on order, so the accumulator is
-// the same as the binned path's.
-// Not inlined into k_voxelize, whose register budget (6 workgroups per CU) it would
-// otherwise share.
-template <bool TEX>
-__global__ __launch_bounds__(256) void k_voxelize_fallback(VoxBatch B, const VoxScene* __restrict__ scenes) {
-  if (gld(B.overflow) == 0u) return;
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6), nwaves = gridDim.x * (blockDim.x >> 6);
-  for (uint32_t sc = 0; sc < B.nscenes; sc++) {
-    const VoxScene& P = scenes[sc];
-    const uint32_t nbr = P.n >> 3;
-    for (uint32_t t = wave; t < P.ntri; t += nwaves) {
-      const TriRec R = gld_rec(P.tris + t);
-      if (!tri_ok(R)) continue;
-      int64_t q[3][3], N[3];
-      load_q(R, q, N);
-      const int nx = R.hi[0] - R.lo[0] + 1, ny = R.hi[1] - R.lo[1] + 1, nz = R.hi[2] - R.lo[2] + 1;
-      const uint32_t r = R.rgb & 0xFFu, g = (R.rgb >> 8) & 0xFFu, b = (R.rgb >> 16) & 0xFFu;
-      unsigned long long i0 = (unsigned long long)r | ((unsigned long long)g << 32);
-      unsigned long long i1 = (unsigned long long)b | (1ull << 32);
-      TexCoef X;
-      X.textured = 0;
-      if constexpr (TEX) load_texcoef(P, t, X);
-      const unsigned long long i2 = (unsigned long long)(uint32_t)(R.nq[0] + kNormalBias) |
-                                    ((unsigned long long)(uint32_t)(R.nq[1] + kNormalBias) << 32);
-      const unsigned long long i3 = (unsigned long long)(uint32_t)(R.nq[2] + kNormalBias);
-      const uint32_t total = (uint32_t)nx * (uint32_t)ny * (uint32_t)nz;
-      for (uint32_t j = lane; j < total; j += 64) {
-        const int x = R.lo[0] + (int)(j % (uint32_t)nx), y = R.lo[1] + (int)((j / (uint32_t)nx) % (uint32_t)ny),
-                  z = R.lo[2] + (int)(j / ((uint32_t)nx * (uint32_t)ny));
-        const int32_t bb[3] = {x << VGI_FIXED_BITS, y << VGI_FIXED_BITS, z << VGI_FIXED_BITS};
-        if (!sat_box(q, N, bb, VGI_FIXED_BITS)) continue;
-        if constexpr (TEX) {
-          if (X.textured) {
-            int64_t e[3];
-            voxel_bary(q, N, R.axis, x, y, z, e);
-            uint32_t rgb;
-            if (!tex_albedo(X, e[0], e[1], e[2], rgb)) continue;  // discarded: nothing, not even the bit
-            i0 = (unsigned long long)(rgb & 0xFFu) | ((unsigned long long)((rgb >> 8) & 0xFFu) << 32);
-            i1 = (unsigned long long)((rgb >> 16) & 0xFFu) | (1ull << 32);
-          }
-        }
-        const uint32_t brick = ((uint32_t)x >> 3) + nbr * (((uint32_t)y >> 3) + nbr * ((uint32_t)z >> 3));
-        const uint32_t l = ((uint32_t)x & 7u) + 8u * ((uint32_t)y & 7u) + 64u * ((uint32_t)z & 7u);
-        unsigned long long* d64 = (unsigned long long*)(P.acc + ((size_t)brick * 512u + l) * kAccWords);
-        gatomic_add(d64 + 0, i0);
-        gatomic_add(d64 + 1, i1);
-        gatomic_add(d64 + 2, i2);
-        gatomic_add(d64 + 3, i3);
-        gatomic_or(P.mask + (size_t)brick * 16u + (l >> 5), 1u << (l & 31u));
-      }
-    }
-  }
-}
-
-hipError_t launch_voxelize_fallback(const VoxBatch& B, uint32_t grid_blocks, hipStream_t s) {
-  if (grid_blocks == 0) return hipSuccess;
-  if (B.textured) hipLaunchKernelGGL(k_voxelize_fallback<true>, dim3(grid_blocks), dim3(256), 0, s, B, B.scenes);
-  else hipLaunchKernelGGL(k_voxelize_fallback<false>, dim3(grid_blocks), dim3(256), 0, s, B, B.scenes);
-  return hipGetLastError();
-}
 
 }  // namespace vgi

@@ -559,3 +559,40 @@ def test_cone_counts_vs_fp64(ctx, soup, num_diffuse, specular):
         norm = np.linalg.norm(ref)
         assert np.linalg.norm(got - ref) <= 1e-3 * norm if norm else not got.any()
     f.release()
+
+
+@pytest.mark.parametrize("meshes", [1, 120])
+def test_queued_calls_keep_their_descriptors(ctx, soup, meshes):
+    """Thirty frames queued without waiting, each with its own lights, eye and mesh split (more
+    calls than the ring of descriptor slots holds; 120 meshes take several copying
+    workgroups): every frame's output is the one it gives alone."""
+    vgi = _vgi()
+    w = soup["w"]
+    print(f"case queued calls, {meshes} meshes", flush=True)
+    pos = w.positions.reshape(-1, 9)
+    step = -(-len(pos) // meshes)
+    parts = [vgi.MeshData(ctx, pos[i:i + step].reshape(-1, 3), albedo=w.albedo[i:i + step])
+             for i in range(0, len(pos), step)]
+    grid = vgi.make_grid(**w.grid)
+    n = 64 * 24
+    gb = vgi.GBufferData(ctx, w.gb_pos[:n], w.gb_nrm[:n], 64, 24)
+    scene = ctx.scene()
+
+    def frame(k, od):
+        scene.voxelize(parts[: len(parts) - (k % 3) * (meshes > 1)], grid)
+        scene.build_mips(vgi.make_lights([dict(w.lights[0], color=(1.0 + k, 1.0, 2.0))]), vgi.PREC_FP32)
+        scene.trace(gb, vgi.make_cones(**dict(w.cones, eye=(0.1 * k, 0.5, 2.0))), od[0], od[1])
+
+    def outputs():
+        return [vgi.DeviceArray.empty(ctx, (n, 4), np.float32) for _ in range(2)]
+
+    queued = [outputs() for _ in range(30)]
+    for k, od in enumerate(queued):
+        frame(k, od)
+    ctx.sync()
+    for k, od in enumerate(queued):
+        alone = outputs()
+        frame(k, alone)
+        ctx.sync()
+        assert all(np.array_equal(a.numpy(), b.numpy()) for a, b in zip(od, alone)), k
+    scene.release()
