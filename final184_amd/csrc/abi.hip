@@ -546,8 +546,8 @@ struct VoxPlan {
 
 // The kernels of one voxelize call once its descriptors and scratch are in place: B holds
 // their device addresses, the zeroed_bytes at zb (bin counters, per-scene statistics, the
-// overflow word) are cleared first; the first wavefront of k_scatter settles the call
-// (statistics, overflow word). Everything after the scan reads its sizes on the device:
+// overflow word) are cleared first; k_scatter takes the overflow decision, k_voxelize's last
+// workgroup settles the call (statistics). Everything after the scan reads its sizes on the device:
 // k_scatter's role blocks are sized from the host's counts (triangle and bin blocks) and
 // persistent for the
 // large triangles and the split bins, whose counts only the device knows; k_voxelize takes

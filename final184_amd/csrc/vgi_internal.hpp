@@ -61,7 +61,7 @@ struct __align__(16) TriRec {
   uint8_t pad0;
   int16_t lo[3];      // voxel bounding box clipped to the grid (inclusive); lo > hi if empty
   int16_t hi[3];
-  uint32_t pad1;
+  uint32_t hits;      // small triangles: bit j set if it overlaps the j-th bin of its bin box
 };
 static_assert(sizeof(TriRec) == 64, "TriRec layout");
 
@@ -80,8 +80,8 @@ constexpr uint32_t kHostHistWords = 5;
 // Default polls of a predecessor's flag before the bin scan's look-back gives up.
 constexpr uint32_t kScanSpin = 1u << 22;
 
-// A scene's result of one voxelize call, stored by the settle step (the first wavefront of
-// k_scatter, after the bin scan) into the scene's pinned host record, seq once the other
+// A scene's result of one voxelize call, stored by the settle step (a wavefront of
+// k_voxelize, after the bin scan) into the scene's pinned host record, seq once the other
 // words are complete: the record is whole once seq equals the call's number (read by
 // vgi_scene_get_stats).
 struct SceneVoxResult {

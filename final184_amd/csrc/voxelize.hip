@@ -25,14 +25,15 @@
 //                   bins with > 1 unit are listed. In the same pass:
 //   4 scan          one 64-bit exclusive scan over the batch (a look-back between the
 //                   workgroups) gives every bin its pair offset and its first work unit.
-//   5 k_scatter     one launch; its first wavefront settles the call (per-scene totals
-//                   and statistics to the host records, the overflow word for steps 6
-//                   and 7); work unit -> (scene, bin) and the units' order (those of
-//                   two or more chunks first); small triangles to their kept
-//                   slots (no atomics); large triangles after the small ones of each bin;
-//                   clear the accumulator and occupancy mask of bins with several units.
-//   6 k_voxelize    one workgroup per work unit of the batch, in that order; per work item
-//                   (chunk) of it:
+//   5 k_scatter     one launch; it takes the overflow decision for steps 6 and 7; large
+//                   triangles after the small ones of each bin; work unit -> (scene, bin)
+//                   and the units' order (those of two or more chunks first); small
+//                   triangles to their kept slots (no atomics, no bin tests: k_setup left the
+//                   overlapped bins in the record); clear the accumulator and occupancy mask
+//                   of bins with several units.
+//   6 k_voxelize    its last workgroup settles the call (per-scene totals and statistics to
+//                   the host records); one workgroup per work unit of the batch, in that
+//                   order; per work item (chunk) of it:
 //                   triangles' edge/plane coefficients to LDS, columns of the dominant-axis
 //                   projection spread over the workgroup, each column tests its 1-4
 //                   candidate voxels with the exact separating-axis test and adds packed
@@ -146,6 +147,18 @@ __device__ __forceinline__ uint32_t find_mesh(const MeshDev* __restrict__ m, uin
   return lo;
 }
 
+// The same for a wave-uniform triangle, its steps' loads through the scalar cache.
+__device__ __forceinline__ uint32_t find_mesh_uniform(const MeshDev* __restrict__ m, uint32_t nmesh, uint32_t t) {
+  typedef const __attribute__((address_space(4))) uint32_t cu32;
+  uint32_t lo = 0, hi = nmesh - 1;
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi + 1) >> 1;
+    if (*(cu32*)&m[mid].tri_base <= t) lo = mid;
+    else hi = mid - 1;
+  }
+  return lo;
+}
+
 // Exact closed-box test of a triangle against [b, b + d]^3 (fixed-point units, d = 2^dshift),
 // with the bounding boxes already known to overlap. Magnitudes: |q| <= 2^18 (the snap guard),
 // 0 <= b <= 2^18, so |b - q| <= 2^19 and |edge| <= 2^19 fit int32; |N| <= 2^39, d <= 2^13.
@@ -235,6 +248,11 @@ __device__ __forceinline__ bool bin_candidate(const VoxScene& S, const int64_t (
   return sat_box(q, N, b, dshift);
 }
 
+// a / b for a < 8 and 1 <= b <= 8
+__device__ __forceinline__ uint32_t small_div(uint32_t a, uint32_t b) {
+  return (uint32_t)(((float)a + 0.5f) * __builtin_amdgcn_rcpf((float)b));
+}
+
 // Index of bin b's counter in bin_small / bin_big / big_cursor. Bins are scattered over the
 // counter array by an odd multiplier (a bijection modulo the power-of-two bin count), so
 // spatially adjacent bins -- a wall's run of bins, each hit by many workgroups -- do not
@@ -268,13 +286,18 @@ __device__ __forceinline__ uint32_t first_item(const VoxBatch& B, const VoxScene
 // 1 setup
 // ---------------------------------------------------------------------------
 
-__device__ void make_record(const VoxScene& P, uint32_t t, TriRec& R) {
+// Fills R; true if the grid clips the triangle's voxel box.
+__device__ bool make_record(const VoxScene& P, uint32_t t, TriRec& R) {
   // the mesh descriptor: through the scalar cache when the wavefront's triangles share
   // one mesh (the usual case), which shortens the fetch chain ahead of the index loads
-  const uint32_t mi = find_mesh(P.meshes, P.nmesh, t);
-  const uint32_t mi0 = __builtin_amdgcn_readfirstlane(mi);
+  // (the search likewise: for the wavefront's first triangle with scalar loads, and per lane
+  // only where the last lane's triangle lies beyond that mesh)
+  const uint32_t mi0 = find_mesh_uniform(P.meshes, P.nmesh, __builtin_amdgcn_readfirstlane(t));
+  const MeshDev M0 = sld_rec(P.meshes + mi0);
+  uint32_t mi = mi0;
+  if (!__all(t - M0.tri_base < M0.ntri)) mi = find_mesh(P.meshes, P.nmesh, t);
   MeshDev M;
-  if (__all(mi == mi0)) M = sld_rec(P.meshes + mi0);
+  if (__all(mi == mi0)) M = M0;
   else M = gld_rec(P.meshes + mi);
   const uint32_t lt = t - M.tri_base;
   uint32_t vid[3];
@@ -325,7 +348,7 @@ __device__ void make_record(const VoxScene& P, uint32_t t, TriRec& R) {
   R.nq[0] = R.nq[1] = R.nq[2] = 0;
   R.axis = 2;
   R.pad0 = 0;
-  R.pad1 = 0;
+  R.hits = 0;
   int64_t N[3] = {0, 0, 0};
   if (status == 0) {
     int64_t q[3][3];
@@ -339,6 +362,7 @@ __device__ void make_record(const VoxScene& P, uint32_t t, TriRec& R) {
   } else {
     rgb = M.base_rgb & 0xFFFFFFu;
   }
+  bool clipped = false;
 #pragma unroll
   for (int a = 0; a < 3; a++) { R.lo[a] = 1; R.hi[a] = 0; }
   if (status == 0) {
@@ -361,6 +385,7 @@ __device__ void make_record(const VoxScene& P, uint32_t t, TriRec& R) {
       const int32_t mx = max(qi[0][a], max(qi[1][a], qi[2][a]));
       const int32_t l = max((mn - 1) >> 8, 0);               // floor((mn-1)/256)
       const int32_t h = min(mx >> 8, (int32_t)P.n - 1);      // floor(mx/256)
+      clipped = clipped || l != (mn - 1) >> 8 || h != mx >> 8;
       lo[a] = (int16_t)l;
       hi[a] = (int16_t)h;
       empty = empty || l > h;
@@ -370,6 +395,7 @@ __device__ void make_record(const VoxScene& P, uint32_t t, TriRec& R) {
       for (int a = 0; a < 3; a++) { R.lo[a] = lo[a]; R.hi[a] = hi[a]; }
   }
   R.rgb = rgb | (status << 24);
+  return clipped;
 }
 
 // Slots of small triangles in their bins, aggregated per workgroup: each (triangle, bin)
@@ -382,14 +408,29 @@ constexpr uint32_t kSlotTable = 1024;  // distinct bins per workgroup before ove
 constexpr uint32_t kProbe = 32;
 constexpr uint32_t kNoKey = 0xFFFFFFFFu;
 
+// Which of its bins a small triangle overlaps. In a box with more than one bin on at most one
+// axis every bin is: the triangle lies within the box (its voxel box is not clipped by the
+// grid), so the point of it in a bin's slab along that axis is in the bin. About five of six
+// triangles of a few voxels need no test. The others' (triangle, bin) candidates are listed
+// in LDS and tested by all threads in turn, one each: with every thread testing its own
+// triangle's, a wavefront ran eight exact tests for its few lanes that had them.
 __global__ __launch_bounds__(256) void k_setup(VoxBatch B, const VoxScene* __restrict__ scenes) {
   __shared__ uint32_t s_key[kSlotTable], s_cnt[kSlotTable], s_base[kSlotTable];
   __shared__ uint32_t s_big_n, s_big_base;  // the workgroup's large triangles and their list run
+  __shared__ uint32_t s_npair;              // listed candidates
+  __shared__ uint16_t s_pair[kBlockTris * kSmallBins];  // thread | candidate << 8
+  __shared__ uint32_t s_hits[kBlockTris];
+  __shared__ int32_t s_q[9][kBlockTris];
+  __shared__ uint32_t s_box[kBlockTris];  // first bin x | y << 8 | z << 16 | nx - 1 << 24 | ny - 1 << 27
   for (uint32_t e = threadIdx.x; e < kSlotTable; e += blockDim.x) {
     s_key[e] = kNoKey;
     s_cnt[e] = 0u;
   }
-  if (threadIdx.x == 0) s_big_n = 0u;
+  s_hits[threadIdx.x] = 0u;
+  if (threadIdx.x == 0) {
+    s_big_n = 0u;
+    s_npair = 0u;
+  }
   const uint2 blk = tri_block(B);  // a workgroup never spans two scenes
   const VoxScene& P = scenes[blk.x];
   const uint32_t t = blk.y + threadIdx.x;
@@ -397,21 +438,26 @@ __global__ __launch_bounds__(256) void k_setup(VoxBatch B, const VoxScene* __res
   TriRec R;
   bool small = false, big = false;
   BinBox bb{0, 0, 0, 0, 0, 0};
-  int64_t q[3][3], N[3];
+  uint32_t hits = 0;   // bit j: the triangle overlaps the j-th bin of its box
+  uint32_t ntest = 0;  // candidates to test
   if (in) {
-    make_record(P, t, R);
-    gst_rec(P.tris + t, R);
+    const bool clipped = make_record(P, t, R);
     const uint32_t status = R.rgb >> 24;
     if (status == 1) gatomic_add(&P.stats->rejected, 1ull);
     if (status == 2) gatomic_add(&P.stats->degenerate, 1ull);
     if (tri_ok(R)) {
       bb = bin_box(R, P.bin_shift);
-      small = bb.count() <= kSmallBins;
+      const int n = bb.count();
+      small = n <= kSmallBins;
       big = !small;
-      if (small) load_q(R, q, N);
+      if (small) {
+        const bool line = n == max(bb.nx, max(bb.ny, bb.nz));  // more than one bin on at most one axis
+        if (line && !clipped) hits = (1u << n) - 1u;
+        else ntest = (uint32_t)n;
+      }
     }
   }
-  __syncthreads();  // table and large-triangle count cleared
+  __syncthreads();  // tables and counts cleared
   // large triangles: a rank within the workgroup (one LDS atomic per wavefront); the
   // workgroup's run of the list is reserved with one global atomic beside the bin
   // reservations below, and the ids are written after it
@@ -426,16 +472,43 @@ __global__ __launch_bounds__(256) void k_setup(VoxBatch B, const VoxScene* __res
       big_rank = __shfl(base, leader) + (uint32_t)__popcll(bm & ((1ull << lane) - 1ull));
     }
   }
+  if (ntest != 0u) {
+    const uint32_t k = atomicAdd(&s_npair, ntest);
+    for (uint32_t j = 0; j < ntest; j++) s_pair[k + j] = (uint16_t)(threadIdx.x | (j << 8));
+#pragma unroll
+    for (int i = 0; i < 9; i++) s_q[i][threadIdx.x] = R.q[i];
+    // bins per axis <= 128, at most 8 of them in the box
+    s_box[threadIdx.x] = (uint32_t)bb.x0 | ((uint32_t)bb.y0 << 8) | ((uint32_t)bb.z0 << 16) |
+                         ((uint32_t)(bb.nx - 1) << 24) | ((uint32_t)(bb.ny - 1) << 27);
+  }
+  __syncthreads();
+  for (uint32_t k = threadIdx.x; k < s_npair; k += kBlockTris) {
+    const uint32_t e = s_pair[k], o = e & 255u, j = e >> 8, box = s_box[o];
+    TriRec T;
+#pragma unroll
+    for (int i = 0; i < 9; i++) T.q[i] = s_q[i][o];
+    int64_t q[3][3], N[3];
+    load_q(T, q, N);
+    const uint32_t nx = ((box >> 24) & 7u) + 1u, ny = ((box >> 27) & 7u) + 1u;
+    const uint32_t jy = small_div(j, nx), jz = small_div(jy, ny);
+    const uint32_t dshift = VGI_FIXED_BITS + P.bin_shift;
+    const int32_t c[3] = {(int32_t)(((box & 255u) + j - jy * nx) << dshift),
+                          (int32_t)((((box >> 8) & 255u) + jy - jz * ny) << dshift),
+                          (int32_t)((((box >> 16) & 255u) + jz) << dshift)};  // <= n * 256 <= 2^18
+    if (sat_box(q, N, c, dshift)) atomicOr(&s_hits[o], 1u << j);
+  }
+  __syncthreads();
+  if (ntest != 0u) hits = s_hits[threadIdx.x];
   // rank each (triangle, bin) pair within the workgroup
   uint32_t ent[kSmallBins], rank[kSmallBins];  // table entry (or kNoKey: own atomic) and rank
-  uint32_t hits = 0;                           // bit j: candidate j overlaps its bin
 #pragma unroll
   for (int j = 0; j < kSmallBins; j++) {
     ent[j] = kNoKey;
     rank[j] = 0;
-    uint32_t bin = 0;
-    if (small && j < bb.count() && bin_candidate(P, q, N, bb, j, bin)) {
-      hits |= 1u << j;
+    if ((hits >> j) & 1u) {
+      const uint32_t jy = small_div((uint32_t)j, (uint32_t)bb.nx), jz = small_div(jy, (uint32_t)bb.ny);
+      const uint32_t bin = (uint32_t)bb.x0 + (uint32_t)j - jy * (uint32_t)bb.nx +
+                           P.nbins_axis * ((uint32_t)bb.y0 + jy - jz * (uint32_t)bb.ny + P.nbins_axis * ((uint32_t)bb.z0 + jz));
       uint32_t h = (bin * 0x9E3779B1u) >> 22;  // 10-bit hash
       for (uint32_t probe = 0; probe < kProbe; probe++) {
         const uint32_t k = atomicCAS(&s_key[h], kNoKey, bin);
@@ -448,6 +521,10 @@ __global__ __launch_bounds__(256) void k_setup(VoxBatch B, const VoxScene* __res
       }
       if (ent[j] == kNoKey) rank[j] = gatomic_add(P.bin_small + ctr(P, bin), 1u);  // table overflow
     }
+  }
+  if (in) {  // with the overlapped bins, so that k_scatter need not test them again
+    R.hits = hits;
+    gst_rec(P.tris + t, R);
   }
   __syncthreads();
   {  // reserve every listed bin's run (all four returning atomics in flight together) and
@@ -663,20 +740,16 @@ hipError_t launch_bins(const VoxBatch& B, uint32_t blocks, hipStream_t s) {
   return hipGetLastError();
 }
 
-// The settle step, after the scan (the first wavefront of k_scatter; every wavefront of
-// k_scatter takes the overflow decision itself, call_overflow): each scene's totals (work
-// units << 32 | pairs of its bins) and statistics go to its pinned host record; the
-// batch's exact pair count (a 64-bit sum of the per-scene counts, which the packed 32-bit
-// field cannot hold beyond 2^32) and unit count are checked against the pair list and
-// work map the host sized, and the overflow word tells steps 6-7 which path to take (it
-// was a kernel of its own, k_settle: folding it into k_scatter saved a launch, about
-// 3 us a frame). The batch totals (pairs, units,
-// large triangles, split bins) go to the stream's pinned history, from which the host
-// sizes later calls. Both are coherent host memory, written with system-scope stores; each
-// record's call number (and the history's) is stored once the other words are complete,
-// and the host reads a record once it finds the call's number there. No event is recorded
-// between the call's kernels for it: on the room each event between two kernels left the
-// GPU idle about 4 us (the two this replaced, 7.8 us of a 0.89 ms frame).
+// The settle step, after the scan (one wavefront of k_voxelize's last workgroup, which takes
+// no units, so that the round trips to host memory hide behind the launch; every wavefront
+// of k_scatter takes the overflow decision itself, call_overflow): each scene's totals (work
+// units << 32 | pairs of its bins) and statistics go to its pinned host record; the batch
+// totals (pairs, units, large triangles, split bins) go to the stream's pinned history, from
+// which the host sizes later calls. Both are coherent host memory, written with system-scope
+// stores; each record's call number (and the history's) is stored once the other words are
+// complete, and the host reads a record once it finds the call's number there. No event is
+// recorded between the call's kernels for it: on the room each event between two kernels
+// left the GPU idle about 4 us.
 // a store to coherent host memory performed at system scope (written through the caches)
 __device__ __forceinline__ void sys_store(unsigned long long* p, unsigned long long v) {
   __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
@@ -704,8 +777,8 @@ __device__ __forceinline__ uint32_t call_overflow(const VoxBatch& B, const VoxSc
   return (pairs > B.pair_cap || units > B.work_cap || gld(B.overflow + 3) != 0u) ? 1u : 0u;
 }
 
-// The settle step, by one wavefront (the first of k_scatter's first workgroup).
-__device__ void settle_wave(const VoxBatch& B, const VoxScene* __restrict__ scenes, uint32_t ovf) {
+__device__ void settle_wave(const VoxBatch& B, const VoxScene* __restrict__ scenes) {
+  const uint32_t ovf = gld(B.overflow);
   const uint32_t lane = __lane_id();
   unsigned long long pairs = 0, big = 0, split = 0;
   for (uint32_t sc = lane; sc < B.nscenes; sc += 64) {
@@ -744,7 +817,6 @@ __device__ void settle_wave(const VoxBatch& B, const VoxScene* __restrict__ scen
     sys_store_last(dst + kSeqWord, src[kSeqWord]);
   }
   if (lane == 0) {
-    gst(B.overflow, ovf);
     sys_store(B.host_hist + 0, pairs);
     sys_store(B.host_hist + 1, (unsigned long long)units);
     sys_store(B.host_hist + 2, big);
@@ -819,19 +891,38 @@ __device__ __forceinline__ void emit_small_block(const VoxBatch& B, const VoxSce
   const VoxScene& P = scenes[blk.x];
   const uint32_t t = blk.y + threadIdx.x;
   if (t >= P.ntri) return;
-  const TriRec R = gld_rec(P.tris + t);
-  if (!tri_ok(R)) return;
-  const BinBox bb = bin_box(R, P.bin_shift);
-  if (bb.count() > kSmallBins) return;
-  int64_t q[3][3], N[3];
-  load_q(R, q, N);
-  uint32_t nslot = 0;
-  for (int j = 0; j < bb.count(); j++) {
-    uint32_t bin;
-    if (!bin_candidate(P, q, N, bb, j, bin)) continue;
-    const uint32_t pos = pair_base(B, P, bin) + gld(P.tri_slot + (size_t)t * kSmallBins + nslot++);
-    if (pos < B.pair_cap) gst(B.pairs_all + pos, t);
+  // the box and the bins that k_setup found overlapped are the record's last 16 bytes; with
+  // the kept slots they are all this needs (testing the bins again took most of the launch)
+  struct Box {
+    int16_t lo[3], hi[3];
+    uint32_t hits;
+  };
+  static_assert(sizeof(Box) == 16 && offsetof(TriRec, lo) == 48 && offsetof(TriRec, hits) == 60, "a record's tail");
+  const Box R = __builtin_bit_cast(Box, gld4((const uint4*)(P.tris + t) + 3));
+  if (R.hits == 0u) return;  // rejected, degenerate, outside the grid, or a large triangle
+  const int bs = (int)P.bin_shift;
+  const int x0 = R.lo[0] >> bs, y0 = R.lo[1] >> bs, z0 = R.lo[2] >> bs;
+  const int nx = (R.hi[0] >> bs) - x0 + 1, ny = (R.hi[1] >> bs) - y0 + 1;  // nx ny nz <= 8
+  const uint4* sp = (const uint4*)(P.tri_slot + (size_t)t * kSmallBins);
+  const uint4 s0 = gld4(sp), s1 = gld4(sp + 1);  // all eight in flight; the used ones come first
+  const uint32_t slot[kSmallBins] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+  uint32_t base[kSmallBins];
+  uint32_t m = R.hits;
+#pragma unroll
+  for (int i = 0; i < kSmallBins; i++) {  // the i-th overlapped bin
+    base[i] = 0xFFFFFFFFu;
+    if (m != 0u) {
+      const int j = __builtin_ctz(m);
+      const int jy = (int)small_div((uint32_t)j, (uint32_t)nx), jz = (int)small_div((uint32_t)jy, (uint32_t)ny);
+      const int bx = x0 + j - jy * nx, by = y0 + jy - jz * ny, bz = z0 + jz;
+      base[i] = pair_base(B, P, (uint32_t)bx + P.nbins_axis * ((uint32_t)by + P.nbins_axis * (uint32_t)bz));
+      m &= m - 1u;
+    }
   }
+  const uint32_t n = (uint32_t)__builtin_popcount(R.hits);
+#pragma unroll
+  for (uint32_t i = 0; i < (uint32_t)kSmallBins; i++)
+    if (i < n && base[i] + slot[i] < B.pair_cap) gst(B.pairs_all + base[i] + slot[i], t);
 }
 
 // Workgroups blk, blk + nblk, ... of the listed bins clear them.
@@ -876,29 +967,29 @@ __device__ __forceinline__ void clear_bins_block(const VoxBatch& Bt, const VoxSc
   }
 }
 
-// One launch after the scan, before k_voxelize: workgroups [0, nblk_b) map work units, the
-// next nblk_t scatter small triangles, the next nblk_big place large triangles (one
-// wavefront each), the rest clear the bins that several work units add into (none on most
-// scenes). They write disjoint outputs. When the pair list or the work map would overflow,
-// workgroups [0, nblk_b) clear every bin with pairs instead and the rest do nothing.
+// One launch after the scan, before k_voxelize: the first nblk_big workgroups place large
+// triangles (one wavefront each; first, since each is a chain of dependent loads and a
+// returning atomic per bin), the next nblk_b map work units, the next nblk_t scatter small
+// triangles, the rest clear the bins that several work units add into (none on most scenes).
+// They write disjoint outputs. When the pair list or the work map would overflow, the nblk_b
+// workgroups clear every bin with pairs instead and the rest do nothing.
 __global__ __launch_bounds__(256) void k_scatter(VoxBatch B, const VoxScene* __restrict__ scenes, uint32_t nblk_b,
                                                  uint32_t nblk_t, uint32_t nblk_big) {
   const uint32_t b = blockIdx.x;
   const uint32_t ovf = call_overflow(B, scenes);  // the same in every wavefront
-  if (b == 0 && threadIdx.x < 64) settle_wave(B, scenes, ovf);
+  if (b == 0 && threadIdx.x == 0) gst(B.overflow, ovf);
   if (ovf != 0u) {
-    if (b < nblk_b) clear_bins_block(B, scenes, b);
+    if (b >= nblk_big && b < nblk_big + nblk_b) clear_bins_block(B, scenes, b - nblk_big);
     return;
   }
-  if (b < nblk_b) {
-    workmap_block(B, scenes, b);
-  } else if (b < nblk_b + nblk_t) {
-    emit_small_block(B, scenes, b - nblk_b);
-  } else if (b < nblk_b + nblk_t + nblk_big) {
-    const uint32_t w0 = b - nblk_b - nblk_t;
-    big_pass<true>(B, scenes, w0 * (blockDim.x >> 6) + (threadIdx.x >> 6), nblk_big * (blockDim.x >> 6));
+  if (b < nblk_big) {
+    big_pass<true>(B, scenes, b * (blockDim.x >> 6) + (threadIdx.x >> 6), nblk_big * (blockDim.x >> 6));
+  } else if (b < nblk_big + nblk_b) {
+    workmap_block(B, scenes, b - nblk_big);
+  } else if (b < nblk_big + nblk_b + nblk_t) {
+    emit_small_block(B, scenes, b - nblk_big - nblk_b);
   } else {
-    const uint32_t first = nblk_b + nblk_t + nblk_big;
+    const uint32_t first = nblk_big + nblk_b + nblk_t;
     zero_pass(B, scenes, b - first, gridDim.x - first);
   }
 }
@@ -1177,9 +1268,9 @@ struct TileLayout {
 // reaches 2^32), and set the voxel's occupancy bit. Integer sums do not depend on order, so
 // the accumulator is the same as the binned path's.
 template <bool TEX>
-__device__ __forceinline__ void fallback_pass(const VoxBatch& B, const VoxScene* __restrict__ scenes) {
+__device__ __forceinline__ void fallback_pass(const VoxBatch& B, const VoxScene* __restrict__ scenes, uint32_t nwg) {
   const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6), nwaves = gridDim.x * (blockDim.x >> 6);
+  const uint32_t wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6), nwaves = nwg * (blockDim.x >> 6);
   for (uint32_t sc = 0; sc < B.nscenes; sc++) {
     const VoxScene& P = scenes[sc];
     const uint32_t nbr = P.n >> 3;
@@ -1251,15 +1342,20 @@ void k_voxelize(VoxBatch Bt, const VoxScene* __restrict__ scenes) {
 
   const uint32_t tid = threadIdx.x;
   const uint32_t lane = tid & 63u;
+  const uint32_t nwg = gridDim.x - 1u;  // workgroups that voxelize; the last one settles the call
+  if (blockIdx.x == nwg) {
+    if (tid < 64u) settle_wave(Bt, scenes);
+    return;
+  }
   if (gld(Bt.overflow) != 0u) {  // uniform over the launch
-    fallback_pass<TEX>(Bt, scenes);
+    fallback_pass<TEX>(Bt, scenes, nwg);
     return;
   }
   // the batch's work units, from the scan (the launch is sized from earlier calls: normally
   // one unit per workgroup, and workgroups take further units in turn when it falls short)
   const uint32_t nwork = (uint32_t)(gld(Bt.scan_all + Bt.total_bins) >> 32);
 
-  for (uint32_t w = blockIdx.x; w < nwork; w += gridDim.x) {
+  for (uint32_t w = blockIdx.x; w < nwork; w += nwg) {
     const uint32_t u = gld(Bt.unit_order + w);  // the longest units first
     const uint2 item = gld2(Bt.work_map + u);
     const VoxScene& P = scenes[item.x];
@@ -1429,6 +1525,7 @@ void k_voxelize(VoxBatch Bt, const VoxScene* __restrict__ scenes) {
 hipError_t launch_voxelize(const VoxBatch& B, uint32_t tile, uint32_t grid_blocks, hipStream_t s) {
   if (grid_blocks == 0) return hipSuccess;
   static_assert(TileLayout<8>::ENTRIES == 582 && TileLayout<16>::ENTRIES == 4366, "tile layout");
+  grid_blocks += 1;  // the settling workgroup
   if (B.textured) {
     if (tile == 8) hipLaunchKernelGGL((k_voxelize<8, true>), dim3(grid_blocks), dim3(256), 0, s, B, B.scenes);
     else hipLaunchKernelGGL((k_voxelize<16, true>), dim3(grid_blocks), dim3(256), 0, s, B, B.scenes);

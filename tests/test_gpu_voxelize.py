@@ -305,3 +305,27 @@ def test_scan_lookback_giving_up_takes_per_triangle_path(monkeypatch):
         assert np.array_equal(acc, ref), _diff_msg(acc, ref)
     finally:
         c.close()
+
+
+@pytest.mark.parametrize("span,lattice", [(1, 1), (2, 4), (3, 8), (9, 2)])
+@pytest.mark.parametrize("nmeshes", [1, 37])
+def test_triangles_on_bin_faces_match_oracle(ctx, span, lattice, nmeshes):
+    """Vertices on a lattice of whole voxels around and beyond the grid: triangles that touch
+    bins at faces, edges and corners only, that stay within one bin or a row of bins, and
+    that the grid clips. Meshes of a few triangles each put several meshes in a wavefront."""
+    vgi = _vgi()
+    n, count = 64, 4000
+    rng = np.random.default_rng(span * 100 + lattice)
+    base = rng.integers(-8 // lattice, (n + 8) // lattice + 1, (count, 1, 3)) * lattice
+    off = rng.integers(-span, span + 1, (count, 3, 3)) * lattice
+    pos = np.ascontiguousarray(((base + off) / n).astype(np.float32).reshape(count, 9))
+    alb = rng.integers(0, 256, (count, 3), dtype=np.uint8)
+    grid = dict(origin=(0.0, 0.0, 0.0), extent=1.0, n=n, levels=6)
+    print(f"case bin faces span={span} lattice={lattice} meshes={nmeshes}", flush=True)
+    step = -(-count // nmeshes)
+    meshes = [vgi.MeshData(ctx, pos[i:i + step].reshape(-1, 3), albedo=alb[i:i + step]) for i in range(0, count, step)]
+    s = ctx.scene()
+    s.voxelize(meshes, vgi.make_grid(**grid))
+    ref, _ = orc.voxelize(pos, grid, albedo=alb)
+    assert np.array_equal(s.read_voxels(), ref)
+    s.release()
