@@ -1119,6 +1119,19 @@ uint32_t trace_wavefronts(size_t blocks, uint32_t cones, uint32_t diffuse, bool 
   return std::max(1u, std::min(w, cones));
 }
 
+// Up to here a launch leaves most of each CU's wavefront slots empty, its length is that of
+// the specular cone's chain of samples, and a block's wavefronts march that cone together
+// (k_trace SHARED): twelve of them, for FP32, whose footprints keep L1 busier, eight (room, 9
+// + 1 cones: 96 x 54 pixels FP16 x-pair 44.7 us dealt, 37.2 / 31.5 / 31.3 with 8 / 12 / 16,
+// FP16 47.6 / 39.4 / 32.2 / 32.3, FP32 53.9 / 51.1 / 49.4 / 48.7; 256 x 144, 576 blocks:
+// 54.8 / 55.6 / 45.9 / 60.4 and FP32 89.1 / 79.7 / 81.2; 256 x 256, 1024 blocks: 58.9 /
+// 65.0 / 60.4, FP32 94.9 / 94.7 / 112.5).
+constexpr size_t kSharedTraceBlocks = 600;
+uint32_t shared_wavefronts(uint32_t prec, uint32_t cones, uint32_t diffuse) {
+  const uint32_t w = prec == VGI_PREC_FP32 ? 8u : 12u;
+  return cones > diffuse ? w : std::max(1u, std::min(w, diffuse));  // (no specular cone: one each)
+}
+
 // March schedule of a cone whose sample distances do not depend on the pixel (a fixed
 // aperture): the per-pixel recurrence of the cone march evaluated once, in FP32 -- diameter
 // d = max(h, 2 t tan), level max(0, log2(d / h)), next t = t + step d -- while
@@ -1171,7 +1184,7 @@ int trace_batch(vgi_context* ctx, const vgi_trace_item* items, uint32_t count, v
     uint32_t band;  // work items an XCD takes in a row (k_trace's block order)
     uint32_t waves, max_diffuse;
     size_t items;   // screen tiles
-    bool full;
+    bool full, shared;
   };
   // per item: its parameters and the schedules of its fixed-aperture cones
   std::vector<TraceParams> tp(count);
@@ -1187,7 +1200,7 @@ int trace_batch(vgi_context* ctx, const vgi_trace_item* items, uint32_t count, v
   size_t max_entries = 0;
   for (uint32_t p = 0; p < kPrecisions; p++) {
     if (group[p].empty()) continue;
-    Launch L{p, (uint32_t)group[p].size(), 0, 0, 0, 0, 0, 0, 0, tn.address_mode == VGI_ADDRESS_AUTO, 0, 0, 0, 0, false};
+    Launch L{p, (uint32_t)group[p].size(), 0, 0, 0, 0, 0, 0, 0, tn.address_mode == VGI_ADDRESS_AUTO, 0, 0, 0, 0, false, false};
     uint32_t cones = 0;
     for (uint32_t i : group[p]) {
       L.nsched += sched[2 * i].size() + sched[2 * i + 1].size();
@@ -1203,7 +1216,8 @@ int trace_batch(vgi_context* ctx, const vgi_trace_item* items, uint32_t count, v
     L.nblocks = morton ? L.entries / 64 : L.items << sub_shift;
     // bands of kTraceBandRows rows of the first item's tiles
     L.band = morton ? 0u : kTraceBandRows * (tp[group[p][0]].tiles_x << sub_shift);
-    L.waves = trace_wavefronts(L.nblocks, cones, L.max_diffuse, morton);
+    L.shared = L.buffer_path && L.nblocks <= kSharedTraceBlocks;
+    L.waves = L.shared ? shared_wavefronts(p, cones, L.max_diffuse) : trace_wavefronts(L.nblocks, cones, L.max_diffuse, morton);
     L.full = L.nblocks >= kFullTraceBlocks;
     if (L.nblocks >= (1ull << 31) || L.entries >= (1ull << 32))
       return fail(VGI_E_RANGE, "trace batch too large (%zu workgroups)", L.nblocks);
@@ -1280,6 +1294,7 @@ int trace_batch(vgi_context* ctx, const vgi_trace_item* items, uint32_t count, v
       B.waves = L.waves;
       B.full = L.full ? 1u : 0u;
       B.max_diffuse = L.max_diffuse;
+      B.shared = L.shared ? 1u : 0u;
       if (morton && L.entries > 0) {
         unsigned long long* keys = (unsigned long long*)w->sort_keys;
         uint32_t* pix = (uint32_t*)w->sort_pix;

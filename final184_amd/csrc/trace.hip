@@ -419,16 +419,32 @@ __device__ __forceinline__ float cone_origin(float o, float origin, float inv_h)
   return fmaf(o - origin, inv_h, 0.0f);
 }
 
+// One sample of a schedule: quadrilinear (levels l0 + 1 and l0), or the top level alone.
+//
+// The coarse footprint (level l0 + 1) holds the parents of every fine (level l0) footprint
+// texel. When the coarse footprint's opacity is zero and zero opacity implies an all-zero
+// subtree, the fine gather is exactly zero and is skipped (skip_fine_ok).
+template <int PREC>
+__device__ __forceinline__ void fixed_sample(const TraceParams& P, const SchedEntry& e, float ux, float uy, float uz,
+                                             float4& s, uint32_t& count) {
+  uint32_t abits = 0;
+  if (e.code & kSchedTop) {
+    gather_uniform<PREC, true>(P, e.code & ~kSchedTop, ux, uy, uz, 1.0f, kHalfOne, s, abits);
+    count += 1;
+  } else {
+    gather_uniform<PREC, true>(P, e.code + 1, ux, uy, uz, e.fr, e.hfr, s, abits);
+    if (abits || !skip_fine_ok<PREC>(e.code))
+      gather_uniform<PREC, false>(P, e.code, ux, uy, uz, e.gr, e.hgr, s, abits);
+    count += 2;
+  }
+}
+
 // One fixed-aperture cone: its samples (distance, levels, level weights) come from the
 // schedule the host computed once for the aperture, read with scalar loads, so the whole
 // wavefront takes each sample at the same distance and level with no per-lane schedule
 // arithmetic. Sample: quadrilinear gather (levels l0 + 1 and l0, or the top level alone),
 // then front-to-back compositing; the march ends at the schedule's end (max distance),
 // the grid boundary or opacity >= cutoff.
-//
-// The coarse footprint (level l0 + 1) holds the parents of every fine (level l0) footprint
-// texel. When the coarse footprint's opacity is zero and zero opacity implies an all-zero
-// subtree, the fine gather is exactly zero and is skipped (skip_fine_ok).
 template <int PREC>
 __device__ __forceinline__ float4 cone_march_fixed(const TraceParams& P, const SchedEntry* __restrict__ sched,
                                                    uint32_t nsched, float ox, float oy, float oz, float dx,
@@ -451,16 +467,7 @@ __device__ __forceinline__ float4 cone_march_fixed(const TraceParams& P, const S
     const float uz = fmaf(udz, e.t, uoz);
     if (!inside_grid(ux, uy, uz, nf)) break;
     float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
-    uint32_t abits = 0;
-    if (e.code & kSchedTop) {
-      gather_uniform<PREC, true>(P, e.code & ~kSchedTop, ux, uy, uz, 1.0f, kHalfOne, s, abits);
-      count += 1;
-    } else {
-      gather_uniform<PREC, true>(P, e.code + 1, ux, uy, uz, e.fr, e.hfr, s, abits);
-      if (abits || !skip_fine_ok<PREC>(e.code))
-        gather_uniform<PREC, false>(P, e.code, ux, uy, uz, e.gr, e.hgr, s, abits);
-      count += 2;
-    }
+    fixed_sample<PREC>(P, e, ux, uy, uz, s, count);
     composite(s, cr, cg, cb, a);
     if (a >= cutoff) break;
   }
@@ -529,6 +536,66 @@ __device__ __forceinline__ float4 cone_march_lane(const TraceParams& P, float ox
   return make_float4(cr, cg, cb, a);
 }
 
+// One cone of a block marched by all wavefronts of its workgroup together: in each round
+// wavefront w gathers sample w of the next blockDim.x / 64, the samples meet in LDS, and
+// every wavefront composites them in order, so each holds the march's whole state and the
+// result is that of one wavefront marching alone, bit for bit. A sample's position does not
+// depend on the ones before it; samples past the end of a lane's march go unused. buf: two
+// sets of a sample per wavefront and lane (a round is gathered while the last is read);
+// valid: the lanes whose sample lies on the march (within its distance and the grid).
+template <int PREC, bool BUF>
+__device__ __forceinline__ float4 cone_march_shared(const TraceParams& P, bool fixed, float ox, float oy, float oz,
+                                                    float dx, float dy, float dz, float tan_half, bool alive,
+                                                    float4* buf, uint64_t* valid, uint32_t& count) {
+  const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t nw = blockDim.x >> 6;
+  float cr = 0.f, cg = 0.f, cb = 0.f, a = 0.f;
+  float t = P.start_off * P.h;
+  const float nf = (float)P.n;
+  const float top = (float)(P.levels - 1);
+  const float uox = cone_origin(ox, P.origin[0], P.inv_h), udx = dx * P.inv_h;
+  const float uoy = cone_origin(oy, P.origin[1], P.inv_h), udy = dy * P.inv_h;
+  const float uoz = cone_origin(oz, P.origin[2], P.inv_h), udz = dz * P.inv_h;
+  const float h = P.h, inv_h = P.inv_h, step = P.step, cutoff = P.cutoff, max_dist = P.max_dist;
+  const uint32_t n = fixed ? __builtin_amdgcn_readfirstlane(P.sched_len[1]) : (uint32_t)VGI_MAX_MARCH_STEPS;
+  for (uint32_t it = 0, half = 0;; it += nw, half ^= nw) {
+    bool in = alive && it + wave < n;
+    uint32_t taken = 0;
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (fixed) {
+      const uint32_t i = it + wave;
+      const SchedEntry e = sld_rec(P.sched[1] + (i < n ? i : 0u));
+      const float ux = fmaf(udx, e.t, uox), uy = fmaf(udy, e.t, uoy), uz = fmaf(udz, e.t, uoz);
+      in = in && inside_grid(ux, uy, uz, nf);
+      if (in) fixed_sample<PREC>(P, e, ux, uy, uz, s, taken);
+    } else {
+      float mine = t;
+      for (uint32_t j = 0; j < nw; j++) {
+        if (j == wave) mine = t;
+        t = fmaf(step, fmaxf(h, 2.0f * t * tan_half), t);
+      }
+      const float ux = fmaf(udx, mine, uox), uy = fmaf(udy, mine, uoy), uz = fmaf(udz, mine, uoz);
+      in = in && mine <= max_dist && inside_grid(ux, uy, uz, nf);
+      const float lvl = fmaxf(0.0f, __log2f(fmaxf(h, 2.0f * mine * tan_half) * inv_h));
+      if (in) lane_sample<PREC, BUF>(P, ux, uy, uz, lvl, top, s, taken);
+    }
+    buf[64u * (half + wave) + lane] = s;
+    const uint64_t m = __ballot(in);
+    if (lane == 0) valid[half + wave] = m;
+    __syncthreads();
+    for (uint32_t j = 0; j < nw; j++) {
+      alive = alive && ((valid[half + j] >> lane) & 1u);
+      if (alive) {
+        composite(buf[64u * (half + j) + lane], cr, cg, cb, a);
+        if (j == wave) count += taken;
+        alive = !(a >= cutoff);
+      }
+    }
+    if (__ballot(alive) == 0ull) break;  // the same in every wavefront
+  }
+  return make_float4(cr, cg, cb, a);
+}
+
 // Work item of workgroup b in the XCD-aware order: block b runs on XCD b % 8. The batch's
 // work list (tiles of one scene are consecutive, row-major; sorted runs are consecutive in
 // Morton order) is dealt to the XCDs in bands of Bt.band consecutive items, XCD x taking
@@ -592,8 +659,11 @@ __device__ __forceinline__ float4 march_diffuse(const TraceParams& P, const floa
              : cone_march_lane<PREC, BUF>(P, ox, oy, oz, dx, dy, dz, P.tan_d, count);
 }
 
-template <int PREC, bool BUF>
-__device__ __forceinline__ float4 march_specular(const TraceParams& P, const float* f, size_t p, uint32_t& count) {
+// The specular cone's direction and, with a roughness buffer, its half-angle tangent.
+struct Specular {
+  float x, y, z, tan_half;
+};
+__device__ __forceinline__ Specular specular_cone(const TraceParams& P, const float* f, size_t p) {
 #pragma clang fp contract(off)
   const float px = gld(P.pos + p * 3), py = gld(P.pos + p * 3 + 1), pz = gld(P.pos + p * 3 + 2);
   const float nx = f[64 * kNx], ny = f[64 * kNy], nz = f[64 * kNz];
@@ -602,14 +672,18 @@ __device__ __forceinline__ float4 march_specular(const TraceParams& P, const flo
   const float vi = vl2 > 0.f ? 1.0f / __builtin_sqrtf(vl2) : 0.f;
   const float ix = -vx * vi, iy = -vy * vi, iz = -vz * vi;
   const float dn2 = 2.0f * fmaf(nz, iz, fmaf(nx, ix, ny * iy));
-  const float rx = fmaf(-dn2, nx, ix), ry = fmaf(-dn2, ny, iy), rz = fmaf(-dn2, nz, iz);
+  Specular s;
+  s.x = fmaf(-dn2, nx, ix), s.y = fmaf(-dn2, ny, iy), s.z = fmaf(-dn2, nz, iz);
+  s.tan_half = P.rough ? fminf(fmaxf(gld(P.rough + p), 0.0087f), 1.0f) : P.tan_s;
+  return s;
+}
+
+template <int PREC, bool BUF>
+__device__ __forceinline__ float4 march_specular(const TraceParams& P, const float* f, size_t p, uint32_t& count) {
+  const Specular s = specular_cone(P, f, p);
   const float ox = f[64 * kOx], oy = f[64 * kOy], oz = f[64 * kOz];
-  if (P.rough) {
-    const float th = fminf(fmaxf(gld(P.rough + p), 0.0087f), 1.0f);
-    return cone_march_lane<PREC, BUF>(P, ox, oy, oz, rx, ry, rz, th, count);
-  }
-  return BUF ? cone_march_fixed<PREC>(P, P.sched[1], P.sched_len[1], ox, oy, oz, rx, ry, rz, count)
-             : cone_march_lane<PREC, BUF>(P, ox, oy, oz, rx, ry, rz, P.tan_s, count);
+  if (BUF && !P.rough) return cone_march_fixed<PREC>(P, P.sched[1], P.sched_len[1], ox, oy, oz, s.x, s.y, s.z, count);
+  return cone_march_lane<PREC, BUF>(P, ox, oy, oz, s.x, s.y, s.z, s.tan_half, count);
 }
 
 __device__ __forceinline__ void store_out(float4* out, float4 v) {
@@ -620,7 +694,7 @@ __device__ __forceinline__ void store_out(float4* out, float4 v) {
 // Adds the workgroup's gathers to the counter: one global atomic per workgroup (all add to
 // one address).
 __device__ __forceinline__ void add_count(unsigned long long* counter, uint32_t count) {
-  __shared__ unsigned long long s_count[kMaxTraceWaves];
+  __shared__ unsigned long long s_count[kMaxSharedWaves];
   unsigned long long c = count;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
@@ -649,8 +723,12 @@ constexpr int trace_waves(int prec, bool full) { return prec == VGI_PREC_FP32 &&
 // launch (96 x 54 pixels, 9 + 1 cones: 104 us, 47 with three wavefronts), and of a large
 // launch keeps twice the blocks resident per CU, whose footprints share its L1 (1280 x 720:
 // FP32 439 -> 388 us, FP16 436 -> 410, BF16 470 -> 427, FP16 x-pair 364 -> 341).
-template <int PREC, bool BUF, bool SORTED, bool FULL>
-__global__ __launch_bounds__(64 * kMaxTraceWaves) __attribute__((amdgpu_waves_per_eu(trace_waves(PREC, FULL))))
+// SHARED (a launch of few blocks): all wavefronts, up to sixteen, first march the specular
+// cone together (cone_march_shared), whose chain of samples sets the length of such a
+// launch, then take the diffuse cones as above.
+template <int PREC, bool BUF, bool SORTED, bool FULL, bool SHARED>
+__global__ __launch_bounds__(64 * (SHARED ? kMaxSharedWaves : kMaxTraceWaves))
+__attribute__((amdgpu_waves_per_eu(SHARED ? 4 : trace_waves(PREC, FULL))))
 void k_trace(TraceBatch Bt, const TraceParams* __restrict__ scenes, const uint2* __restrict__ blocks,
              const unsigned long long* __restrict__ skeys, const uint32_t* __restrict__ spix) {
   extern __shared__ float4 s_cone[];  // diffuse cone c of lane l at 64 c + l
@@ -691,13 +769,25 @@ void k_trace(TraceBatch Bt, const TraceParams* __restrict__ scenes, const uint2*
     if (lane == 0) s_cones = m;
   }
   const bool spec = P.out_s && P.specular;
-  const uint32_t ntask = P.num_diffuse + (spec ? 1u : 0u);
   __syncthreads();
   const bool cones = (s_cones >> lane) & 1u;
+  if constexpr (SHARED) {
+    if (spec) {
+      __shared__ uint64_t s_valid[2 * kMaxSharedWaves];
+      Specular c{0.f, 0.f, 0.f, 0.f};
+      if (cones) c = specular_cone(P, frame, p);
+      const float4 r = cone_march_shared<PREC, BUF>(P, BUF && !P.rough, frame[64 * kOx], frame[64 * kOy], frame[64 * kOz],
+                                                    c.x, c.y, c.z, c.tan_half, cones, s_cone + 64u * Bt.max_diffuse,
+                                                    s_valid, count);
+      if (wave == 0 && cones) store_out(P.out_s + p, r);
+    }
+  }
+  const bool spec_task = spec && !SHARED;
+  const uint32_t ntask = P.num_diffuse + (spec_task ? 1u : 0u);
   for (uint32_t k = wave; k < ntask;) {
-    const uint32_t c = spec ? k - 1u : k;  // diffuse cone, or all ones for the specular cone
+    const uint32_t c = spec_task ? k - 1u : k;  // diffuse cone, or all ones for the specular cone
     if (cones) {
-      if (c == ~0u) store_out(P.out_s + p, march_specular<PREC, BUF>(P, frame, p, count));
+      if (!SHARED && c == ~0u) store_out(P.out_s + p, march_specular<PREC, BUF>(P, frame, p, count));
       else s_cone[64u * c + lane] = march_diffuse<PREC, BUF>(P, frame, c, count);
     }
     uint32_t next = 0;
@@ -728,12 +818,13 @@ void k_trace(TraceBatch Bt, const TraceParams* __restrict__ scenes, const uint2*
 template <int PREC, bool SORTED>
 static void launch_trace_prec(const TraceBatch& B, bool buffer_path, hipStream_t s) {
   const dim3 grid(B.nblocks), block(64u * B.waves);
-  const uint32_t lds = B.max_diffuse * 64u * (uint32_t)sizeof(float4);
-#define VGI_LAUNCH(BUF, FULL) \
-  hipLaunchKernelGGL((k_trace<PREC, BUF, SORTED, FULL>), grid, block, lds, s, B, B.scenes, B.blocks, B.skeys, B.spix)
-  if (!buffer_path) VGI_LAUNCH(false, false);
-  else if (PREC == VGI_PREC_FP32 && B.full) VGI_LAUNCH(true, PREC == VGI_PREC_FP32);  // (other forms: one variant)
-  else VGI_LAUNCH(true, false);
+  const uint32_t lds = (B.max_diffuse + (B.shared ? 2u * B.waves : 0u)) * 64u * (uint32_t)sizeof(float4);
+#define VGI_LAUNCH(BUF, FULL, SHARED) \
+  hipLaunchKernelGGL((k_trace<PREC, BUF, SORTED, FULL, SHARED>), grid, block, lds, s, B, B.scenes, B.blocks, B.skeys, B.spix)
+  if (!buffer_path) VGI_LAUNCH(false, false, false);
+  else if (B.shared) VGI_LAUNCH(true, false, true);
+  else if (PREC == VGI_PREC_FP32 && B.full) VGI_LAUNCH(true, PREC == VGI_PREC_FP32, false);  // (other forms: one variant)
+  else VGI_LAUNCH(true, false, false);
 #undef VGI_LAUNCH
 }
 

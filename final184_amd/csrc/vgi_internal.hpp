@@ -306,12 +306,14 @@ struct TraceBatch {
   uint32_t sub_shift;    // log2 of the 8x8 blocks in a screen tile
   uint32_t waves;        // wavefronts that share a 64-pixel block's cones
   uint32_t full;         // the launch has wavefronts to fill every SIMD (trace_waves)
+  uint32_t shared;       // few blocks: the wavefronts march the specular cone together
   uint32_t max_diffuse;  // most diffuse cones of the launch's items (the LDS it takes)
 };
 
 constexpr uint32_t kNoPixel = 0xFFFFFFFFu;
 constexpr uint32_t kSortBlock = 256;  // a scene's sorted entries are padded to a multiple of this
-constexpr uint32_t kMaxTraceWaves = 4;
+constexpr uint32_t kMaxTraceWaves = 4;    // wavefronts a block's cones are dealt to
+constexpr uint32_t kMaxSharedWaves = 16;  // ... that march its specular cone together
 
 // Texel bytes per precision.
 inline uint32_t texel_bytes(uint32_t prec) { return (prec == VGI_PREC_FP32 || prec == VGI_PREC_FP16X2) ? 16u : 8u; }

@@ -507,13 +507,15 @@ def test_shadowed_and_plain_scenes_in_one_batch(ctx, soup):
         b.release()
 
 
-@pytest.mark.parametrize("prec", ["fp32", "fp16x2"])
-def test_trace_is_independent_of_launch_size(ctx, soup, prec):
+@pytest.mark.parametrize("rough", [False, True])
+@pytest.mark.parametrize("prec", ["fp32", "fp16", "bf16", "fp16x2"])
+def test_trace_is_independent_of_launch_size(ctx, soup, prec, rough):
     """Launches of few, many and very many 8x8 blocks share a block's cones among other
-    numbers of wavefronts (and FP32 has a register variant for each side): the first rows of
-    a large G-buffer, traced by themselves, give the same bits. 728 x 728 pixels (8281
-    blocks) are past the line where FP32 changes its variant, 888 x 888 (12321) past the one
-    where two wavefronts share a block."""
+    numbers of wavefronts, the smallest march the specular cone together, and FP32 has a
+    register variant for each side: the first rows of a large G-buffer, traced by themselves,
+    give the same bits. 200 x 200 pixels (625 blocks) are past the line for the specular
+    cone, 728 x 728 (8281) past the one where FP32 changes its variant, 888 x 888 (12321)
+    past the one where two wavefronts share a block."""
     vgi = _vgi()
     w = soup["w"]
     f = Frame(ctx, w, prec)
@@ -521,17 +523,18 @@ def test_trace_is_independent_of_launch_size(ctx, soup, prec):
     pick = rng.integers(0, w.num_pixels, 888 * 888)
     pos, nrm = w.gb_pos[pick].copy(), w.gb_nrm[pick].copy()
     nrm[rng.random(len(pick)) < 0.02] = 0.0  # pixels without a surface
+    tan = rng.uniform(0.0, 1.2, len(pick)).astype(np.float32) if rough else None
 
     def trace(n, width, height):
-        gb = vgi.GBufferData(ctx, pos[:n], nrm[:n], width, height)
+        gb = vgi.GBufferData(ctx, pos[:n], nrm[:n], width, height, tan[:n] if rough else None)
         od = vgi.DeviceArray.empty(ctx, (n, 4), np.float32)
         osp = vgi.DeviceArray.empty(ctx, (n, 4), np.float32)
         f.scene.trace(gb, vgi.make_cones(**w.cones), od, osp)
         return od.numpy(), osp.numpy()
 
     d0, s0 = trace(72 * 9, 72, 9)
-    for side in (728, 888):
-        print(f"case trace {prec} {side}x{side}", flush=True)
+    for side in (200, 728, 888):
+        print(f"case trace {prec} rough={rough} {side}x{side}", flush=True)
         d, s = trace(side * side, side, side)
         assert np.array_equal(d[:len(d0)], d0) and np.array_equal(s[:len(s0)], s0)
     f.release()
