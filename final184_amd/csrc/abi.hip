@@ -166,7 +166,7 @@ struct vgi_workspace {
   size_t pairs_bytes = 0;
   void* scan_tmp = nullptr;
   size_t scan_tmp_bytes = 0;
-  void* sort_keys = nullptr;  // Morton order: keys in | keys out (u64)
+  void* sort_keys = nullptr;  // Morton order: keys in | keys out (u32)
   size_t sort_keys_bytes = 0;
   void* sort_pix = nullptr;   // pixel indices in | out (u32)
   size_t sort_pix_bytes = 0;
@@ -1235,9 +1235,9 @@ int trace_batch(vgi_context* ctx, const vgi_trace_item* items, uint32_t count, v
   std::lock_guard<std::mutex> wl(w->mu);
   if (morton) {  // sort buffers for the largest launch (grown; queued work drained first)
     size_t tmp_need = 0;
-    HIP_TRY(sort_pixels(nullptr, &tmp_need, nullptr, nullptr, nullptr, nullptr, (uint32_t)max_entries, 64, st));
-    if (w->sort_keys_bytes < max_entries * 16 || w->sort_tmp_bytes < tmp_need) HIP_TRY(hipStreamSynchronize(st));
-    TRY(grow_bytes(&w->sort_keys, &w->sort_keys_bytes, max_entries * 16, "sort keys"));
+    HIP_TRY(sort_pixels(nullptr, &tmp_need, nullptr, nullptr, nullptr, nullptr, (uint32_t)max_entries, 32, st));
+    if (w->sort_keys_bytes < max_entries * 8 || w->sort_tmp_bytes < tmp_need) HIP_TRY(hipStreamSynchronize(st));
+    TRY(grow_bytes(&w->sort_keys, &w->sort_keys_bytes, max_entries * 8, "sort keys"));
     TRY(grow_bytes(&w->sort_pix, &w->sort_pix_bytes, max_entries * 8, "sort pixels"));
     TRY(grow_bytes(&w->sort_tmp, &w->sort_tmp_bytes, std::max<size_t>(tmp_need, 1), "sort scratch"));
   }
@@ -1296,13 +1296,14 @@ int trace_batch(vgi_context* ctx, const vgi_trace_item* items, uint32_t count, v
       B.max_diffuse = L.max_diffuse;
       B.shared = L.shared ? 1u : 0u;
       if (morton && L.entries > 0) {
-        unsigned long long* keys = (unsigned long long*)w->sort_keys;
+        uint32_t* keys = (uint32_t*)w->sort_keys;
         uint32_t* pix = (uint32_t*)w->sort_pix;
         B.seg = (const uint32_t*)(sl.d + L.o_seg);
+        const uint32_t scene_bits = L.nscenes > 1 ? ilog2(L.nscenes - 1) + 1 : 0;
+        B.code_bits = std::min(kMortonBits, 32 - scene_bits);
         HIP_TRY(launch_morton_keys(B, keys, pix, (uint32_t)L.entries, st));
-        const int end_bit = 32 + (int)ilog2(std::max<uint32_t>(L.nscenes - 1, 1)) + 1;
         HIP_TRY(sort_pixels(w->sort_tmp, &w->sort_tmp_bytes, keys, keys + max_entries, pix, pix + max_entries,
-                            (uint32_t)L.entries, std::min(end_bit, 64), st));
+                            (uint32_t)L.entries, (int)(scene_bits + B.code_bits), st));
         B.skeys = keys + max_entries;
         B.spix = pix + max_entries;
       }

@@ -288,16 +288,19 @@ struct TraceParams {
   float4* out_s;
 };
 
+constexpr uint32_t kMortonBits = 30;  // of a position quantized to 1024^3
+
 struct TraceBatch {
   const TraceParams* scenes;
   const uint2* blocks;            // (scene, tile) per screen tile (screen-tile order, > 1 scene)
   unsigned long long* counter;    // trilinear gathers (may be null)
   // Morton order (null in screen-tile order): the batch's pixels sorted by
-  // (scene << 32 | Morton code of the position); scene s owns entries [seg[s], seg[s+1]),
-  // a multiple of 256, padded with pixel index kNoPixel after its sorted pixels.
-  const unsigned long long* skeys;
+  // (scene << code_bits | Morton code of the position); scene s owns entries [seg[s],
+  // seg[s+1]), a multiple of 256, padded with pixel index kNoPixel after its sorted pixels.
+  const uint32_t* skeys;
   const uint32_t* spix;
   const uint32_t* seg;
+  uint32_t code_bits;  // the scenes leave of the key's 32, at most kMortonBits
   uint32_t nblocks;
   uint32_t tile_w, tile_h;
   uint32_t prec;
@@ -451,11 +454,9 @@ hipError_t launch_mips(const MipBatch& B, uint32_t prec, bool from_acc, uint32_t
 hipError_t launch_tiles(const TileArgs& t, const StageArgs& a, uint32_t ntiles, hipStream_t s);
 hipError_t launch_trace(const TraceBatch& B, bool buffer_path, hipStream_t s);
 // Morton keys of every pixel of a batch (entries seg[0]..seg[nscenes], padding included).
-hipError_t launch_morton_keys(const TraceBatch& B, unsigned long long* keys, uint32_t* pix, uint32_t entries,
-                              hipStream_t s);
-hipError_t sort_pixels(void* tmp, size_t* tmp_bytes, const unsigned long long* keys_in,
-                       unsigned long long* keys_out, const uint32_t* pix_in, uint32_t* pix_out, uint32_t n,
-                       int end_bit, hipStream_t s);
+hipError_t launch_morton_keys(const TraceBatch& B, uint32_t* keys, uint32_t* pix, uint32_t entries, hipStream_t s);
+hipError_t sort_pixels(void* tmp, size_t* tmp_bytes, const uint32_t* keys_in, uint32_t* keys_out,
+                       const uint32_t* pix_in, uint32_t* pix_out, uint32_t n, int end_bit, hipStream_t s);
 
 // ---- screen-space passes (screen.hip); arguments validated by the caller ----
 hipError_t launch_gbuffer_decode(const vgi_gbuffer_ref& in, float* pos, float* nrm, float* view_depth,

@@ -109,6 +109,44 @@ def test_batch_equals_alone(ctx, bin_size, tile, order):
         ctx.set_tuning()
 
 
+@pytest.mark.parametrize("frames", [1, 2, 4, 5, 17])
+def test_morton_key_bits(ctx, frames):
+    """The sort key holds a frame's number and, in the bits that leaves of 32 (30 at most),
+    its pixels' Morton codes: one, two and four frames leave 30, five 29, seventeen 27.
+    Pixels in the grid's last cell share the padding's code; others lie outside the grid."""
+    vgi = _vgi()
+    print(f"case morton_key_bits frames={frames}", flush=True)
+    w = sg.batch_scenes(count=1, median=3000.0, tri_range=(2000, 4000), grids=(32,), sides=(64,))[0]
+    job = Job(ctx, w)
+    _run_alone(ctx, [job], [vgi.PREC_FP16])
+    rng = np.random.default_rng(frames)
+    sides = [(64, 64), (16, 16), (17, 15), (1, 1), (33, 40)]
+    size = np.float32(w.grid["extent"])
+    corner = np.asarray(w.grid["origin"], np.float32) + size
+    gbs, outs = [], []
+    for i in range(frames):
+        width, height = sides[i % len(sides)]
+        pick = rng.integers(0, w.num_pixels, width * height)
+        pos, nrm = w.gb_pos.reshape(-1, 3)[pick].copy(), w.gb_nrm.reshape(-1, 3)[pick]
+        pos[rng.random(len(pick)) < 0.2] = corner * np.float32(1 - 1e-6)
+        pos[rng.random(len(pick)) < 0.1] += 2 * size
+        gbs.append(vgi.GBufferData(ctx, pos, nrm, width, height))
+
+    def run():
+        out = [[vgi.DeviceArray.empty(ctx, (g.num_pixels, 4), np.float32) for _ in range(2)] for g in gbs]
+        ctx.trace_batch([(job.scene, g, job.cones, d, s) for g, (d, s) in zip(gbs, out)])
+        ctx.sync()
+        return [[x.numpy() for x in o] for o in out]
+
+    try:
+        tiles = run()
+        ctx.set_tuning(pixel_order=vgi.ORDER_MORTON)
+        for a, b in zip(tiles, run()):
+            assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+    finally:
+        ctx.set_tuning()
+
+
 def test_batch_two_streams(ctx):
     """Two batches on two streams at once give the same results as one after the other."""
     vgi = _vgi()
