@@ -13,8 +13,10 @@
 // Arithmetic is FP32 in the order the definitions write it, with fused multiply-adds
 // only where written (the blur's weighted sums and its depth term), IEEE division and
 // square root, and a polynomial exp2, so the results are reproducible bit for bit on
-// any IEEE machine. The blur is VALU-bound (about 300 operations per pixel, mostly the
-// 12 exp2 evaluations), the other two passes HBM-bound.
+// any IEEE machine. The blur is VALU-bound (about 320 instructions per pixel, mostly the
+// 12 exp2 evaluations), the other two passes HBM-bound. (Tried for the blur: a thread taking
+// 2, 4 or 8 pixels of one parity along the axis, which share texels and weights: no faster
+// at 1080p and at 4K, for want of wavefronts.)
 #include "vgi_internal.hpp"
 
 #pragma clang fp contract(off)
@@ -26,16 +28,24 @@ namespace {
 constexpr uint32_t kRowBlockX = 64;  // decode / temporal block: 64 x 4 pixels
 constexpr uint32_t kRowBlockY = 4;
 
+// A texel as it lies in memory, and decoded.
+template <bool HALF> struct Raw { typedef uint4 type; };
+template <> struct Raw<true> { typedef uint2 type; };
+template <bool HALF>
+__device__ __forceinline__ typename Raw<HALF>::type load_raw(const void* img, size_t i) {
+  if constexpr (HALF) return gld2(static_cast<const uint16_t*>(img) + 4 * i);
+  else return gld4(static_cast<const float*>(img) + 4 * i);
+}
+__device__ __forceinline__ float4 decode_raw(uint2 u) {
+  return make_float4(f16_bits_to_f32((uint16_t)(u.x & 0xFFFFu)), f16_bits_to_f32((uint16_t)(u.x >> 16)),
+                     f16_bits_to_f32((uint16_t)(u.y & 0xFFFFu)), f16_bits_to_f32((uint16_t)(u.y >> 16)));
+}
+__device__ __forceinline__ float4 decode_raw(uint4 u) {
+  return make_float4(__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w));
+}
 template <bool HALF>
 __device__ __forceinline__ float4 load_texel(const void* img, size_t i) {
-  if constexpr (HALF) {
-    const uint2 u = gld2(static_cast<const uint16_t*>(img) + 4 * i);
-    return make_float4(f16_bits_to_f32((uint16_t)(u.x & 0xFFFFu)), f16_bits_to_f32((uint16_t)(u.x >> 16)),
-                       f16_bits_to_f32((uint16_t)(u.y & 0xFFFFu)), f16_bits_to_f32((uint16_t)(u.y >> 16)));
-  } else {
-    const uint4 u = gld4(static_cast<const float*>(img) + 4 * i);
-    return make_float4(__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w));
-  }
+  return decode_raw(load_raw<HALF>(img, i));
 }
 
 template <bool HALF>
@@ -174,11 +184,12 @@ __global__ __launch_bounds__(256) void k_temporal(vgi_temporal_params p) {
 // truncation error is below 6e-9 relative) evaluated by Horner's rule with FMAs;
 // 0 for x <= -125 and NaN, so every non-zero result is a normal number.
 __device__ __forceinline__ float exp2_poly(float x) {
-  // Branch-free: the polynomial runs on max(x, -126) (NaN -> -126) and a select returns
-  // 0 below -125, so the taps of a pixel keep their loads in flight together.
-  const float xc = fmaxf(x, -126.0f);
-  const float k = rintf(xc);
-  const float f = xc - k;
+  // rint(x) is the low bits of x + 1.5 * 2^23, and adding them to q's exponent is the
+  // multiplication by 2^k (q in [0.7, 1.42], so the result is normal for x > -125; below,
+  // where the sum may not even hold k, the select drops it). Branch-free, so the taps of a
+  // pixel keep their loads in flight together.
+  const float t = x + 12582912.0f;
+  const float f = x - (t - 12582912.0f);
   float q = 1.525273365e-05f;
   q = __builtin_fmaf(q, f, 1.540352969e-04f);
   q = __builtin_fmaf(q, f, 1.333355787e-03f);
@@ -187,7 +198,7 @@ __device__ __forceinline__ float exp2_poly(float x) {
   q = __builtin_fmaf(q, f, 2.402265072e-01f);
   q = __builtin_fmaf(q, f, 6.931471825e-01f);
   q = __builtin_fmaf(q, f, 1.0f);
-  const float r = ldexpf(q, (int)k);
+  const float r = __uint_as_float(__float_as_uint(q) + (__float_as_uint(t) << 23));
   return x > -125.0f ? r : 0.0f;
 }
 
@@ -235,13 +246,29 @@ __global__ __launch_bounds__(256) void k_blur(vgi_blur_params p, uint32_t ntx, u
   const int x0 = (int)tx * T::TX - (AXIS == 0 ? kBlurReach : 0);
   const int y0 = (int)ty * T::TY - (AXIS == 1 ? kBlurReach : 0);
 
-  for (int e = threadIdx.x; e < T::LX * T::LY; e += 256) {
+  // All of a thread's loads are issued before the first is waited for: one round trip to
+  // memory a workgroup instead of eight along y, three along x (with the
+  // exp2 above, all four screen passes: 1080p FP16 71.9 -> 68.1 us, 4K 265 -> 247, 643 x 361
+  // FP32 22.4 -> 20.4).
+  constexpr int kStage = (T::LX * T::LY + 255) / 256;
+  typename Raw<IN_HALF>::type raw[kStage];
+  float depth[kStage];
+#pragma unroll
+  for (int k = 0; k < kStage; k++) {
+    const int e = min((int)threadIdx.x + 256 * k, T::LX * T::LY - 1);
     const int lx = e % T::LX, ly = e / T::LX;
     const int gx = min(max(x0 + lx, 0), W - 1), gy = min(max(y0 + ly, 0), H - 1);  // clamp to edge
     const size_t gi = (size_t)gy * (size_t)W + (size_t)gx;
-    float4 c = load_texel<IN_HALF>(p.color, gi);
-    c.w = gld(p.depth + gi);
-    s_tex[e] = c;
+    raw[k] = load_raw<IN_HALF>(p.color, gi);
+    depth[k] = gld(p.depth + gi);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int k = 0; k < kStage; k++) {
+    const int e = (int)threadIdx.x + 256 * k;
+    float4 c = decode_raw(raw[k]);
+    c.w = depth[k];
+    if (e < T::LX * T::LY) s_tex[e] = c;
   }
   __syncthreads();
 

@@ -151,6 +151,31 @@ def test_blur_matches_oracle(ctx, W, H, axis, in_fmt, out_fmt):
     _same(d_out.numpy(), ref)
 
 
+@pytest.mark.parametrize("axis", [0, 1])
+def test_blur_depth_extremes(ctx, axis):
+    """Weights where exp2's argument crosses -125 (0 below it), and far below, infinite and
+    not a number: depth steps of 0.0205 to 0.0225 around sqrt(125 - r^2/32) / 512, of 1e3, 1e30
+    and 3e38, infinities and NaN."""
+    print(f"case blur extremes axis={axis}", flush=True)
+    vgi = _vgi()
+    rng = np.random.default_rng(axis)
+    W, H = 288, 64
+    dep = (0.0205 + 0.002 * rng.random(W * H)).astype(np.float32)
+    dep[rng.random(W * H) < 0.5] = 0.0
+    for share, v in ((0.04, 1e3), (0.03, 1e30), (0.03, 3e38), (0.03, np.inf), (0.03, -np.inf), (0.03, np.nan)):
+        dep[rng.random(W * H) < share] = v
+    col = rng.uniform(0.0, 4.0, (W * H, 4)).astype(np.float32)
+    d_col, d_dep = _image(ctx, col, F32), vgi.DeviceArray.from_numpy(ctx, dep)
+    d_out = _empty_image(ctx, W * H, F32)
+    ctx.bilateral_blur(d_col, d_dep, d_out, W, H, axis, F32, F32)
+    ctx.sync()
+    with np.errstate(all="ignore"):
+        ref = orc.bilateral_blur(col, dep, W, H, axis)
+    out = d_out.numpy()
+    assert np.array_equal(np.isnan(out), np.isnan(ref))
+    _same(np.nan_to_num(out, nan=0.0, posinf=np.inf, neginf=-np.inf), np.nan_to_num(ref, nan=0.0, posinf=np.inf, neginf=-np.inf))
+
+
 def test_blur_full_frame_both_axes(ctx):
     """1920x1080, the reference's order: blurX.frag (along y) then blurY.frag (along x)."""
     print("case blur 1920x1080 chain", flush=True)
