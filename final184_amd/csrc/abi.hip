@@ -66,6 +66,13 @@ int fail(int code, const char* fmt, ...) {
   } while (0)
 
 bool is_pow2(uint32_t v) { return v && !(v & (v - 1)); }
+// A scene's mip tile state (vgi_scene::live): ten words per 16^3 tile, 64 of counts, and a bit
+// per bin of 8^3 voxels.
+uint64_t tile_state_bytes(uint64_t n) {
+  const uint64_t tpa = n / std::min<uint64_t>(n, 16), nb = n / 8;
+  return (tpa * tpa * tpa * 10 + 64 + (nb * nb * nb + 31) / 32) * sizeof(uint32_t);
+}
+
 uint32_t ilog2(uint32_t v) {
   uint32_t r = 0;
   while ((1u << (r + 1)) <= v) r++;
@@ -172,6 +179,8 @@ struct vgi_workspace {
   size_t sort_pix_bytes = 0;
   void* sort_tmp = nullptr;
   size_t sort_tmp_bytes = 0;
+  void* vis = nullptr;        // mip builds with shadow-casting lights: vis bytes (MipScene)
+  size_t vis_bytes = 0;
   // pinned: the last call's batch pairs, work units, large triangles and split bins, then
   // its call number, which the settle step stores once the four totals are complete
   unsigned long long* hist = nullptr;
@@ -182,7 +191,7 @@ struct vgi_workspace {
   size_t device_bytes() const {
     size_t b = tris_bytes + tritex_bytes + tri_slot_bytes + big_list_bytes + zeroed_bytes + zero_list_bytes +
                scan_bytes + work_bytes + pairs_bytes + scan_tmp_bytes + sort_keys_bytes + sort_pix_bytes +
-               sort_tmp_bytes;
+               sort_tmp_bytes + vis_bytes;
     for (const Slot& s : slot) b += s.cap;
     return b;
   }
@@ -259,7 +268,8 @@ size_t scene_device_bytes(const vgi_scene* s) {
 
 void free_workspace(vgi_workspace* w) {
   void* dev[] = {w->tris,     w->tritex,   w->tri_slot, w->big_list, w->zeroed,    w->zero_list, w->scan_all,
-                 w->work_map, w->pairs,    w->scan_tmp, w->sort_keys, w->sort_pix, w->sort_tmp};
+                 w->work_map, w->pairs,    w->scan_tmp, w->sort_keys, w->sort_pix, w->sort_tmp,
+                 w->vis};
   for (void* p : dev)
     if (p) (void)hipFree(p);
   for (Slot& s : w->slot) {
@@ -813,9 +823,9 @@ int scene_levels(vgi_scene* s, uint32_t precision, hipStream_t st) {
     // The levels start all zero and a tile's texels (a level-0 x-row's) are stored only
     // while the tile (the row) or its previous build held occupied voxels, so every texel
     // of the levels stays exact: one word per tile, then eight row words per tile; then
-    // the injecting launch's tile list (a word per tile) and its two counts.
-    const size_t tpa = g.n / std::min<uint32_t>(g.n, 16u);
-    const size_t bytes = tpa * tpa * tpa * 10 * sizeof(uint32_t) + 256;
+    // the injecting launch's tile list (a word per tile) and its counts; then a bit per bin
+    // (of 8^3 voxels or more) for the visibility walks.
+    const size_t bytes = tile_state_bytes(g.n);
     hipError_t e = hipMalloc((void**)&s->live, bytes);
     if (e != hipSuccess) {
       (void)hipGetLastError();
@@ -895,13 +905,34 @@ int mips_batch(vgi_context* ctx, const vgi_mips_item* items, uint32_t count, uin
   size_t nblocks = 0;
   for (const auto& v : stages) nblocks += v.size();
   size_t total_lights = 0;
-  bool shadow = false;  // the injecting launch walks toward shadow-casting lights
-  for (uint32_t i = 0; i < count; i++)
+  // Builds with shadow-casting lights: where every scene has at most 32 and there is memory
+  // for an answer byte a voxel per eight of them, k_visibility walks before the injecting
+  // launch; otherwise (or when that memory is missing under stream capture) that launch walks
+  // by itself.
+  bool shadow = false, vis = true;
+  size_t vis_need = 0;
+  std::vector<size_t> vis_off(count);
+  for (uint32_t i = 0; i < count; i++) {
+    uint32_t ns = 0;
     if (items[i].lights) {
       total_lights += items[i].lights->count;
       for (uint32_t l = 0; l < items[i].lights->count; l++)
-        shadow = shadow || (items[i].lights->light[l].type & VGI_LIGHT_SHADOW) != 0;
+        ns += (items[i].lights->light[l].type & VGI_LIGHT_SHADOW) != 0;
     }
+    shadow = shadow || ns > 0;
+    vis = vis && ns <= kMaxVisLights;
+    const size_t n = items[i].scene->grid.n;
+    vis_off[i] = vis_need;
+    vis_need += align_up(n * n * n * ((ns + 7) / 8), 256) + (ns ? align_up(n * n * n / kVisVoxels * sizeof(uint32_t), 256) : 0);
+  }
+  vis = vis && shadow;
+  if (vis && w->vis_bytes < vis_need) {
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    HIP_TRY(hipStreamIsCapturing(st, &capturing));
+    vis = capturing == hipStreamCaptureStatusNone;
+    if (vis) HIP_TRY(hipStreamSynchronize(st));
+    vis = vis && grow_bytes(&w->vis, &w->vis_bytes, vis_need, "visibility") == VGI_OK;
+  }
   Carve cv;
   const size_t o_scenes = cv.take((size_t)count * sizeof(MipScene));
   const size_t o_blocks = cv.take(table ? nblocks * sizeof(MipBlock) : 0);
@@ -922,6 +953,8 @@ int mips_batch(vgi_context* ctx, const vgi_mips_item* items, uint32_t count, uin
     {
       const size_t tpa = g.n / std::min<uint32_t>(g.n, 16u);
       P.order = s->live + 9 * tpa * tpa * tpa;
+      P.vis_count = s->live + 10 * tpa * tpa * tpa + 32;
+      P.bin_bits = s->live + 10 * tpa * tpa * tpa + 64;
     }
     for (uint32_t k = 0; k < g.levels; k++) {
       P.level[k] = s->level[k];
@@ -936,8 +969,16 @@ int mips_batch(vgi_context* ctx, const vgi_mips_item* items, uint32_t count, uin
     const vgi_lights* L = items[i].lights;
     P.nlights = L ? L->count : 0;
     P.lights = (const LightDev*)(d + o_lights) + lbase;
-    for (uint32_t l = 0; l < P.nlights; l++) hl[lbase + l] = light_dev(L->light[l], P.origin, P.h);
+    uint32_t ns = 0;
+    for (uint32_t l = 0; l < P.nlights; l++) {
+      LightDev& D = hl[lbase + l] = light_dev(L->light[l], P.origin, P.h);
+      if (D.shadow) D.shadow = ++ns;
+    }
     lbase += P.nlights;
+    P.vis = vis && ns ? (uint8_t*)w->vis + vis_off[i] : nullptr;
+    P.vis_planes = P.vis ? (ns + 7) / 8 : 0;
+    const size_t n3 = (size_t)g.n * g.n * g.n;
+    P.vis_units = P.vis ? (uint32_t*)(P.vis + align_up(n3 * P.vis_planes, 256)) : nullptr;
   }
   MipBlock* hb = (MipBlock*)(h + o_blocks);
   size_t boff = 0;
@@ -947,6 +988,12 @@ int mips_batch(vgi_context* ctx, const vgi_mips_item* items, uint32_t count, uin
       boff += v.size();
     }
   };
+  uint32_t max_bins = 0, max_bricks = 0;
+  for (uint32_t i = 0; i < count; i++) {
+    const uint32_t nb = items[i].scene->nbins_axis, nbr = items[i].scene->grid.n / 8;
+    max_bins = std::max(max_bins, nb * nb * nb);
+    max_bricks = std::max(max_bricks, nbr * nbr * nbr);
+  }
   const bool prof = ctx->profiling != 0;
   auto launch = [&](const Slot& sl, const StageArgs& stage) -> int {
     if (prof) HIP_TRY(hipEventRecord(ctx->ev[5], st));
@@ -959,10 +1006,11 @@ int mips_batch(vgi_context* ctx, const vgi_mips_item* items, uint32_t count, uin
       B.src = stages[j][0].src;  // one scene: every block of the stage shares src and nout
       B.nout = stages[j][0].nout;
       B.shadow = shadow;
+      B.vis = vis;
       // (not for a one-level chain: its launch writes every texel of every tile and keeps no
-      // tile words, so every tile is visited; not with visibility walks, whose cost does not
-      // follow the pair count: the room's shadowed builds were 3-5% slower in list order)
-      const bool ordered = j == 0 && !table && stages[0][0].nout > 0 && !shadow;
+      // tile words, so every tile is visited; not with walks in the launch itself, whose cost
+      // does not follow the pair count: the room's were 3-5% slower in list order)
+      const bool ordered = j == 0 && !table && stages[0][0].nout > 0 && (!shadow || vis);
       if (ordered) {  // the injecting launch's tile list, dense tiles first; the descriptors with it
         vgi_scene* sc = items[0].scene;
         const vgi_grid& g = sc->grid;
@@ -973,11 +1021,13 @@ int mips_batch(vgi_context* ctx, const vgi_mips_item* items, uint32_t count, uin
         B.counts = counts + 2 * sc->tile_pair;
         B.clear_counts = counts + 2 * (sc->tile_pair ^ 1u);
         const TileArgs t{(const unsigned long long*)sc->bin_packed, sc->live, sc->live + 9 * ntl, B.counts, g.n,
-                         sc->bin_shift, sc->nbins_axis};
+                         sc->bin_shift, sc->nbins_axis, shadow ? sc->live + 10 * ntl + 64 : nullptr, sc->live + 10 * ntl + 32, 0};
         HIP_TRY(launch_tiles(t, stage, (uint32_t)ntl, st));
       } else if (j == 0) {
         HIP_TRY(launch_stage(stage, st));
+        if (shadow) HIP_TRY(launch_bin_bits(B.scenes, count, max_bins, st));
       }
+      if (j == 0 && vis) HIP_TRY(launch_visibility(B.scenes, count, max_bricks, st));
       HIP_TRY(launch_mips(B, precision, j == 0, (uint32_t)stages[j].size(), st));
       if (B.counts) {
         items[0].scene->tile_counts_zero = true;
@@ -1546,9 +1596,8 @@ uint64_t vgi_scene_bytes_estimate(const vgi_grid* g, uint32_t precision, uint64_
   (void)ntri;
   if (!g || !is_pow2(g->n) || g->n < 8 || g->levels == 0 || g->levels > VGI_MAX_LEVELS) return 0;
   const uint64_t n = g->n;
-  const uint64_t tpa = n / std::min<uint64_t>(n, 16);  // 16^3 tiles per axis (mip tile state)
   uint64_t b = n * n * n * kAccWords * 4 + (n / 8) * (n / 8) * (n / 8) * 64 + (n / 8) * (n / 8) * (n / 8) * 8 +
-               tpa * tpa * tpa * 10 * 4 + 256;
+               tile_state_bytes(n);
   for (uint32_t k = 0; k < g->levels; k++) {
     const uint64_t p = (n >> k) + 2;
     b += p * p * p * texel_bytes(precision);

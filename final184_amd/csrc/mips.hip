@@ -24,6 +24,7 @@
 // holds voxels or held them at the last build (one bit per row). A surface leaves most
 // tiles empty (70% at 256^3 for the room), so most level bytes are not rewritten each
 // build, and every texel still equals the full computation.
+#include <algorithm>
 #include <cmath>
 
 #include "vgi_internal.hpp"
@@ -189,21 +190,36 @@ __device__ __forceinline__ uint32_t group_occupancy(const MipScene& P, uint32_t 
 __device__ __forceinline__ int32_t sign_i32(int32_t v) { return (v > 0) - (v < 0); }
 __device__ __forceinline__ uint32_t abs_u32(int32_t v) { return v < 0 ? 0u - (uint32_t)v : (uint32_t)v; }
 
-// Visibility of shadow-casting light L from occupied voxel (x, y, z) whose summed normal
-// (unbiased integer sums) is (n0, n1, n2): a walk through the level-0 occupancy toward the
-// light in 16.16 fixed point. Start: the voxel centre moved one voxel along the dominant
-// axis of the normal sum (ties to the lowest axis). Each sample advances exactly one voxel
-// along the direction's dominant axis, so a walk leaves the grid within n + 1 samples; a
-// point light's walk also ends when it reaches the light's distance along that axis. The
-// voxel itself is passed over. Integer steps and IEEE single-precision subtraction,
-// division and rounding only, so every build of the walk takes the same decisions.
-__device__ bool light_visible(const MipScene& P, const LightDev& L, uint32_t x, uint32_t y, uint32_t z,
-                              int32_t n0, int32_t n1, int32_t n2) {
+// The move of a walk's start off its voxel: one voxel along the dominant axis of the summed
+// normal (unbiased integer sums; ties to the lowest axis).
+__device__ __forceinline__ void walk_offset(int32_t n0, int32_t n1, int32_t n2, int32_t& o0, int32_t& o1, int32_t& o2) {
   const uint32_t m0 = abs_u32(n0), m1 = abs_u32(n1), m2 = abs_u32(n2);
-  int32_t o0 = 0, o1 = 0, o2 = 0;
-  if (m0 >= m1 && m0 >= m2) o0 = sign_i32(n0);
-  else if (m1 >= m2) o1 = sign_i32(n1);
-  else o2 = sign_i32(n2);
+  const bool first = m0 >= m1 && m0 >= m2, second = !first && m1 >= m2;
+  o0 = first ? sign_i32(n0) : 0;
+  o1 = second ? sign_i32(n1) : 0;
+  o2 = !first && !second ? sign_i32(n2) : 0;
+}
+
+// 1 / |s|, rounded down, for the samples a brick holds; for 0 what makes it more than any other's.
+__device__ __forceinline__ float brick_samples(int32_t s) {
+  return s == 0 ? 0x1p-10f : __builtin_amdgcn_rcpf((float)abs(s)) * (1.0f - 0x1p-20f);
+}
+
+// Visibility of a shadow-casting light from occupied voxel (x, y, z): a walk through the
+// level-0 occupancy toward the light in 16.16 fixed point. Start: the voxel centre moved by
+// (o0, o1, o2) (walk_offset). Each sample advances exactly one voxel along the direction's
+// dominant axis, so a walk leaves the grid within n + 1 samples; a point light's walk also
+// ends when it reaches the light's distance along that axis. The voxel itself is passed
+// over. Integer steps and IEEE single-precision subtraction, division and rounding only, so
+// every build of the walk takes the same decisions. bins(w): word w of the scene's bin bits.
+//
+// Bound by VALU issue, at about 30 instructions for a brick passed whole and 100 for four
+// samples tested; one sample an iteration, its bin's entry and mask word loaded each time,
+// took about 45 a sample.
+constexpr int kWalkTests = 4;  // (2: the room's build 2-4% slower; 8: 256^3 and 512^3 5-7%)
+template <class Bins>
+__device__ __forceinline__ bool light_visible(const MipScene& P, const Bins& bins, const LightDev& L, uint32_t x,
+                                              uint32_t y, uint32_t z, int32_t o0, int32_t o1, int32_t o2) {
   const int32_t p0 = (int32_t)x + o0, p1 = (int32_t)y + o1, p2 = (int32_t)z + o2;
   int32_t s0, s1, s2;
   uint32_t steps = P.n + 2u;
@@ -225,29 +241,98 @@ __device__ bool light_visible(const MipScene& P, const LightDev& L, uint32_t x, 
     if (c < (float)steps) steps = (uint32_t)c;
   }
   int32_t q0 = p0 * 65536 + 32768, q1 = p1 * 65536 + 32768, q2 = p2 * 65536 + 32768;
-  const uint32_t bs = P.bin_shift, nb = P.nbins_axis, nbr = P.n >> 3;
-  // One sample per iteration: issuing the loads of 2, 4 or 8 samples together before
-  // testing the first measured no faster (0.27, 0.31, 0.43 ms against 0.27 ms for the
-  // room's four shadowed lights), the extra samples' work being wasted when a walk ends.
-  for (uint32_t m = 0; m < steps; m++) {
-    const int32_t c0 = q0 >> 16, c1 = q1 >> 16, c2 = q2 >> 16;  // floor
-    if ((uint32_t)c0 >= P.n || (uint32_t)c1 >= P.n || (uint32_t)c2 >= P.n) return true;
-    const uint32_t u0 = (uint32_t)c0, u1 = (uint32_t)c1, u2 = (uint32_t)c2;
-    const uint32_t bin = (u0 >> bs) + nb * ((u1 >> bs) + nb * (u2 >> bs));
-    const uint32_t brick = (u0 >> 3) + nbr * ((u1 >> 3) + nbr * (u2 >> 3));
-    const uint32_t local = (u0 & 7u) + 8u * ((u1 & 7u) + 8u * (u2 & 7u));
-    // both loads in flight together (the mask word of an empty bin is stale and unused);
-    // byte offsets below 2^32 (bins * 8 B, bricks * 64 B for n <= 1024), a bin entry's pair
-    // count is its low word
-    const uint32_t pairs = gld_at((const uint32_t*)P.bin_packed, bin * 8u);
-    const uint32_t word = gld_at(P.mask, brick * 64u + ((local >> 5) << 2));
-    const bool self = u0 == x && u1 == y && u2 == z;
-    if (!self && pairs != 0u && ((word >> (local & 31u)) & 1u) != 0u) return false;
-    q0 += s0;
-    q1 += s1;
-    q2 += s2;
+  // Brick by brick (8^3 voxels, all in one bin): the samples from q on that lie in q's brick
+  // are 1 + floor(e / |s|) of them along each axis, e the distance to the brick's last position
+  // on the way. k is the least of that or, for the rounding of the products, one less: the
+  // samples it leaves are met next time. A brick whose bin is empty is passed whole; of
+  // another kWalkTests samples are tested, their mask words loaded together.
+  const uint32_t n = P.n, bs = P.bin_shift + 16u, nsh = (uint32_t)__builtin_ctz(P.nbins_axis), nbr = n >> 3;
+  const uint32_t self_brick = (x >> 3) + nbr * ((y >> 3) + nbr * (z >> 3)), self_bit = (x & 7u) | (y & 7u) << 3 | (z & 7u) << 6;
+  const int32_t last = (8 << 16) - 1;
+  const int32_t d0 = ~(s0 >> 31), d1 = ~(s1 >> 31), d2 = ~(s2 >> 31);  // all ones: upwards
+  const float i0 = brick_samples(s0), i1 = brick_samples(s1), i2 = brick_samples(s2);
+  for (int32_t left = (int32_t)steps; left > 0;) {
+    if (((uint32_t)(q0 | q1 | q2) >> 16) >= n) return true;  // (n is a power of two)
+    const uint32_t bin = ((uint32_t)q0 >> bs) + (((uint32_t)q1 >> bs) << nsh) + (((uint32_t)q2 >> bs) << (2 * nsh));
+    const bool held = (bins(bin >> 5) >> (bin & 31u)) & 1u;
+    const float f = fminf(fminf((float)((q0 ^ d0) & last) * i0, (float)((q1 ^ d1) & last) * i1),
+                          (float)((q2 ^ d2) & last) * i2);
+    int32_t k = 1 + (int32_t)f;
+    if (held) {
+      k = min(k, kWalkTests);
+      const int32_t tests = min(k, left);
+      const uint32_t brick = ((uint32_t)q0 >> 19) + nbr * (((uint32_t)q1 >> 19) + nbr * ((uint32_t)q2 >> 19));
+      const uint32_t self = brick == self_brick ? self_bit : ~0u;
+      uint32_t word[kWalkTests], bit[kWalkTests];
+#pragma unroll
+      for (int j = 0; j < kWalkTests; j++) {  // (samples past k wrap within the brick and go unused)
+        bit[j] = __builtin_amdgcn_ubfe((uint32_t)(q0 + j * s0), 16, 3) | __builtin_amdgcn_ubfe((uint32_t)(q1 + j * s1), 16, 3) << 3 |
+                 __builtin_amdgcn_ubfe((uint32_t)(q2 + j * s2), 16, 3) << 6;
+        word[j] = gld_at(P.mask, brick * 64u + ((bit[j] >> 3) & 60u));  // byte offset < 2^32 for n <= 1024
+      }
+      uint32_t hit = 0;
+#pragma unroll
+      for (int j = 0; j < kWalkTests; j++)
+        hit |= j < tests && bit[j] != self ? __builtin_amdgcn_ubfe(word[j], bit[j], 1) : 0u;
+      if (hit) return false;
+    }
+    left -= k;
+    q0 += __mul24(k, s0);
+    q1 += __mul24(k, s1);
+    q2 += __mul24(k, s2);
   }
   return true;
+}
+
+// The mean normal of an occupied voxel from its record's count c (rc = 1 / c) and biased
+// sums, and the unbiased integer sums.
+struct VoxelNormal {
+  float x, y, z;
+  int32_t i0, i1, i2;
+};
+__device__ __forceinline__ VoxelNormal voxel_normal(uint32_t c, uint4 sums, float rc) {
+  const float inv = rc * 0x1p-10f;  // 1 / (1024 c): scaling by 2^-10 commutes with the rounding
+  const int32_t bias = (int32_t)(1024u * c);
+  VoxelNormal q;
+  q.i0 = (int32_t)sums.x - bias, q.i1 = (int32_t)sums.y - bias, q.i2 = (int32_t)sums.z - bias;
+  q.x = (float)q.i0 * inv, q.y = (float)q.i1 * inv, q.z = (float)q.i2 * inv;
+  return q;
+}
+__device__ __forceinline__ void voxel_centre(const MipScene& P, uint32_t x, uint32_t y, uint32_t z, float& px, float& py,
+                                             float& pz) {
+  px = P.origin[0] + ((float)x + 0.5f) * P.h;
+  py = P.origin[1] + ((float)y + 0.5f) * P.h;
+  pz = P.origin[2] + ((float)z + 0.5f) * P.h;
+}
+
+// The light's factor at a voxel centre (Lambert term, with the falloff for a point light)
+// and whether it reaches the voxel's front.
+__device__ __forceinline__ bool light_factor(const LightDev& L, float nx, float ny, float nz, float px, float py,
+                                             float pz, float& f) {
+  f = 0.f;
+  if (L.type == VGI_LIGHT_DIRECTIONAL) {
+    f = (nx * -L.vec[0] + ny * -L.vec[1]) + nz * -L.vec[2];
+    return f > 0.f;
+  }
+  const float dx = L.vec[0] - px, dy = L.vec[1] - py, dz = L.vec[2] - pz;
+  const float d2 = (dx * dx + dy * dy) + dz * dz;
+  if (!(d2 > 0.f)) return false;
+  const float cosv = ((nx * dx + ny * dy) + nz * dz) / __builtin_sqrtf(d2);
+  const float md = L.min_distance;
+  f = cosv / fmaxf(d2, md * md);
+  return cosv > 0.f;
+}
+
+// A scene's bin bits are kept in LDS up to this many bins an axis (4 KB), else read from memory.
+constexpr uint32_t kBitsAxis = 32;
+constexpr uint32_t kVisWaves = 4;
+constexpr uint32_t kVisBlocks = 8192;  // workgroups, which take the units in turn
+
+
+// Orders a wavefront's LDS accesses before and after it (they pass between its lanes).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
 
 // Radiance of an occupied level-0 voxel (x, y, z) from its accumulator record. SHADOW:
@@ -264,7 +349,11 @@ __device__ __forceinline__ uint32_t rounded_mean(uint32_t s, uint32_t c, float r
   return r < 0 ? q - 1u : (r >= (int32_t)c ? q + 1u : q);
 }
 
-template <bool SHADOW>
+// How the injecting launch cuts shadow-casting lights: not at all (no light casts shadows),
+// by the scene's vis bytes, or by its own walks.
+enum { kNoShadow = 0, kShadowVis = 1, kShadowWalk = 2 };
+
+template <int SHADOW>
 __device__ float4 inject(const MipScene& P, const float* lut, uint32_t x, uint32_t y, uint32_t z) {
   const uint32_t nbr = P.n >> 3;
   const uint32_t brick = (x >> 3) + nbr * ((y >> 3) + nbr * (z >> 3));
@@ -276,35 +365,29 @@ __device__ float4 inject(const MipScene& P, const float* lut, uint32_t x, uint32
   const float lr = lut[rounded_mean(s0.x, c, rc)];
   const float lg = lut[rounded_mean(s0.y, c, rc)];
   const float lb = lut[rounded_mean(s0.z, c, rc)];
-  const float inv = rc * 0x1p-10f;  // 1 / (1024 c): scaling by 2^-10 commutes with the rounding
-  const int32_t bias = (int32_t)(1024u * c);
-  const float nx = (float)((int32_t)s1.x - bias) * inv;
-  const float ny = (float)((int32_t)s1.y - bias) * inv;
-  const float nz = (float)((int32_t)s1.z - bias) * inv;
-  const float px = P.origin[0] + ((float)x + 0.5f) * P.h;
-  const float py = P.origin[1] + ((float)y + 0.5f) * P.h;
-  const float pz = P.origin[2] + ((float)z + 0.5f) * P.h;
+  const VoxelNormal q = voxel_normal(c, s1, rc);
+  const float nx = q.x, ny = q.y, nz = q.z;
+  float px, py, pz;
+  voxel_centre(P, x, y, z, px, py, pz);
+  uint32_t vis = 0;  // bit per shadow-casting light
+  if constexpr (SHADOW == kShadowVis)
+    for (uint32_t k = 0; k < P.vis_planes; k++)
+      vis |= (uint32_t)gld(P.vis + ((size_t)k * P.n * P.n * P.n + (size_t)brick * 512u + local)) << (8u * k);
   float er = 0.f, eg = 0.f, eb = 0.f;
   for (uint32_t l = 0; l < P.nlights; l++) {
     const LightDev& L = P.lights[l];
-    float f = 0.f;  // the light's factor: Lambert term, with the falloff for a point light
-    bool lit;
-    if (L.type == VGI_LIGHT_DIRECTIONAL) {
-      f = (nx * -L.vec[0] + ny * -L.vec[1]) + nz * -L.vec[2];
-      lit = f > 0.f;
-    } else {
-      const float dx = L.vec[0] - px, dy = L.vec[1] - py, dz = L.vec[2] - pz;
-      const float d2 = (dx * dx + dy * dy) + dz * dz;
-      lit = false;
-      if (d2 > 0.f) {
-        const float cosv = ((nx * dx + ny * dy) + nz * dz) / __builtin_sqrtf(d2);
-        lit = cosv > 0.f;
-        const float md = L.min_distance;
-        f = cosv / fmaxf(d2, md * md);
+    float f;
+    bool lit = light_factor(L, nx, ny, nz, px, py, pz, f);
+    if constexpr (SHADOW == kShadowVis) {
+      if (L.shadow) lit = lit && ((vis >> (L.shadow - 1u)) & 1u) != 0u;
+    } else if constexpr (SHADOW == kShadowWalk) {
+      const auto bins = [&](uint32_t w) { return gld(P.bin_bits + w); };
+      if (lit && L.shadow) {
+        int32_t o0, o1, o2;
+        walk_offset(q.i0, q.i1, q.i2, o0, o1, o2);
+        lit = light_visible(P, bins, L, x, y, z, o0, o1, o2);
       }
     }
-    if constexpr (SHADOW)  // one walk site for both kinds of light
-      if (lit && L.shadow) lit = light_visible(P, L, x, y, z, (int32_t)s1.x - bias, (int32_t)s1.y - bias, (int32_t)s1.z - bias);
     if (lit) {
       er = er + L.color[0] * f;
       eg = eg + L.color[1] * f;
@@ -312,6 +395,135 @@ __device__ float4 inject(const MipScene& P, const float* lut, uint32_t x, uint32
     }
   }
   return make_float4(lr * er, lg * eg, lb * eb, 1.0f);
+}
+
+// The units of a build's visibility walks: (brick * kVisUnits + k) for the k-th kVisVoxels occupied
+// voxels of an 8^3 brick, one thread a brick, appended with one atomic a wavefront.
+__global__ __launch_bounds__(256) void k_vis_list(const MipScene* __restrict__ scenes) {
+  const MipScene& P = scenes[blockIdx.y];
+  const uint32_t nbr = P.n >> 3, nbricks = nbr * nbr * nbr, brick = blockIdx.x * 256u + threadIdx.x;
+  if (P.vis_planes == 0u || blockIdx.x * 256u >= nbricks) return;
+  uint32_t units = 0;
+  if (brick < nbricks) {
+    const uint32_t bs = P.bin_shift - 3u, nb = P.nbins_axis;
+    const uint32_t bx = (brick % nbr) >> bs, by = ((brick / nbr) % nbr) >> bs, bz = (brick / (nbr * nbr)) >> bs;
+    if ((uint32_t)gld(P.bin_packed + (bx + nb * (by + nb * bz))) != 0u) {
+      uint32_t nocc = 0;
+#pragma unroll
+      for (uint32_t i = 0; i < 16u; i += 4u) {
+        const uint4 m = gld4(P.mask + (size_t)brick * 16u + i);
+        nocc += (uint32_t)(__popc(m.x) + __popc(m.y) + __popc(m.z) + __popc(m.w));
+      }
+      units = (nocc + kVisVoxels - 1u) / kVisVoxels;
+    }
+  }
+  const uint32_t lane = threadIdx.x & 63u;
+  uint32_t incl = units;
+#pragma unroll
+  for (uint32_t d = 1; d < 64u; d <<= 1) {
+    const uint32_t o = __shfl_up(incl, d);
+    if (lane >= d) incl += o;
+  }
+  uint32_t base = 0;
+  if (lane == 63u && incl) base = gatomic_add(P.vis_count, incl);
+  base = __shfl(base, 63) + incl - units;
+  for (uint32_t k = 0; k < units; k++) gst(P.vis_units + base + k, brick * kVisUnits + k);
+}
+
+// The visibility walks of a build. A wavefront takes a unit's voxels, lists the pairs of a
+// voxel and a light that reaches its front, for eight shadow-casting lights at a time, and
+// walks 64 pairs at once; the voxels' answers, a bit per light, go to the scene's vis bytes,
+// which the injecting launch reads.
+//
+// The walks were part of the injecting launch, one thread a voxel, light after light: its
+// length was that of the tile with most voxels, most of whose 25 walks in a row ran while
+// other CUs were idle (textured room at 128^3, four point lights: 114 us, of which 98 were
+// walks that keep the card's VALUs 15 us busy). Spread over the card in units of 32 voxels,
+// about one round of pairs with four lights: 35 us here, 20 in the injecting launch and 5 in
+// k_vis_list; the whole frame 408 -> 356 us (units of 16: 358), at 256^3 452 -> 353 (16:
+// 392), at 512^3 2102 -> 1291 (4096 workgroups: 1323).
+__global__ __launch_bounds__(64 * kVisWaves) void k_visibility(const MipScene* __restrict__ scenes) {
+  __shared__ uint32_t s_bits[kBitsAxis * kBitsAxis * kBitsAxis / 32];
+  __shared__ uint32_t s_vis[kVisWaves][64];
+  __shared__ uint16_t s_item[kVisWaves][64];
+  __shared__ uint16_t s_pair[kVisWaves][512];  // light << 6 | lane
+  const MipScene& P = scenes[blockIdx.y];
+  if (P.vis_planes == 0u) return;
+  const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t n = P.n, nbr = n >> 3, nb = P.nbins_axis, nlights = P.nlights;
+  const uint32_t total = __builtin_amdgcn_readfirstlane(gld(P.vis_count));
+  if (blockIdx.x * kVisWaves >= total) return;
+  const bool lds = nb <= kBitsAxis;
+  if (lds)
+    for (uint32_t w = threadIdx.x; w * 32u < nb * nb * nb; w += 64u * kVisWaves) s_bits[w] = gld(P.bin_bits + w);
+  __syncthreads();
+  const auto bins = [&](uint32_t w) { return lds ? s_bits[w] : gld(P.bin_bits + w); };
+  for (uint32_t u = blockIdx.x * kVisWaves + wave; u < total; u += gridDim.x * kVisWaves) {
+    const uint32_t unit = __builtin_amdgcn_readfirstlane(gld(P.vis_units + u));
+    const uint32_t brick = unit / kVisUnits, first = (unit % kVisUnits) * kVisVoxels;
+    const uint32_t bx = 8u * (brick % nbr), by = 8u * ((brick / nbr) % nbr), bz = 8u * (brick / (nbr * nbr));
+    const unsigned long long* mask = (const unsigned long long*)(P.mask + (size_t)brick * 16u);
+    uint32_t nocc = 0;
+#pragma unroll
+    for (uint32_t g = 0; g < 8u; g++) {  // 64 voxels each
+      const uint64_t m = mask[g];
+      const uint32_t rank = nocc + (uint32_t)__popcll(m & ((1ull << lane) - 1ull)) - first;
+      if (((m >> lane) & 1u) && rank < 64u) s_item[wave][rank] = (uint16_t)(64u * g + lane);
+      nocc += (uint32_t)__popcll(m);
+    }
+    wave_lds_fence();
+    const bool has = first + lane < nocc && lane < kVisVoxels;
+    const uint32_t v = has ? s_item[wave][lane] : 0u;
+    VoxelNormal q{};
+    float px = 0.f, py = 0.f, pz = 0.f;
+    uint32_t from = 0;  // voxel and start offset, one to three for -1 to 1 an axis
+    if (has) {
+      const uint32_t* a = P.acc + ((size_t)brick * 512u + v) * kAccWords;
+      const uint32_t c = gld(a + 3);
+      q = voxel_normal(c, gld4(a + 4), 1.0f / (float)c);
+      voxel_centre(P, bx + (v & 7u), by + ((v >> 3) & 7u), bz + (v >> 6), px, py, pz);
+      int32_t o0, o1, o2;
+      walk_offset(q.i0, q.i1, q.i2, o0, o1, o2);
+      from = v | (uint32_t)(o0 + 1) << 9 | (uint32_t)(o1 + 1) << 11 | (uint32_t)(o2 + 1) << 13;
+    }
+    for (uint32_t l = 0, plane = 0; plane < P.vis_planes; plane++) {
+      uint32_t pairs = 0;
+      for (uint32_t k = 0; k < 8u && l < nlights; l++) {
+        const LightDev& L = P.lights[l];
+        if (!L.shadow) continue;
+        k++;
+        float f;
+        const bool lit = has && light_factor(L, q.x, q.y, q.z, px, py, pz, f);
+        const uint64_t m = __ballot(lit);
+        if (lit) s_pair[wave][pairs + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)(l << 6 | lane);
+        pairs += (uint32_t)__popcll(m);
+      }
+      s_vis[wave][lane] = 0u;
+      wave_lds_fence();
+      for (uint32_t i = lane; i < ((pairs + 63u) & ~63u); i += 64u) {
+        const uint32_t pair = i < pairs ? s_pair[wave][i] : 0u;
+        const uint32_t w = __shfl(from, pair & 63u);
+        if (i >= pairs) continue;
+        const LightDev& L = P.lights[pair >> 6];
+        if (light_visible(P, bins, L, bx + (w & 7u), by + ((w >> 3) & 7u), bz + ((w >> 6) & 7u),
+                          (int32_t)((w >> 9) & 3u) - 1, (int32_t)((w >> 11) & 3u) - 1, (int32_t)(w >> 13) - 1))
+          atomicOr(&s_vis[wave][pair & 63u], 1u << ((L.shadow - 1u) & 7u));
+      }
+      wave_lds_fence();
+      if (has) gst(P.vis + ((size_t)plane * n * n * n + (size_t)brick * 512u + v), (uint8_t)s_vis[wave][lane]);
+    }
+  }
+}
+
+hipError_t launch_visibility(const MipScene* scenes, uint32_t count, uint32_t max_bricks, hipStream_t s) {
+  constexpr uint32_t kMaxY = 32768;
+  for (uint32_t i = 0; i < count; i += kMaxY) {
+    const uint32_t c = std::min(count - i, kMaxY);
+    hipLaunchKernelGGL(k_vis_list, dim3((max_bricks + 255) / 256, c), dim3(256), 0, s, scenes + i);
+    const uint32_t x = std::min(kVisUnits * max_bricks / kVisWaves, std::max(kVisBlocks / c, 64u));
+    hipLaunchKernelGGL(k_visibility, dim3(x, c), dim3(64 * kVisWaves), 0, s, scenes + i);
+  }
+  return hipGetLastError();
 }
 
 // Threads per 16^3 tile. The FP32 injecting launch without shadows runs 1024: its 64 KB LDS
@@ -322,11 +534,11 @@ __device__ float4 inject(const MipScene& P, const float* lut, uint32_t x, uint32
 // better (FP16 x-pair 67.5 us either way). With visibility walks 1024 threads were slower
 // (FP32 0.32 -> 0.43 ms, FP16 x-pair 0.28 -> 0.45 ms on the room's four shadowed lights).
 // The reducing launch runs one thread per 2x2x2 group of a 16^3 block.
-constexpr uint32_t mips_threads(int prec, bool src_acc, bool shadow) {
-  return src_acc && !shadow && prec == VGI_PREC_FP32 ? 1024u : 512u;
+constexpr uint32_t mips_threads(int prec, bool src_acc, int shadow) {
+  return src_acc && shadow != kShadowWalk && prec == VGI_PREC_FP32 ? 1024u : 512u;
 }
 
-template <int PREC, bool SRC_ACC, bool SHADOW>
+template <int PREC, bool SRC_ACC, int SHADOW>
 __global__ __launch_bounds__(1024) void k_mips(const MipScene* __restrict__ scenes,
                                                const MipBlock* __restrict__ blocks,
                                                const float* __restrict__ lut, uint32_t src1, uint32_t nout1,
@@ -524,16 +736,25 @@ __global__ __launch_bounds__(1024) void k_mips(const MipScene* __restrict__ scen
 
 template <int PREC>
 static void launch_mips_prec(const MipBatch& B, bool from_acc, dim3 g, hipStream_t s) {
-  const dim3 b(mips_threads(PREC, from_acc, from_acc && B.shadow));
-  if (!from_acc)
-    hipLaunchKernelGGL((k_mips<PREC, false, false>), g, b, 0, s, B.scenes, B.blocks, B.lut, B.src, B.nout,
-                       (const uint32_t*)nullptr, (uint32_t*)nullptr);
-  else if (B.shadow)
-    hipLaunchKernelGGL((k_mips<PREC, true, true>), g, b, 0, s, B.scenes, B.blocks, B.lut, B.src, B.nout,
-                       B.counts, B.clear_counts);
-  else
-    hipLaunchKernelGGL((k_mips<PREC, true, false>), g, b, 0, s, B.scenes, B.blocks, B.lut, B.src, B.nout,
-                       B.counts, B.clear_counts);
+  const int shadow = !from_acc || !B.shadow ? kNoShadow : B.vis ? kShadowVis : kShadowWalk;
+  const dim3 b(mips_threads(PREC, from_acc, shadow));
+#define VGI_LAUNCH(SRC_ACC, SHADOW, COUNTS, CLEAR) \
+  hipLaunchKernelGGL((k_mips<PREC, SRC_ACC, SHADOW>), g, b, 0, s, B.scenes, B.blocks, B.lut, B.src, B.nout, COUNTS, CLEAR)
+  if (!from_acc) VGI_LAUNCH(false, kNoShadow, (const uint32_t*)nullptr, (uint32_t*)nullptr);
+  else if (shadow == kShadowVis) VGI_LAUNCH(true, kShadowVis, B.counts, B.clear_counts);
+  else if (shadow == kShadowWalk) VGI_LAUNCH(true, kShadowWalk, B.counts, B.clear_counts);
+  else VGI_LAUNCH(true, kNoShadow, B.counts, B.clear_counts);
+#undef VGI_LAUNCH
+}
+
+// One bit per bin, set while the bin holds triangles: 256 bins of workgroup b. Also clears the
+// count of walk units (k_vis_list).
+__device__ __forceinline__ void bin_bits_block(const unsigned long long* bin_packed, uint32_t nb, uint32_t* bits,
+                                               uint32_t* vis_count, uint32_t b) {
+  const uint32_t nbins = nb * nb * nb, i = b * 256u + threadIdx.x;
+  if (i == 0u && vis_count) gst(vis_count, 0u);
+  const uint64_t m = __ballot(i < nbins && (uint32_t)gld(bin_packed + min(i, nbins - 1u)) != 0u);
+  if ((threadIdx.x & 31u) == 0u && i < nbins) gst(bits + (i >> 5), (uint32_t)(m >> (threadIdx.x & 32u)));
 }
 
 // The injecting launch's tiles for one scene, densest first: a tile is listed when its bins
@@ -550,6 +771,10 @@ constexpr uint32_t kDenseTilePairs = 384;
 __global__ __launch_bounds__(256) void k_tiles(TileArgs P, StageArgs stage) {
   if (blockIdx.x < stage.blocks) {  // the tables that the build's other kernels read
     stage_block(stage, blockIdx.x);
+    return;
+  }
+  if (P.bin_bits && blockIdx.x >= P.tile_blocks) {  // the bits that the visibility walks read
+    bin_bits_block(P.bin_packed, P.nbins_axis, P.bin_bits, P.vis_count, blockIdx.x - P.tile_blocks);
     return;
   }
   const uint32_t ns = P.n, S = ns < 16u ? ns : 16u, tpa = ns / S, ntl = tpa * tpa * tpa;
@@ -595,8 +820,21 @@ __global__ __launch_bounds__(256) void k_tiles(TileArgs P, StageArgs stage) {
   if (other) gst(P.order + ntl - 1u - (obase + (uint32_t)__popcll(om & below)), t);
 }
 
-hipError_t launch_tiles(const TileArgs& t, const StageArgs& a, uint32_t ntiles, hipStream_t s) {
-  hipLaunchKernelGGL(k_tiles, dim3(a.blocks + (ntiles + 255) / 256), dim3(256), 0, s, t, a);
+__global__ __launch_bounds__(256) void k_bin_bits(const MipScene* __restrict__ scenes) {
+  const MipScene& P = scenes[blockIdx.x];
+  if (blockIdx.y * 256u < P.nbins_axis * P.nbins_axis * P.nbins_axis)
+    bin_bits_block(P.bin_packed, P.nbins_axis, P.bin_bits, P.vis_count, blockIdx.y);
+}
+
+hipError_t launch_bin_bits(const MipScene* scenes, uint32_t count, uint32_t max_bins, hipStream_t s) {
+  hipLaunchKernelGGL(k_bin_bits, dim3(count, (max_bins + 255) / 256), dim3(256), 0, s, scenes);
+  return hipGetLastError();
+}
+
+hipError_t launch_tiles(TileArgs t, const StageArgs& a, uint32_t ntiles, hipStream_t s) {
+  t.tile_blocks = a.blocks + (ntiles + 255) / 256;
+  const uint32_t nbins = t.bin_bits ? t.nbins_axis * t.nbins_axis * t.nbins_axis : 0u;
+  hipLaunchKernelGGL(k_tiles, dim3(t.tile_blocks + (nbins + 255) / 256), dim3(256), 0, s, t, a);
   return hipGetLastError();
 }
 

@@ -178,7 +178,8 @@ struct LightDev {
   float vec[3];
   float color[3];
   float min_distance;
-  uint32_t shadow;  // 1: cut where the visibility walk toward the light meets an occupied voxel
+  uint32_t shadow;  // 1 + its number among the scene's such lights: cut where the visibility walk
+                    // toward the light meets an occupied voxel; 0: not cut
   int32_t step[3];  // directional, shadow: the walk's step toward the light, 16.16 fixed point
   float pv[3];      // point, shadow: position in voxel units of level 0, (vec - origin) / h
   uint32_t pad;
@@ -189,6 +190,10 @@ static_assert(sizeof(LightDev) == 64, "one light is 64 bytes of the descriptor u
 // visibility walk's precomputed step (directional) or voxel-unit position (point).
 LightDev light_dev(const vgi_light& L, const float origin[3], float h);
 
+constexpr uint32_t kMaxVisLights = 32;  // shadow-casting lights of a scene that vis bytes serve
+constexpr uint32_t kVisVoxels = 32;     // occupied voxels of a brick to a unit of walks
+constexpr uint32_t kVisUnits = 512 / kVisVoxels;  // units of a brick at most
+
 // One scene of a mip batch (device memory).
 struct MipScene {
   const uint32_t* acc;
@@ -198,6 +203,7 @@ struct MipScene {
                    // after the tiles' words, 8 words per tile: bit (ly + 16 lz) while that
                    // x-row's stored level-0 texels are not all zero
   uint32_t* order; // the injecting launch's tiles, dense ones first (one word per tile; k_tiles)
+  uint32_t* bin_bits;  // one bit per bin, set while it holds triangles (builds with visibility walks)
   void* level[VGI_MAX_LEVELS];
   uint32_t nk[VGI_MAX_LEVELS];
   uint32_t n;
@@ -208,6 +214,13 @@ struct MipScene {
   float origin[3];
   float h;
   const LightDev* lights;  // nlights entries, in the call's descriptor upload
+  // builds with visibility walks: per voxel (brick by brick, as the accumulator) the visible
+  // ones of the shadow-casting lights, eight to a plane of n^3 bytes; null: the injecting
+  // launch walks by itself
+  uint8_t* vis;
+  uint32_t* vis_units;  // the walks' units (k_vis_list), and their count
+  uint32_t* vis_count;
+  uint32_t vis_planes;
 };
 
 // Mip workgroup: scene, tile of its source level, source level, levels produced.
@@ -222,6 +235,9 @@ struct TileArgs {
   uint32_t* order;
   uint32_t* counts;
   uint32_t n, bin_shift, nbins_axis;
+  uint32_t* bin_bits;    // written too, if not null
+  uint32_t* vis_count;   // cleared with them, if not null
+  uint32_t tile_blocks;  // workgroups before those of bin_bits (launch_tiles)
 };
 
 struct MipBatch {
@@ -230,7 +246,8 @@ struct MipBatch {
                            // scene 0 with the launch's src and nout
   const float* lut;        // 256 entries: (i/255)^2.2
   uint32_t src, nout;
-  bool shadow;             // some light of the batch casts shadows (the injecting launch walks)
+  bool shadow;             // some light of the batch casts shadows
+  bool vis;                // and k_visibility has answered the walks (else the injecting launch walks)
   // an ordered build's injecting launch (one scene): block b takes the listed tile b; the
   // list's two counts (dense and other tiles), and the next build's pair, which it zeroes
   uint32_t* counts;
@@ -451,7 +468,9 @@ hipError_t launch_scatter(const VoxBatch& B, uint32_t nblk_b, uint32_t nblk_t, u
                           uint32_t zero_blocks, hipStream_t s);
 hipError_t launch_voxelize(const VoxBatch& B, uint32_t tile, uint32_t grid_blocks, hipStream_t s);
 hipError_t launch_mips(const MipBatch& B, uint32_t prec, bool from_acc, uint32_t blocks, hipStream_t s);
-hipError_t launch_tiles(const TileArgs& t, const StageArgs& a, uint32_t ntiles, hipStream_t s);
+hipError_t launch_tiles(TileArgs t, const StageArgs& a, uint32_t ntiles, hipStream_t s);
+hipError_t launch_visibility(const MipScene* scenes, uint32_t count, uint32_t max_bricks, hipStream_t s);
+hipError_t launch_bin_bits(const MipScene* scenes, uint32_t count, uint32_t max_bins, hipStream_t s);
 hipError_t launch_trace(const TraceBatch& B, bool buffer_path, hipStream_t s);
 // Morton keys of every pixel of a batch (entries seg[0]..seg[nscenes], padding included).
 hipError_t launch_morton_keys(const TraceBatch& B, uint32_t* keys, uint32_t* pix, uint32_t entries, hipStream_t s);

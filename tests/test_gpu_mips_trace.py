@@ -483,6 +483,61 @@ def test_shadowed_lights_bit_exact(ctx):
         sc.release()
 
 
+@pytest.mark.parametrize("n,bin_size", [(8, 8), (16, 16), (32, 8), (32, 32)])
+@pytest.mark.parametrize("count", [1, 8, 9, 32, 33])
+def test_shadow_casting_light_counts(ctx, n, bin_size, count):
+    """Eight lights' answers share a plane of bytes, and beyond 32 lights the injecting launch
+    walks by itself; a third of the lights cast no shadow and take no place among them."""
+    vgi = _vgi()
+    levels = int(np.log2(n))
+    w = sg.room(ntri=3000, n=n, levels=levels, width=32, height=18)
+    base = _shadow_lights(w)
+    rng = np.random.default_rng(count)
+    lights = []
+    while sum(bool(l["shadow"]) for l in lights) < count:
+        l = dict(base[len(lights) % len(base)])
+        l["color"] = tuple(rng.uniform(0.1, 1.0, 3))
+        l["shadow"] = len(lights) % 3 != 1
+        lights.append(l)
+    print(f"case shadow lights n={n} bin={bin_size} count={count}", flush=True)
+    acc, _ = orc.voxelize(w.positions, w.grid, albedo=w.albedo)
+    mesh = vgi.MeshData(ctx, w.positions.reshape(-1, 3), albedo=w.albedo)
+    sc = ctx.scene()
+    try:
+        ctx.set_tuning(bin_size=bin_size)
+        sc.voxelize([mesh], vgi.make_grid(**w.grid))
+        sc.build_mips(vgi.make_lights(lights), vgi.PREC_FP32)
+        ref = orc.inject_mips(acc, w.grid, lights, "fp32")
+        for k in range(levels):
+            assert np.array_equal(sc.read_level(k), ref[k]), f"level {k}"
+    finally:
+        ctx.set_tuning()
+        sc.release()
+
+
+def test_shadow_walks_at_512(ctx):
+    """64 bins an axis (their bits stay in memory) against 32 (in LDS), and against the
+    injecting launch's own walks, which 30 lights of no colour bring about."""
+    vgi = _vgi()
+    print("case shadow walks 512", flush=True)
+    w = sg.room(ntri=20_000, n=512, levels=6, width=32, height=18)
+    lights = _shadow_lights(w)
+    black = [dict(lights[0], color=(0.0, 0.0, 0.0))] * 30
+    mesh = vgi.MeshData(ctx, w.positions.reshape(-1, 3), albedo=w.albedo)
+    sc, out = ctx.scene(), []
+    try:
+        for bin_size, ls in ((8, lights), (16, lights), (16, lights + black)):
+            ctx.set_tuning(bin_size=bin_size)
+            sc.voxelize([mesh], vgi.make_grid(**w.grid))
+            sc.build_mips(vgi.make_lights(ls), vgi.PREC_FP32)
+            out.append([sc.read_level(k) for k in (3, 5)])
+        for o in out[1:]:
+            assert all(np.array_equal(a, b) for a, b in zip(out[0], o))
+    finally:
+        ctx.set_tuning()
+        sc.release()
+
+
 def test_shadowed_and_plain_scenes_in_one_batch(ctx, soup):
     """One mip batch with a shadowed-light scene and a plain-light scene: the launch walks for
     the batch, and each scene still equals the oracle under its own lights."""
