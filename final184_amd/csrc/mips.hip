@@ -20,8 +20,8 @@
 // are zero-filled when allocated, and the first launch stores a 16^3 tile (its level-0
 // texels and its blocks of the four levels above) only while the tile holds occupied
 // voxels, plus once, as zeros, when it has lost them; a per-tile word records which, and
-// for the 16-byte texel forms a level-0 x-row of a stored tile is stored only while it
-// holds voxels or held them at the last build (one bit per row). A surface leaves most
+// a level-0 x-row of a stored tile is stored only while it holds voxels or held them at the
+// last build (one bit per row). A surface leaves most
 // tiles empty (70% at 256^3 for the room), so most level bytes are not rewritten each
 // build, and every texel still equals the full computation.
 #include <algorithm>
@@ -599,12 +599,11 @@ __global__ __launch_bounds__(1024) void k_mips(const MipScene* __restrict__ scen
     // occupancy pass: 1 while its stored texels (level 0 and its blocks of the levels
     // produced here) are not all zero; and per level-0 x-row, 1 while the row's stored
     // texels are not all zero (the rows' words follow the tiles' words)
-    // (rows are skipped for the 16-byte texel forms, FP32 and FP16 x-pairs, whose level-0
-    // stores cost most; for 8-byte texels the row bookkeeping cost more than it saved)
-    constexpr bool ROWS = PREC == VGI_PREC_FP32 || PREC == VGI_PREC_FP16X2;
+    // (the launch is bound by what it stores: 16 soups with 8-byte texels 392 us with every
+    // row of a stored tile, 263 with these; the room's as before)
     const uint32_t ntiles = tpa * tpa * tpa, nrw = (S * S + 31u) >> 5;
     const uint32_t was_v = g == 0 ? gld(P.live + tile) : 0u;
-    const uint32_t rows_v = ROWS && g < nrw ? gld(P.live + ntiles + tile * 8u + g) : 0u;
+    const uint32_t rows_v = g < nrw ? gld(P.live + ntiles + tile * 8u + g) : 0u;
     uint16_t* s_item = (uint16_t*)s_a;  // occupied voxel list (group * 8 + bit), before s_a is used
     static_assert(sizeof(s_a) >= 4096 * sizeof(uint16_t), "item list fits in s_a");
     const uint32_t ssh = gsh + 1u, NV = S * S * S;
@@ -614,9 +613,23 @@ __global__ __launch_bounds__(1024) void k_mips(const MipScene* __restrict__ scen
     if (g < 8) s_rows_now[g] = 0u;
     __syncthreads();
     const uint32_t occ = grp ? group_occupancy(P, tx * S + 2 * gx, ty * S + 2 * gy, tz * S + 2 * gz) : 0u;
-    if constexpr (ROWS) {
+    // x-rows (2 gy + dy, 2 gz + dz) of the groups that hold voxels
+    if (S == 16u) {  // a wavefront has one gz, the 32 rows of one word, and eight lanes a row
+      uint32_t rows = 0;
 #pragma unroll
-      for (uint32_t q = 0; q < 4; q++)  // x-rows (2 gy + dy, 2 gz + dz) of the group that hold voxels
+      for (uint32_t q = 0; q < 4; q++) {
+        uint64_t m = __ballot(((occ >> (2 * q)) & 3u) != 0u);
+        m |= m >> 4;
+        m |= m >> 2;
+        m = (m | m >> 1) & 0x0101010101010101ull;  // bit 8 gy, and from there to bit 2 gy
+        m = (m | m >> 6) & 0x0005000500050005ull;
+        m = (m | m >> 12) & 0x0000005500000055ull;
+        rows |= ((uint32_t)(m | m >> 24) & 0x5555u) << ((q & 1u) + 16u * (q >> 1));
+      }
+      if (grp && lane == 0u) s_rows_now[gz] = rows;
+    } else {
+#pragma unroll
+      for (uint32_t q = 0; q < 4; q++)
         if ((occ >> (2 * q)) & 3u) {
           const uint32_t row = (2 * gy + (q & 1u)) + S * (2 * gz + (q >> 1));
           atomicOr(&s_rows_now[row >> 5], 1u << (row & 31u));
@@ -645,7 +658,7 @@ __global__ __launch_bounds__(1024) void k_mips(const MipScene* __restrict__ scen
     const uint32_t was = s_was;
     if (nocc == 0u && was == 0u) return;  // uniform: both values come from LDS
     if (g == 0 && (nocc != 0u) != (was != 0u)) gst(P.live + tile, nocc != 0u ? 1u : 0u);
-    if (ROWS && g < nrw && s_rows_now[g] != s_rows_prev[g]) gst(P.live + ntiles + tile * 8u + g, s_rows_now[g]);
+    if (g < nrw && s_rows_now[g] != s_rows_prev[g]) gst(P.live + ntiles + tile * 8u + g, s_rows_now[g]);
     for (uint32_t it = g; it < nocc; it += kThreads) {
       const uint32_t e = s_item[it], gi = e >> 3, bit = e & 7u;
       const uint32_t lx = 2 * (gi & (G - 1u)) + (bit & 1u);
@@ -671,7 +684,7 @@ __global__ __launch_bounds__(1024) void k_mips(const MipScene* __restrict__ scen
     } else {
       for (uint32_t v = g; v < NV; v += kThreads) {
         const uint32_t row = v >> ssh;
-        if (ROWS && !(((s_rows_now[row >> 5] | s_rows_prev[row >> 5]) >> (row & 31u)) & 1u)) continue;
+        if (!(((s_rows_now[row >> 5] | s_rows_prev[row >> 5]) >> (row & 31u)) & 1u)) continue;
         const uint32_t lx = v & (S - 1u), ly = (v >> ssh) & (S - 1u), lz = v >> (2 * ssh);
         TX::store_packed(P.level[0], padded_index(tx * S + lx, ty * S + ly, tz * S + lz, ns), s_val[v]);
       }

@@ -159,6 +159,30 @@ def test_mips_after_geometry_changes(ctx):
     sc.release()
 
 
+@pytest.mark.parametrize("prec", ["fp32", "fp16", "bf16", "fp16x2"])
+@pytest.mark.parametrize("n", [8, 16, 64])
+def test_mips_rows_follow_geometry(ctx, n, prec):
+    """Level-0 rows that lose their voxels are cleared and rows that gain some are stored: three
+    sparse soups of different seeds, one after another in one scene, then the first again."""
+    vgi = _vgi()
+    print(f"case mips rows n={n} {prec}", flush=True)
+    levels = int(np.log2(n))
+    ws = [sg.batch_scenes(seed=s, count=1, median=40 * n // 8, tri_range=(4, 40 * n), grids=(n,), sides=(16,))[0]
+          for s in (1, 2, 3)]
+    sc = ctx.scene()
+    try:
+        for w in ws + ws[:1]:
+            grid = dict(w.grid, levels=levels)
+            sc.voxelize([vgi.MeshData(ctx, w.positions.reshape(-1, 3), albedo=w.albedo)], vgi.make_grid(**grid))
+            sc.build_mips(vgi.make_lights(w.lights), vgi.PREC_NAMES[prec])
+            acc, _ = orc.voxelize(w.positions, grid, albedo=w.albedo)
+            ref = orc.inject_mips(acc, grid, w.lights, ORC_PREC[prec])
+            for k in range(levels):
+                assert np.array_equal(sc.read_level(k), ref[k]), f"level {k}"
+    finally:
+        sc.release()
+
+
 def test_trace_fp32_vs_fp64(ctx, soup):
     w = soup["w"]
     print(f"case {w.name} trace fp32", flush=True)
