@@ -755,8 +755,7 @@ int voxelize_batch(vgi_context* ctx, const vgi_voxelize_item* items, uint32_t co
   B.scan_flags = (uint32_t*)((uint8_t*)w->zeroed + flags_off);
   B.scan_vals = (unsigned long long*)w->scan_tmp;
   B.scan_spin = ctx->scan_spin;
-  B.work_map = (uint2*)w->work_map;
-  B.unit_order = (uint32_t*)(B.work_map + work_cap);
+  B.units = (uint32_t*)w->work_map;
   B.pairs_all = (uint32_t*)w->pairs;
   B.pair_cap = pair_cap;
   B.work_cap = work_cap;
@@ -1744,8 +1743,7 @@ int vgi_voxelize_noalloc(vgi_context* ctx, vgi_scene* sc, const vgi_mesh* meshes
   B.scan_flags = (uint32_t*)(base + o_zero + flags_off);
   B.scan_vals = (unsigned long long*)(base + o_stmp);
   B.scan_spin = ctx->scan_spin;
-  B.work_map = (uint2*)(base + o_work);
-  B.unit_order = (uint32_t*)(B.work_map + work_cap64);
+  B.units = (uint32_t*)(base + o_work);
   B.pairs_all = (uint32_t*)(base + o_pairs);
   B.pair_cap = (uint32_t)pair_cap64;
   B.work_cap = (uint32_t)work_cap64;

@@ -21,7 +21,9 @@ constexpr int kSmallBins = 8;          // a triangle whose bin box has <= 8 bins
 constexpr uint32_t kBlockTris = 256;   // triangles per setup / emit workgroup
 constexpr uint32_t kBlockBins = 256;   // bins per bins / workmap workgroup
 constexpr uint32_t kUnitItems = 16;    // chunks one voxelize workgroup takes in turn (8^3 bins)
-constexpr size_t kWorkEntryBytes = 12;  // per work unit: its (scene, bin) and its place in the order
+constexpr size_t kWorkEntryBytes = 12;  // per work unit (VoxBatch::units)
+constexpr uint32_t kUnitCountShift = 21;  // bins < 2^21 (1024^3 voxels in bins of 8^3)
+static_assert(kUnitItems * kMaxChunk <= 1u << (31 - kUnitCountShift), "a unit's pairs fit its record");
 
 // Per-mesh descriptor, device resident.
 struct MeshDev {
@@ -156,11 +158,12 @@ struct VoxBatch {
                                     // published (cleared with the overflow word)
   unsigned long long* scan_vals;    // per k_bins workgroup: its total, then its inclusive prefix
   uint32_t scan_spin;               // polls of a predecessor's flag before the look-back gives up
-  uint2* work_map;                  // (scene, bin) of every work unit (work_cap entries)
-  uint32_t* unit_order;             // the order k_voxelize takes the units in (work_cap entries)
+  // the work units in the order k_voxelize takes them, three words each (work_cap entries):
+  // scene; bin | (pairs - 1) << kUnitCountShift | several units in the bin << 31; first pair
+  uint32_t* units;
   uint32_t* pairs_all;              // triangle ids grouped by bin, every scene's bins in turn
   uint32_t pair_cap;                // entries of pairs_all
-  uint32_t work_cap;                // entries of work_map
+  uint32_t work_cap;                // entries of units
   uint32_t* overflow;               // device word: 1 when the pairs or units exceed the caps;
                                     // the two words after it (cleared with it) are the unit
                                     // order's front and back cursors, the third is set when

@@ -248,7 +248,7 @@ __device__ __forceinline__ bool bin_candidate(const VoxScene& S, const int64_t (
   return sat_box(q, N, b, dshift);
 }
 
-// a / b for a < 8 and 1 <= b <= 8
+// a / b for a < 256 and 1 <= b <= 16
 __device__ __forceinline__ uint32_t small_div(uint32_t a, uint32_t b) {
   return (uint32_t)(((float)a + 0.5f) * __builtin_amdgcn_rcpf((float)b));
 }
@@ -273,13 +273,9 @@ __device__ __forceinline__ uint2 tri_block(const VoxBatch& B) { return tri_block
 __device__ __forceinline__ uint2 bin_block(const VoxBatch& B) { return bin_block(B, blockIdx.x); }
 
 // Offset of bin b's first pair in the batch's pair list (the scenes' lists follow each
-// other in bin order, so this is the low half of the batch-wide exclusive scan), and its
-// first work unit within the batch (the high half).
+// other in bin order, so this is the low half of the batch-wide exclusive scan).
 __device__ __forceinline__ uint32_t pair_base(const VoxBatch& B, const VoxScene& S, uint32_t b) {
   return (uint32_t)gld(B.scan_all + S.bin_base + b);
-}
-__device__ __forceinline__ uint32_t first_item(const VoxBatch& B, const VoxScene& S, uint32_t b) {
-  return (uint32_t)(gld(B.scan_all + S.bin_base + b) >> 32);
 }
 
 // ---------------------------------------------------------------------------
@@ -827,7 +823,7 @@ __device__ void settle_wave(const VoxBatch& B, const VoxScene* __restrict__ scen
 }
 
 
-// work unit -> (scene, bin), from the scanned unit offsets; workgroup blk of the bins. Also
+// The work units' records (VoxBatch::units) of workgroup blk_id's bins, in
 // the order in which k_voxelize takes the units: those of two or more chunks first, from
 // the front of the order, then the single-chunk ones from the back. A unit's time grows
 // with its chunks (on the room a 4-chunk unit runs about 27 us against 5-8 us for one
@@ -839,17 +835,17 @@ __device__ __forceinline__ void workmap_block(const VoxBatch& B, const VoxScene*
   const VoxScene& P = scenes[blk.x];
   const uint32_t nbins = P.nbins_axis * P.nbins_axis * P.nbins_axis;
   const uint32_t b = blk.y + threadIdx.x;
-  uint32_t units = 0, first = 0, heavy = 0;
+  uint32_t units = 0, first = 0, pairs = 0, heavy = 0;
   if (b < nbins) {
     const unsigned long long packed = gld(P.bin_packed + b);
     units = (uint32_t)(packed >> 32);
     if (units) {
-      first = first_item(B, P, b);
+      first = pair_base(B, P, b);
+      pairs = (uint32_t)packed;
       // units 0 .. units-2 hold unit_items chunks each, the last one the rest
-      const uint32_t items = ((uint32_t)packed + P.chunk - 1) / P.chunk;
+      const uint32_t items = (pairs + P.chunk - 1) / P.chunk;
       const uint32_t last = items - (units - 1) * P.unit_items;
       heavy = (P.unit_items >= 2u ? units - 1u : 0u) + (last >= 2u ? 1u : 0u);
-      for (uint32_t i = 0; i < units; i++) gst2(B.work_map + first + i, make_uint2(blk.x, b));
     }
   }
   // places in the order: one cursor atomic per wavefront and class
@@ -878,7 +874,11 @@ __device__ __forceinline__ void workmap_block(const VoxBatch& B, const VoxScene*
   for (uint32_t i = 0; i < units; i++) {
     const bool h = i < heavy;  // units 0 .. heavy-1 are the heavy ones (the last may be light)
     const uint32_t pos = h ? hbase + i : nwork - 1u - (lbase + (i - heavy));
-    gst(B.unit_order + pos, first + i);
+    const uint32_t at = i * P.unit_items * P.chunk, cnt = min(P.unit_items * P.chunk, pairs - at);
+    uint32_t* rec = B.units + 3u * (size_t)pos;
+    gst(rec, blk.x);
+    gst(rec + 1, b | (cnt - 1u) << kUnitCountShift | (units > 1u ? 1u << 31 : 0u));
+    gst(rec + 2, first + at);
   }
 }
 
@@ -1318,6 +1318,12 @@ __device__ __forceinline__ void fallback_pass(const VoxBatch& B, const VoxScene*
   }
 }
 
+__device__ __forceinline__ void load_unit(const VoxBatch& B, uint32_t w, uint32_t (&rec)[3]) {
+  const uint32_t* r = B.units + 3u * (size_t)w;
+#pragma unroll
+  for (int i = 0; i < 3; i++) rec[i] = gld(r + i);
+}
+
 // Registers: the 8^3 tile's unit accumulators (14 per thread) are held at 6 waves per SIMD
 // (80 VGPRs; 6 resident workgroups per CU, as many as LDS allows at 25.5 KB each), which
 // keeps the binned path in registers (only the fallback pass spills: as a launch of its own
@@ -1347,28 +1353,31 @@ void k_voxelize(VoxBatch Bt, const VoxScene* __restrict__ scenes) {
     if (tid < 64u) settle_wave(Bt, scenes);
     return;
   }
-  if (gld(Bt.overflow) != 0u) {  // uniform over the launch
+  // The batch's work units, from the scan (the launch is sized from earlier calls: normally
+  // one unit per workgroup, and workgroups take further units in turn when it falls short).
+  // A unit's record says all that leads to its triangles, and the first is loaded with the
+  // two words that decide whether it counts: a chain of four loads to the triangle records
+  // where there were eight (the order, the unit's bin, the bin's pairs and offsets; 16 soups
+  // 439 -> 387 us, room 256^3 58 -> 55, 512^3 346 -> 330).
+  const uint32_t overflow = gld(Bt.overflow);
+  const unsigned long long totals = gld(Bt.scan_all + Bt.total_bins);
+  uint32_t rec[3] = {0u, 0u, 0u};
+  if (blockIdx.x < Bt.work_cap) load_unit(Bt, blockIdx.x, rec);
+  if (overflow != 0u) {  // uniform over the launch
     fallback_pass<TEX>(Bt, scenes, nwg);
     return;
   }
-  // the batch's work units, from the scan (the launch is sized from earlier calls: normally
-  // one unit per workgroup, and workgroups take further units in turn when it falls short)
-  const uint32_t nwork = (uint32_t)(gld(Bt.scan_all + Bt.total_bins) >> 32);
+  const uint32_t nwork = (uint32_t)(totals >> 32);
 
   for (uint32_t w = blockIdx.x; w < nwork; w += nwg) {
-    const uint32_t u = gld(Bt.unit_order + w);  // the longest units first
-    const uint2 item = gld2(Bt.work_map + u);
-    const VoxScene& P = scenes[item.x];
-    const uint32_t bin = item.y;
+    if (w != blockIdx.x) load_unit(Bt, w, rec);
+    const VoxScene& P = scenes[__builtin_amdgcn_readfirstlane(rec[0])];
+    const uint32_t word = __builtin_amdgcn_readfirstlane(rec[1]), base = __builtin_amdgcn_readfirstlane(rec[2]);
+    const uint32_t bin = word & ((1u << kUnitCountShift) - 1u);
+    const uint32_t npairs = ((word >> kUnitCountShift) & 1023u) + 1u;
+    const bool multi = (word >> 31) != 0u;  // other workgroups add into this bin: atomics
     const uint32_t nb = P.nbins_axis, B = 1u << P.bin_shift, nbr = P.n >> 3;
     const uint32_t sub = B / TS;  // sub-tiles per bin edge
-    const unsigned long long packed = gld(P.bin_packed + bin);
-    const uint32_t cnt_bin = (uint32_t)packed, units = (uint32_t)(packed >> 32);
-    const uint32_t unit = u - first_item(Bt, P, bin);
-    const uint32_t base = pair_base(Bt, P, bin);
-    const uint32_t items_bin = (cnt_bin + P.chunk - 1) / P.chunk;
-    const uint32_t it0 = unit * P.unit_items, it1 = min(it0 + P.unit_items, items_bin);
-    const bool multi = units > 1;  // other workgroups add into this bin: atomics
     const uint32_t bx = bin % nb, by = (bin / nb) % nb, bz = bin / (nb * nb);
     // A bin that is one 8^3 tile keeps its sums in registers across the chunks of its unit
     // (each thread owns tile entries tid and tid + 256) and is flushed once.
@@ -1379,9 +1388,9 @@ void k_voxelize(VoxBatch Bt, const VoxScene* __restrict__ scenes) {
 #pragma unroll
       for (int k = 0; k < 7; k++) racc[r][k] = 0u;
 
-    for (uint32_t it = it0; it < it1; it++) {
-      const uint32_t first = base + it * P.chunk;
-      const uint32_t cnt = min(P.chunk, cnt_bin - it * P.chunk);
+    for (uint32_t at = 0; at < npairs; at += P.chunk) {
+      const uint32_t first = base + at;
+      const uint32_t cnt = min(P.chunk, npairs - at);
       if ((tid & 63u) < cnt) {  // triangle tid % 64, coefficient part tid / 64
         const uint32_t t = gld(Bt.pairs_all + first + (tid & 63u));
         const TriRec R = gld_rec(P.tris + t);
@@ -1438,9 +1447,9 @@ void k_voxelize(VoxBatch Bt, const VoxScene* __restrict__ scenes) {
           const TriCoef& C = s_tri[lo];
           const uint32_t local = wi - s_pref[lo];
           const int u = (int)C.axis, A = (u + 1) % 3, Bx = (u + 2) % 3;
-          const int wa = C.chi[A] - C.clo[A] + 1;
-          const int va = C.clo[A] + (int)(local % (uint32_t)wa);
-          const int vb = C.clo[Bx] + (int)(local / (uint32_t)wa);
+          const uint32_t wa = (uint32_t)(C.chi[A] - C.clo[A] + 1), row = small_div(local, wa);
+          const int va = C.clo[A] + (int)(local - row * wa);
+          const int vb = C.clo[Bx] + (int)row;
           if (!edge_ok(C, u, va, vb)) continue;
           unsigned long long inc0 = C.inc0;
           if constexpr (TEX) {
@@ -1460,16 +1469,42 @@ void k_voxelize(VoxBatch Bt, const VoxScene* __restrict__ scenes) {
           int k1 = (int)floorf((zc + wd + 4.0f) * (1.0f / kFixedOne));
           k0 = max(k0, (int)C.clo[u]);
           k1 = min(k1, (int)C.chi[u]);
-          const int u1 = (u + 1) % 3, u2 = (u + 2) % 3;
-          for (int k = k0; k <= k1; k++) {
-            const int vx = (u == 0) ? k : (A == 0 ? va : vb);
-            const int vy = (u == 1) ? k : (A == 1 ? va : vb);
-            const int vz = (u == 2) ? k : (A == 2 ? va : vb);
-            const int64_t sv = C.N256[0] * vx + C.N256[1] * vy + C.N256[2] * vz;
-            if (sv + C.pmin > 0 || sv + C.pmax < 0) continue;
-            if (!edge_ok(C, u1, sel3(vx, vy, vz, (u1 + 1) % 3), sel3(vx, vy, vz, (u1 + 2) % 3))) continue;
-            if (!edge_ok(C, u2, sel3(vx, vy, vz, (u2 + 1) % 3), sel3(vx, vy, vz, (u2 + 2) % 3))) continue;
-            const int pi = (vx - tx0) + L::PY * (vy - ty0) + L::PZ * (vz - tz0);
+          if (k0 > k1) continue;
+          // Along the column the plane and the other two projections' edge functions (whose
+          // second and first coordinate k is) are linear in k; each takes its voxels k0 + i
+          // out of the column's bits, one set of values after another: with all of them held at
+          // once the kernel spills at six wavefronts a SIMD (16 soups 673 us, 470 with every
+          // test evaluated anew for each voxel, 439 so; room 256^3 76 / 63 / 58).
+          uint32_t in = 0;
+          {
+            const int64_t sk = C.N256[u], s0 = C.N256[A] * va + C.N256[Bx] * vb, pmin = C.pmin, pmax = C.pmax;
+            for (int k = k0; k <= k1; k++) {
+              const int64_t t = s0 + sk * k;
+              in |= (uint32_t)(t + pmin <= 0 && t + pmax >= 0) << (k - k0);
+            }
+          }
+          if (in == 0u) continue;
+          const auto edges = [&](const int32_t* ev, const int32_t* ek, const int64_t* ec, int v) {
+            int64_t e0[3];
+            int32_t e1[3];
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+              e0[i] = (int64_t)ev[i] * v + ec[i];
+              e1[i] = ek[i];
+            }
+            for (uint32_t m = in; m != 0u; m &= m - 1u) {
+              const int i = __builtin_ctz(m), k = k0 + i;
+              const int64_t out = ((int64_t)e1[0] * k + e0[0]) | ((int64_t)e1[1] * k + e0[1]) | ((int64_t)e1[2] * k + e0[2]);
+              if (out < 0) in &= ~(1u << i);
+            }
+          };
+          edges(C.eA + 3 * A, C.eB + 3 * A, C.eC + 3 * A, vb);
+          edges(C.eB + 3 * Bx, C.eA + 3 * Bx, C.eC + 3 * Bx, va);
+          const int pa = A == 0 ? 1 : (A == 1 ? L::PY : L::PZ), pb = Bx == 0 ? 1 : (Bx == 1 ? L::PY : L::PZ);
+          const int pu = u == 0 ? 1 : (u == 1 ? L::PY : L::PZ);
+          const int p0 = pa * va + pb * vb - (tx0 + L::PY * ty0 + L::PZ * tz0) + pu * k0;
+          for (; in != 0u; in &= in - 1u) {
+            const int pi = p0 + pu * __builtin_ctz(in);
             atomicAdd(&s_acc0[pi], inc0);
             atomicAdd(&s_acc1[pi], C.inc1);
           }

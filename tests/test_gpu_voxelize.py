@@ -64,6 +64,30 @@ def test_bins_and_chunks_same_result(ctx, bin_size, chunk):
     assert np.array_equal(acc, ref), _diff_msg(acc, ref)
 
 
+@pytest.mark.parametrize("count,chunk", [(64, 64), (65, 64), (1024, 64), (1025, 64), (2500, 64), (16, 1), (33, 1)])
+def test_units_of_a_full_bin(ctx, count, chunk):
+    """A bin's triangles are taken in units of up to sixteen chunks: one unit, one of exactly
+    1024 pairs, and several that add into the bin. The triangles lie within the last 8^3 bin
+    of the grid, in every dominant direction and up to the bin's length."""
+    print(f"case units count={count} chunk={chunk}", flush=True)
+    rng = np.random.default_rng(count + chunk)
+    n = 32
+    pos = (n - 8 + 0.05 + 7.9 * rng.random((count, 3, 3))) / n
+    pos[::2] = np.clip(pos[::2, :1] + 0.03 * (rng.random((len(pos[::2]), 3, 3)) - 0.5), (n - 7.95) / n, (n - 0.05) / n)
+    pos = pos.astype(np.float32)
+    alb = rng.integers(0, 256, (count, 3), dtype=np.uint8)
+    grid = dict(origin=(0.0, 0.0, 0.0), extent=1.0, n=n, levels=5)
+    ref, _ = orc.voxelize(pos, grid, albedo=alb)
+    vgi = _vgi()
+    mesh = vgi.MeshData(ctx, pos.reshape(-1, 3), albedo=alb)
+    try:
+        ctx.set_tuning(bin_size=8, chunk_tris=chunk)
+        acc, _ = _gpu_acc(ctx, [mesh], grid)
+    finally:
+        ctx.set_tuning()
+    assert np.array_equal(acc, ref), _diff_msg(acc, ref)
+
+
 def test_room_128_bit_exact(ctx):
     vgi = _vgi()
     w = sg.room(ntri=60_000, n=128, levels=7, width=64, height=36)
