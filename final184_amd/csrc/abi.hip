@@ -1160,6 +1160,10 @@ constexpr uint32_t kTraceBandRows = 1;
 // with four). Sorted pixels take four too: their footprints are scattered, and the fewer
 // blocks a CU holds the more of them its L1 keeps (a frame of 16 scenes in Morton order,
 // FP16: 3.69 ms with two, 3.63 with three, 3.54 with four; 3.61 with a wavefront each).
+// (Scattered pixels left in tile order lose by sharing once they are many: 1636 x 1504
+// points, 4 + 1 cones, BF16, 4.61 ms when one wavefront of a kernel of its own marched each
+// block, 4.93 with two, 4.81 with four; a camera's G-buffer of that size gains, 644 us against
+// 625, and what kind a G-buffer is the launch does not know. Morton order is for the former.)
 constexpr size_t kManyTraceBlocks = 12000;
 // From here a launch fills the chip (k_trace's registers: trace_waves).
 constexpr size_t kFullTraceBlocks = 5000;
