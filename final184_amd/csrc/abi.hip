@@ -1160,14 +1160,20 @@ constexpr uint32_t kTraceBandRows = 1;
 // with four). Sorted pixels take four too: their footprints are scattered, and the fewer
 // blocks a CU holds the more of them its L1 keeps (a frame of 16 scenes in Morton order,
 // FP16: 3.69 ms with two, 3.63 with three, 3.54 with four; 3.61 with a wavefront each).
-// (Scattered pixels left in tile order lose by sharing once they are many: 1636 x 1504
-// points, 4 + 1 cones, BF16, 4.61 ms when one wavefront of a kernel of its own marched each
-// block, 4.93 with two, 4.81 with four; a camera's G-buffer of that size gains, 644 us against
-// 625, and what kind a G-buffer is the launch does not know. Morton order is for the former.)
+//
+// From kOneTraceBlocks up to ten diffuse cones a wavefront takes a block alone again
+// (k_trace_one), but for FP32. There sharing is worth little to a camera's G-buffer and costs
+// scattered pixels in tile order (room and soup, 1636 x 1504, 4 + 1 cones, one / two
+// wavefronts: BF16 618 / 628 us and 4.62 / 4.93 ms, FP16 601 / 599 and 4.60 / 4.77, x-pair
+// 500 / 509 and 4.82 / 5.14; room, 1920 x 1080, 9 + 1: 910 / 905, 891 / 874, 726 / 720),
+// while at 1280 x 720 it is worth 5% (BF16 454 / 433). FP32 gains at every size (room at
+// 1080p 878 / 818).
+constexpr size_t kOneTraceBlocks = 24000;
 constexpr size_t kManyTraceBlocks = 12000;
 // From here a launch fills the chip (k_trace's registers: trace_waves).
 constexpr size_t kFullTraceBlocks = 5000;
-uint32_t trace_wavefronts(size_t blocks, uint32_t cones, uint32_t diffuse, bool sorted) {
+uint32_t trace_wavefronts(size_t blocks, uint32_t cones, uint32_t diffuse, bool sorted, uint32_t prec) {
+  if (!sorted && prec != VGI_PREC_FP32 && diffuse <= 10 && blocks >= kOneTraceBlocks) return 1u;
   const uint32_t w = sorted || diffuse > 10 ? 4u : blocks < kManyTraceBlocks ? 3u : 2u;
   return std::max(1u, std::min(w, cones));
 }
@@ -1270,7 +1276,7 @@ int trace_batch(vgi_context* ctx, const vgi_trace_item* items, uint32_t count, v
     // bands of kTraceBandRows rows of the first item's tiles
     L.band = morton ? 0u : kTraceBandRows * (tp[group[p][0]].tiles_x << sub_shift);
     L.shared = L.buffer_path && L.nblocks <= kSharedTraceBlocks;
-    L.waves = L.shared ? shared_wavefronts(p, cones, L.max_diffuse) : trace_wavefronts(L.nblocks, cones, L.max_diffuse, morton);
+    L.waves = L.shared ? shared_wavefronts(p, cones, L.max_diffuse) : trace_wavefronts(L.nblocks, cones, L.max_diffuse, morton, p);
     L.full = L.nblocks >= kFullTraceBlocks;
     if (L.nblocks >= (1ull << 31) || L.entries >= (1ull << 32))
       return fail(VGI_E_RANGE, "trace batch too large (%zu workgroups)", L.nblocks);

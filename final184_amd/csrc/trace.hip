@@ -624,7 +624,8 @@ enum { kOx, kOy, kOz, kNx, kNy, kNz, kAb, kFrameWords };
 // contraction off: what the compiler fuses by itself depends on the block that a product
 // lands in, and the outputs' bits must not.
 
-// Writes pixel p's frame to f; false (no cones, outputs zero) for a zero normal.
+// Writes pixel p's frame to f, a word every ST; false (no cones, outputs zero) for a zero normal.
+template <int ST>
 __device__ __forceinline__ bool make_frame(const TraceParams& P, size_t p, float* f) {
 #pragma clang fp contract(off)
   const float px = gld(P.pos + p * 3), py = gld(P.pos + p * 3 + 1), pz = gld(P.pos + p * 3 + 2);
@@ -635,17 +636,17 @@ __device__ __forceinline__ bool make_frame(const TraceParams& P, size_t p, float
   const float nx = Nx * inv, ny = Ny * inv, nz = Nz * inv;
   const float off = P.normal_off * P.h;
   const float sign = copysignf(1.0f, nz);
-  f[64 * kOx] = fmaf(nx, off, px), f[64 * kOy] = fmaf(ny, off, py), f[64 * kOz] = fmaf(nz, off, pz);
-  f[64 * kNx] = nx, f[64 * kNy] = ny, f[64 * kNz] = nz;
-  f[64 * kAb] = -1.0f / (sign + nz);
+  f[ST * kOx] = fmaf(nx, off, px), f[ST * kOy] = fmaf(ny, off, py), f[ST * kOz] = fmaf(nz, off, pz);
+  f[ST * kNx] = nx, f[ST * kNy] = ny, f[ST * kNz] = nz;
+  f[ST * kAb] = -1.0f / (sign + nz);
   return true;
 }
 
-template <int PREC, bool BUF>
+template <int PREC, bool BUF, int ST>
 __device__ __forceinline__ float4 march_diffuse(const TraceParams& P, const float* f, uint32_t c, uint32_t& count) {
 #pragma clang fp contract(off)
   const float lx = P.dirs[c][0], ly = P.dirs[c][1], lz = P.dirs[c][2];
-  const float nx = f[64 * kNx], ny = f[64 * kNy], nz = f[64 * kNz], ab = f[64 * kAb];
+  const float nx = f[ST * kNx], ny = f[ST * kNy], nz = f[ST * kNz], ab = f[ST * kAb];
   // tangent (t0, t1, t2), bitangent (bb, b1, -ny)
   const float sign = copysignf(1.0f, nz);
   const float bb = nx * ny * ab;
@@ -654,7 +655,7 @@ __device__ __forceinline__ float4 march_diffuse(const TraceParams& P, const floa
   const float dx = fmaf(nx, lz, fmaf(t0, lx, bb * ly));
   const float dy = fmaf(ny, lz, fmaf(t1, lx, b1 * ly));
   const float dz = fmaf(nz, lz, fmaf(t2, lx, -ny * ly));
-  const float ox = f[64 * kOx], oy = f[64 * kOy], oz = f[64 * kOz];
+  const float ox = f[ST * kOx], oy = f[ST * kOy], oz = f[ST * kOz];
   return BUF ? cone_march_fixed<PREC>(P, P.sched[0], P.sched_len[0], ox, oy, oz, dx, dy, dz, count)
              : cone_march_lane<PREC, BUF>(P, ox, oy, oz, dx, dy, dz, P.tan_d, count);
 }
@@ -663,10 +664,11 @@ __device__ __forceinline__ float4 march_diffuse(const TraceParams& P, const floa
 struct Specular {
   float x, y, z, tan_half;
 };
+template <int ST>
 __device__ __forceinline__ Specular specular_cone(const TraceParams& P, const float* f, size_t p) {
 #pragma clang fp contract(off)
   const float px = gld(P.pos + p * 3), py = gld(P.pos + p * 3 + 1), pz = gld(P.pos + p * 3 + 2);
-  const float nx = f[64 * kNx], ny = f[64 * kNy], nz = f[64 * kNz];
+  const float nx = f[ST * kNx], ny = f[ST * kNy], nz = f[ST * kNz];
   const float vx = P.eye[0] - px, vy = P.eye[1] - py, vz = P.eye[2] - pz;
   const float vl2 = fmaf(vz, vz, fmaf(vx, vx, vy * vy));
   const float vi = vl2 > 0.f ? 1.0f / __builtin_sqrtf(vl2) : 0.f;
@@ -678,10 +680,10 @@ __device__ __forceinline__ Specular specular_cone(const TraceParams& P, const fl
   return s;
 }
 
-template <int PREC, bool BUF>
+template <int PREC, bool BUF, int ST>
 __device__ __forceinline__ float4 march_specular(const TraceParams& P, const float* f, size_t p, uint32_t& count) {
-  const Specular s = specular_cone(P, f, p);
-  const float ox = f[64 * kOx], oy = f[64 * kOy], oz = f[64 * kOz];
+  const Specular s = specular_cone<ST>(P, f, p);
+  const float ox = f[ST * kOx], oy = f[ST * kOy], oz = f[ST * kOz];
   if (BUF && !P.rough) return cone_march_fixed<PREC>(P, P.sched[1], P.sched_len[1], ox, oy, oz, s.x, s.y, s.z, count);
   return cone_march_lane<PREC, BUF>(P, ox, oy, oz, s.x, s.y, s.z, s.tan_half, count);
 }
@@ -765,7 +767,7 @@ void k_trace(TraceBatch Bt, const TraceParams* __restrict__ scenes, const uint2*
   uint32_t count = 0;
   const float* frame = s_frame + lane;
   if (wave == 0) {
-    const uint64_t m = __ballot(active && make_frame(P, p, s_frame + lane));
+    const uint64_t m = __ballot(active && make_frame<64>(P, p, s_frame + lane));
     if (lane == 0) s_cones = m;
   }
   const bool spec = P.out_s && P.specular;
@@ -775,7 +777,7 @@ void k_trace(TraceBatch Bt, const TraceParams* __restrict__ scenes, const uint2*
     if (spec) {
       __shared__ uint64_t s_valid[2 * kMaxSharedWaves];
       Specular c{0.f, 0.f, 0.f, 0.f};
-      if (cones) c = specular_cone(P, frame, p);
+      if (cones) c = specular_cone<64>(P, frame, p);
       const float4 r = cone_march_shared<PREC, BUF>(P, BUF && !P.rough, frame[64 * kOx], frame[64 * kOy], frame[64 * kOz],
                                                     c.x, c.y, c.z, c.tan_half, cones, s_cone + 64u * Bt.max_diffuse,
                                                     s_valid, count);
@@ -787,8 +789,8 @@ void k_trace(TraceBatch Bt, const TraceParams* __restrict__ scenes, const uint2*
   for (uint32_t k = wave; k < ntask;) {
     const uint32_t c = spec_task ? k - 1u : k;  // diffuse cone, or all ones for the specular cone
     if (cones) {
-      if (!SHARED && c == ~0u) store_out(P.out_s + p, march_specular<PREC, BUF>(P, frame, p, count));
-      else s_cone[64u * c + lane] = march_diffuse<PREC, BUF>(P, frame, c, count);
+      if (!SHARED && c == ~0u) store_out(P.out_s + p, march_specular<PREC, BUF, 64>(P, frame, p, count));
+      else s_cone[64u * c + lane] = march_diffuse<PREC, BUF, 64>(P, frame, c, count);
     }
     uint32_t next = 0;
     if (lane == 0) next = atomicAdd(&s_next, 1u);
@@ -815,12 +817,56 @@ void k_trace(TraceBatch Bt, const TraceParams* __restrict__ scenes, const uint2*
   if (Bt.counter) add_count(Bt.counter, count);
 }
 
+// A wavefront for each 8x8 block, marching every cone in turn with the block's frames in
+// registers: for launches of many blocks, where sharing gains a camera's G-buffer little
+// and costs scattered ones 3-7% (the host's kOneTraceBlocks).
+template <int PREC>
+__global__ __launch_bounds__(64) void k_trace_one(TraceBatch Bt, const TraceParams* __restrict__ scenes,
+                                                  const uint2* __restrict__ blocks) {
+  const uint32_t idx = work_index(Bt, blockIdx.x);
+  const uint32_t lane = threadIdx.x;
+  const uint32_t sub = idx & ((1u << Bt.sub_shift) - 1u), item = idx >> Bt.sub_shift;
+  const uint2 st = Bt.nscenes == 1 ? make_uint2(0u, item) : blocks[item];
+  const TraceParams& P = scenes[st.x];
+  const uint32_t tx = st.y % P.tiles_x, ty = st.y / P.tiles_x;
+  const uint32_t bw = Bt.tile_w >> 3;  // 1, 2 or 4 blocks per tile row
+  const uint32_t px = tx * Bt.tile_w + (sub & (bw - 1u)) * 8u + (lane & 7u);
+  const uint32_t py = ty * Bt.tile_h + (sub / bw) * 8u + (lane >> 3);
+  const size_t p = (size_t)py * P.width + px;
+  uint32_t count = 0;
+  if (px < P.width && py < P.height) {
+    float f[kFrameWords];
+    float4 od = make_float4(0.f, 0.f, 0.f, 0.f), os = od;
+    if (make_frame<1>(P, p, f)) {
+      float4 s = od;
+      for (uint32_t c = 0; c < P.num_diffuse; c++) {
+        const float4 r = march_diffuse<PREC, true, 1>(P, f, c, count);
+        const float wc = P.w[c];
+        s.x = fmaf(wc, r.x, s.x);
+        s.y = fmaf(wc, r.y, s.y);
+        s.z = fmaf(wc, r.z, s.z);
+        s.w = fmaf(wc, r.w, s.w);
+      }
+      od = make_float4(s.x, s.y, s.z, 1.0f - s.w);
+      if (P.out_s && P.specular) os = march_specular<PREC, true, 1>(P, f, p, count);
+    }
+    store_out(P.out_d + p, od);
+    if (P.out_s) store_out(P.out_s + p, os);
+  }
+  if (Bt.counter) add_count(Bt.counter, count);
+}
+
 template <int PREC, bool SORTED>
 static void launch_trace_prec(const TraceBatch& B, bool buffer_path, hipStream_t s) {
   const dim3 grid(B.nblocks), block(64u * B.waves);
   const uint32_t lds = (B.max_diffuse + (B.shared ? 2u * B.waves : 0u)) * 64u * (uint32_t)sizeof(float4);
 #define VGI_LAUNCH(BUF, FULL, SHARED) \
   hipLaunchKernelGGL((k_trace<PREC, BUF, SORTED, FULL, SHARED>), grid, block, lds, s, B, B.scenes, B.blocks, B.skeys, B.spix)
+  if constexpr (!SORTED)
+    if (buffer_path && B.waves == 1) {
+      hipLaunchKernelGGL((k_trace_one<PREC>), grid, block, 0, s, B, B.scenes, B.blocks);
+      return;
+    }
   if (!buffer_path) VGI_LAUNCH(false, false, false);
   else if (B.shared) VGI_LAUNCH(true, false, true);
   else if (PREC == VGI_PREC_FP32 && B.full) VGI_LAUNCH(true, PREC == VGI_PREC_FP32, false);  // (other forms: one variant)

@@ -594,12 +594,13 @@ def test_trace_is_independent_of_launch_size(ctx, soup, prec, rough):
     register variant for each side: the first rows of a large G-buffer, traced by themselves,
     give the same bits. 200 x 200 pixels (625 blocks) are past the line for the specular
     cone, 728 x 728 (8281) past the one where FP32 changes its variant, 888 x 888 (12321)
-    past the one where two wavefronts share a block."""
+    past the one where two wavefronts share a block, 1240 x 1240 (24025) past the one where
+    a wavefront takes a block alone."""
     vgi = _vgi()
     w = soup["w"]
     f = Frame(ctx, w, prec)
     rng = np.random.default_rng(9)
-    pick = rng.integers(0, w.num_pixels, 888 * 888)
+    pick = rng.integers(0, w.num_pixels, 1240 * 1240)
     pos, nrm = w.gb_pos[pick].copy(), w.gb_nrm[pick].copy()
     nrm[rng.random(len(pick)) < 0.02] = 0.0  # pixels without a surface
     tan = rng.uniform(0.0, 1.2, len(pick)).astype(np.float32) if rough else None
@@ -612,7 +613,7 @@ def test_trace_is_independent_of_launch_size(ctx, soup, prec, rough):
         return od.numpy(), osp.numpy()
 
     d0, s0 = trace(72 * 9, 72, 9)
-    for side in (200, 728, 888):
+    for side in (200, 728, 888, 1240):
         print(f"case trace {prec} rough={rough} {side}x{side}", flush=True)
         d, s = trace(side * side, side, side)
         assert np.array_equal(d[:len(d0)], d0) and np.array_equal(s[:len(s0)], s0)
