@@ -238,7 +238,9 @@ struct vgi_scene {
   // The injecting launch's tile list has two pairs of counts, used in turn by the ordered
   // builds: a build's list goes with one pair, which is zero, and its injecting launch zeroes
   // the other for the next build. tile_counts_zero is false while that is not known (a call
-  // that failed in between); the next ordered build then clears both.
+  // that failed in between); the next ordered build then clears both. A third pair serves the
+  // builds recorded in HIP graphs, of whose runs the host knows nothing: they clear it
+  // themselves and leave the other two alone.
   bool tile_counts_zero = false;
   uint32_t tile_pair = 0;
   bool has_voxels = false, has_mips = false;
@@ -301,6 +303,14 @@ vgi_workspace* workspace(vgi_context* ctx, hipStream_t st) {
   vgi_workspace* raw = w.get();
   ctx->ws.emplace(st, std::move(w));
   return raw;
+}
+
+// Whether work enqueued on the stream is recorded in a graph instead of run.
+int stream_capturing(hipStream_t st, bool* out) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  HIP_TRY(hipStreamIsCapturing(st, &status));
+  *out = status != hipStreamCaptureStatusNone;
+  return VGI_OK;
 }
 
 vgi_tuning tuning_of(vgi_context* ctx) {
@@ -925,10 +935,10 @@ int mips_batch(vgi_context* ctx, const vgi_mips_item* items, uint32_t count, uin
     vis_need += align_up(n * n * n * ((ns + 7) / 8), 256) + (ns ? align_up(n * n * n / kVisVoxels * sizeof(uint32_t), 256) : 0);
   }
   vis = vis && shadow;
+  bool captured = false;
+  TRY(stream_capturing(st, &captured));
   if (vis && w->vis_bytes < vis_need) {
-    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-    HIP_TRY(hipStreamIsCapturing(st, &capturing));
-    vis = capturing == hipStreamCaptureStatusNone;
+    vis = !captured;
     if (vis) HIP_TRY(hipStreamSynchronize(st));
     vis = vis && grow_bytes(&w->vis, &w->vis_bytes, vis_need, "visibility") == VGI_OK;
   }
@@ -1015,10 +1025,15 @@ int mips_batch(vgi_context* ctx, const vgi_mips_item* items, uint32_t count, uin
         const vgi_grid& g = sc->grid;
         const size_t tpa = g.n / std::min<uint32_t>(g.n, 16u), ntl = tpa * tpa * tpa;
         uint32_t* counts = sc->live + 10 * ntl;
-        if (!sc->tile_counts_zero) HIP_TRY(launch_fill_u32(counts, 0u, 4, st));
-        sc->tile_counts_zero = false;
-        B.counts = counts + 2 * sc->tile_pair;
-        B.clear_counts = counts + 2 * (sc->tile_pair ^ 1u);
+        if (captured) {  // may run any number of times, between any other builds of the scene
+          B.counts = counts + 4;
+          HIP_TRY(launch_fill_u32(B.counts, 0u, 2, st));
+        } else {
+          if (!sc->tile_counts_zero) HIP_TRY(launch_fill_u32(counts, 0u, 4, st));
+          sc->tile_counts_zero = false;
+          B.counts = counts + 2 * sc->tile_pair;
+          B.clear_counts = counts + 2 * (sc->tile_pair ^ 1u);
+        }
         const TileArgs t{(const unsigned long long*)sc->bin_packed, sc->live, sc->live + 9 * ntl, B.counts, g.n,
                          sc->bin_shift, sc->nbins_axis, shadow ? sc->live + 10 * ntl + 64 : nullptr, sc->live + 10 * ntl + 32, 0};
         HIP_TRY(launch_tiles(t, stage, (uint32_t)ntl, st));
@@ -1028,7 +1043,7 @@ int mips_batch(vgi_context* ctx, const vgi_mips_item* items, uint32_t count, uin
       }
       if (j == 0 && vis) HIP_TRY(launch_visibility(B.scenes, count, max_bricks, st));
       HIP_TRY(launch_mips(B, precision, j == 0, (uint32_t)stages[j].size(), st));
-      if (B.counts) {
+      if (B.clear_counts) {
         items[0].scene->tile_counts_zero = true;
         items[0].scene->tile_pair ^= 1u;
       }

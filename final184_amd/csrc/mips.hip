@@ -829,8 +829,9 @@ __global__ __launch_bounds__(256) void k_tiles(TileArgs P, StageArgs stage) {
   }
   dbase = __shfl(dbase, 0);
   obase = __shfl(obase, 0);
-  if (dense) gst(P.order + dbase + (uint32_t)__popcll(dm & below), t);
-  if (other) gst(P.order + ntl - 1u - (obase + (uint32_t)__popcll(om & below)), t);
+  const uint32_t dat = dbase + (uint32_t)__popcll(dm & below), oat = obase + (uint32_t)__popcll(om & below);
+  if (dense && dat < ntl) gst(P.order + dat, t);  // (counts that were not zero must not lead past the list)
+  if (other && oat < ntl) gst(P.order + ntl - 1u - oat, t);
 }
 
 __global__ __launch_bounds__(256) void k_bin_bits(const MipScene* __restrict__ scenes) {

@@ -253,6 +253,7 @@ struct MipBatch {
   bool vis;                // and k_visibility has answered the walks (else the injecting launch walks)
   // an ordered build's injecting launch (one scene): block b takes the listed tile b; the
   // list's two counts (dense and other tiles), and the next build's pair, which it zeroes
+  // (null in a captured build, which clears its own before k_tiles)
   uint32_t* counts;
   uint32_t* clear_counts;
 };
