@@ -108,7 +108,7 @@ struct Slot {
   uint8_t* h = nullptr;
   uint8_t* d = nullptr;
   size_t cap = 0;
-  uint32_t* flags = nullptr;  // pinned, kStageBlocks words
+  uint32_t* flags = nullptr;  // kStageBlocks words behind the host half
   uint32_t blocks = 0;        // workgroups of the copy last enqueued
   uint64_t gen = 0;           // changes whenever the slot is taken for new contents
 };
@@ -181,6 +181,11 @@ struct vgi_workspace {
   size_t sort_tmp_bytes = 0;
   void* vis = nullptr;        // mip builds with shadow-casting lights: vis bytes (MipScene)
   size_t vis_bytes = 0;
+  // the descriptor tables of calls recorded in graphs, and the smaller blocks it replaced,
+  // to which recorded graphs still write
+  void* recorded = nullptr;
+  size_t recorded_bytes = 0, replaced_bytes = 0;
+  std::vector<void*> replaced;
   // pinned: the last call's batch pairs, work units, large triangles and split bins, then
   // its call number, which the settle step stores once the four totals are complete
   unsigned long long* hist = nullptr;
@@ -191,7 +196,7 @@ struct vgi_workspace {
   size_t device_bytes() const {
     size_t b = tris_bytes + tritex_bytes + tri_slot_bytes + big_list_bytes + zeroed_bytes + zero_list_bytes +
                scan_bytes + work_bytes + pairs_bytes + scan_tmp_bytes + sort_keys_bytes + sort_pix_bytes +
-               sort_tmp_bytes + vis_bytes;
+               sort_tmp_bytes + vis_bytes + recorded_bytes + replaced_bytes;
     for (const Slot& s : slot) b += s.cap;
     return b;
   }
@@ -271,13 +276,13 @@ size_t scene_device_bytes(const vgi_scene* s) {
 void free_workspace(vgi_workspace* w) {
   void* dev[] = {w->tris,     w->tritex,   w->tri_slot, w->big_list, w->zeroed,    w->zero_list, w->scan_all,
                  w->work_map, w->pairs,    w->scan_tmp, w->sort_keys, w->sort_pix, w->sort_tmp,
-                 w->vis};
+                 w->vis,      w->recorded};
   for (void* p : dev)
     if (p) (void)hipFree(p);
+  for (void* p : w->replaced) (void)hipFree(p);
   for (Slot& s : w->slot) {
     if (s.d) (void)hipFree(s.d);
     if (s.h) (void)hipHostFree(s.h);
-    if (s.flags) (void)hipHostFree(s.flags);
   }
   if (w->hist) (void)hipHostFree(w->hist);
 }
@@ -291,15 +296,6 @@ vgi_workspace* workspace(vgi_context* ctx, hipStream_t st) {
   if (it != ctx->ws.end()) return it->second.get();
   auto w = std::make_unique<vgi_workspace>();
   w->stream = st;
-  for (Slot& s : w->slot)
-    if (hipHostMalloc((void**)&s.flags, kStageBlocks * sizeof(uint32_t), hipHostMallocCoherent) != hipSuccess) {
-      (void)hipGetLastError();
-      s.flags = nullptr;
-      free_workspace(w.get());
-      return nullptr;
-    } else {
-      std::memset(s.flags, 0, kStageBlocks * sizeof(uint32_t));
-    }
   vgi_workspace* raw = w.get();
   ctx->ws.emplace(st, std::move(w));
   return raw;
@@ -325,8 +321,8 @@ bool slot_read(const Slot& s) {
   return true;
 }
 
-// Waits until it has. The stream is asked now and then, so that a wait ends with an error
-// where the copy can no longer run (and never outlasts the stream's work).
+// Waits until it has. The stream is asked now and then: one that has run all its work holds
+// no copy that could still read.
 int wait_slot(vgi_workspace* w, const Slot& s) {
   for (uint32_t spin = 1; !slot_read(s); spin++) {
     if (spin % 1024u != 0u) {
@@ -336,7 +332,7 @@ int wait_slot(vgi_workspace* w, const Slot& s) {
     const hipError_t e = hipStreamQuery(w->stream);
     if (e == hipErrorNotReady) continue;
     HIP_TRY(e);
-    if (!slot_read(s)) return fail(VGI_E_HIP, "a descriptor copy did not run");
+    break;
   }
   return VGI_OK;
 }
@@ -354,13 +350,16 @@ int acquire_slot(vgi_workspace* w, size_t bytes, Slot** out) {
     if (s.h) (void)hipHostFree(s.h);
     s.d = nullptr;
     s.h = nullptr;
+    s.flags = nullptr;
     s.cap = 0;
     const size_t cap = std::max<size_t>(align_up(bytes + bytes / 2, 4096), 65536);
     if (hipMalloc((void**)&s.d, cap) != hipSuccess ||
-        hipHostMalloc((void**)&s.h, cap, hipHostMallocCoherent) != hipSuccess) {
+        hipHostMalloc((void**)&s.h, cap + kStageBlocks * sizeof(uint32_t), hipHostMallocCoherent) != hipSuccess) {
       (void)hipGetLastError();
       return fail(VGI_E_NOMEM, "staging allocation of %zu bytes failed", cap);
     }
+    s.flags = (uint32_t*)(s.h + cap);
+    std::memset(s.flags, 0, kStageBlocks * sizeof(uint32_t));
     s.cap = cap;
   }
   *out = &s;
@@ -379,6 +378,30 @@ StageArgs stage_args(const Slot& s, size_t bytes) {
   return a;
 }
 
+// Room for `bytes` bytes of recorded descriptors. It may have to grow while the stream is
+// captured, which forbids an allocation unless this thread's capture mode is relaxed. A block
+// that earlier graphs write to stays until the workspace goes; each is twice the one before.
+int recorded_room(vgi_workspace* w, size_t bytes) {
+  if (w->recorded_bytes >= bytes) return VGI_OK;
+  const size_t cap = std::max<size_t>(std::max(align_up(bytes, 4096), 2 * w->recorded_bytes), 65536);
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+  void* p = nullptr;
+  const hipError_t e = hipMalloc(&p, cap);
+  HIP_TRY(hipThreadExchangeStreamCaptureMode(&mode));
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    return fail(VGI_E_NOMEM, "staging allocation of %zu bytes failed", cap);
+  }
+  if (w->recorded) {
+    w->replaced.push_back(w->recorded);
+    w->replaced_bytes += w->recorded_bytes;
+  }
+  w->recorded = p;
+  w->recorded_bytes = cap;
+  return VGI_OK;
+}
+
 // A call's descriptor tables: fill(h, d) writes them into host memory h for a device copy
 // at d (tables may point into themselves). If the site's last copy is still held (its slot
 // not taken since) and the new bytes equal it, that device copy is used as it is and nothing
@@ -386,17 +409,30 @@ StageArgs stage_args(const Slot& s, size_t bytes) {
 // Otherwise a slot is taken and launch(args) enqueues the kernel that copies it. Equal bytes
 // mean the device already holds exactly what the copy would write, so reuse cannot change
 // results. launch is called either way, with no blocks where nothing is to be copied.
+//
+// A call recorded in a graph takes no slot: the graph may never run, or run when the slot has
+// other contents. Its tables go into the graph, as the arguments of the kernels that write
+// them to the stream's recorded block each time it runs, so that graphs recorded on one stream
+// share that block (their runs have to be ordered) and none outlives its tables.
 template <class F, class L>
-int stage_descriptors(vgi_workspace* w, UploadSite site, size_t bytes, F&& fill, L&& launch, Slot** out) {
+int stage_descriptors(vgi_workspace* w, UploadSite site, size_t bytes, F&& fill, L&& launch) {
+  bool captured = false;
+  TRY(stream_capturing(w->stream, &captured));
+  if (captured) {
+    TRY(recorded_room(w, bytes));
+    Slot s;
+    s.d = (uint8_t*)w->recorded;
+    w->staging.assign(bytes, 0);
+    fill(w->staging.data(), s.d);
+    HIP_TRY(launch_stage_values(s.d, w->staging.data(), bytes, w->stream));
+    return launch(s, StageArgs{});
+  }
   UploadCache& c = w->cache[site];
   if (c.slot >= 0 && c.bytes == bytes && w->slot[c.slot].gen == c.gen) {
     Slot& s = w->slot[c.slot];
     w->staging.assign(bytes, 0);
     fill(w->staging.data(), s.d);
-    if (std::memcmp(w->staging.data(), s.h, bytes) == 0) {
-      *out = &s;
-      return launch(s, StageArgs{});
-    }
+    if (std::memcmp(w->staging.data(), s.h, bytes) == 0) return launch(s, StageArgs{});
   }
   Slot* sl = nullptr;
   TRY(acquire_slot(w, bytes, &sl));
@@ -411,7 +447,6 @@ int stage_descriptors(vgi_workspace* w, UploadSite site, size_t bytes, F&& fill,
   c.slot = (int)(sl - w->slot);
   c.gen = sl->gen;
   c.bytes = bytes;
-  *out = sl;
   return VGI_OK;
 }
 
@@ -795,8 +830,7 @@ int voxelize_batch(vgi_context* ctx, const vgi_voxelize_item* items, uint32_t co
     return launch_voxelize_kernels(ctx, B, stage, zb, zeroed_need, nblk_t, nblk_b, ts, grid_blocks, big_blocks,
                                    zero_blocks, scs.data(), count, st, ctx->profiling != 0);
   };
-  Slot* sl = nullptr;
-  TRY(stage_descriptors(w, kSiteVoxelize, cv.off, fill, launch, &sl));
+  TRY(stage_descriptors(w, kSiteVoxelize, cv.off, fill, launch));
   for (uint32_t i = 0; i < count; i++) {
     vgi_scene* s = plan[i].s;
     s->grid = items[i].grid;
@@ -1055,8 +1089,7 @@ int mips_batch(vgi_context* ctx, const vgi_mips_item* items, uint32_t count, uin
     }
     return VGI_OK;
   };
-  Slot* sl = nullptr;
-  TRY(stage_descriptors(w, kSiteMips, cv.off, fill, launch, &sl));
+  TRY(stage_descriptors(w, kSiteMips, cv.off, fill, launch));
   for (uint32_t i = 0; i < count; i++) {
     items[i].scene->prec = precision;
     items[i].scene->has_mips = true;
@@ -1315,7 +1348,6 @@ int trace_batch(vgi_context* ctx, const vgi_trace_item* items, uint32_t count, v
     TRY(grow_bytes(&w->sort_pix, &w->sort_pix_bytes, max_entries * 8, "sort pixels"));
     TRY(grow_bytes(&w->sort_tmp, &w->sort_tmp_bytes, std::max<size_t>(tmp_need, 1), "sort scratch"));
   }
-  Slot* sl = nullptr;
   auto fill = [&](uint8_t* h, const uint8_t* d) {
   for (const Launch& L : launches) {
     TraceParams* hp = (TraceParams*)(h + L.o_params);
@@ -1389,7 +1421,7 @@ int trace_batch(vgi_context* ctx, const vgi_trace_item* items, uint32_t count, v
     }
     return VGI_OK;
   };
-  TRY(stage_descriptors(w, kSiteTrace, cv.off, fill, launch, &sl));
+  TRY(stage_descriptors(w, kSiteTrace, cv.off, fill, launch));
   return VGI_OK;
 }
 

@@ -460,6 +460,8 @@ int check_request_input(const vgi_mesh* meshes, uint32_t num_meshes, const vgi_g
 // ---- launchers (each returns hipError_t) ----
 hipError_t launch_fill_u32(uint32_t* p, uint32_t value, size_t count, hipStream_t s);
 hipError_t launch_stage(const StageArgs& a, hipStream_t s);
+// Kernels that store `bytes` bytes at src, as they are now, to dst (16-byte words, the last padded).
+hipError_t launch_stage_values(void* dst, const void* src, size_t bytes, hipStream_t s);
 // Zeroes `words` words at zb and copies a call's descriptor tables, in one launch.
 hipError_t launch_begin(const StageArgs& a, uint32_t* zb, size_t words, hipStream_t s);
 hipError_t launch_copy(void* dst, const void* src, size_t bytes, hipStream_t s);

@@ -52,6 +52,7 @@
 // voxel set and the integer sums do not depend on order, rounding or thread mapping.
 #include <algorithm>
 #include <cstddef>
+#include <cstring>
 
 #include "vgi_internal.hpp"
 
@@ -82,6 +83,31 @@ __global__ __launch_bounds__(256) void k_stage(StageArgs a) { stage_block(a, blo
 hipError_t launch_stage(const StageArgs& a, hipStream_t s) {
   if (a.blocks == 0) return hipSuccess;
   hipLaunchKernelGGL(k_stage, dim3(a.blocks), dim3(256), 0, s, a);
+  return hipGetLastError();
+}
+
+// A recorded call's descriptor tables, a part of them in the arguments of each launch.
+constexpr uint32_t kValueQuads = 224;  // with the rest under the 4 KB that a launch's arguments may take
+struct StageValues {
+  uint4* dst;
+  uint32_t quads;
+  uint32_t pad;
+  uint4 v[kValueQuads];
+};
+__global__ __launch_bounds__(256) void k_stage_values(StageValues a) {
+  const uint32_t i = threadIdx.x;
+  if (i < a.quads) gst4(a.dst + i, a.v[i]);
+}
+
+hipError_t launch_stage_values(void* dst, const void* src, size_t bytes, hipStream_t s) {
+  for (size_t at = 0; at < bytes; at += sizeof(StageValues::v)) {
+    const size_t n = std::min(bytes - at, sizeof(StageValues::v));
+    StageValues a{};
+    a.dst = (uint4*)((uint8_t*)dst + at);
+    a.quads = (uint32_t)((n + 15) / 16);
+    std::memcpy(a.v, (const uint8_t*)src + at, n);
+    hipLaunchKernelGGL(k_stage_values, dim3(1), dim3(256), 0, s, a);
+  }
   return hipGetLastError();
 }
 

@@ -101,3 +101,86 @@ def test_recorded_mip_build_replays(ctx, n, levels):
     finally:
         sc.release()
         ctx.stream_destroy(stream)
+
+
+def _trace_setup(ctx, w, stream):
+    vgi = _vgi()
+    sc = ctx.scene()
+    mesh = vgi.MeshData(ctx, w.positions.reshape(-1, 3), albedo=w.albedo)
+    sc.voxelize([mesh], vgi.make_grid(**w.grid), stream)
+    sc.build_mips(vgi.make_lights(w.lights), vgi.PREC_FP32, stream)
+    gb = vgi.GBufferData(ctx, w.gb_pos, w.gb_nrm, w.width, w.height, w.gb_rough)
+    out = [vgi.DeviceArray.empty(ctx, (w.num_pixels, 4), np.float32) for _ in range(2)]
+    ctx.sync(stream)
+    return sc, gb, out, mesh
+
+
+def test_recorded_traces_and_the_descriptor_ring(ctx):
+    """A recorded trace carries its own descriptors: eager calls with other ones, more of them
+    than the stream has staging slots, run before the graph's first run and between its runs, and
+    each kind leaves the other's results alone. A graph that never runs stops nothing. The eager
+    calls are what every replay is compared with."""
+    vgi = _vgi()
+    print("case recorded traces", flush=True)
+    w = sg.random_soup(ntri=2000, n=32, levels=5, width=48, height=40)
+    stream = ctx.stream_create()
+    sc, gb, out, mesh = _trace_setup(ctx, w, stream)
+    cones = [vgi.make_cones(**dict(w.cones, normal_offset=1.0 + 0.01 * i)) for i in range(30)]
+
+    def trace(i, batch=1):
+        ctx.trace_batch([(sc, gb, cones[i], out[0], out[1])] * batch, stream)
+
+    def read():
+        ctx.sync(stream)
+        return np.concatenate([o.numpy() for o in out], 1)
+
+    def fresh(run):
+        for o in out:
+            o.zero()
+        run()
+        return read()
+
+    try:
+        eager = [fresh(lambda: trace(i)) for i in range(30)]
+        assert len({e.tobytes() for e in eager}) == 30
+        never = Recorded(stream, lambda: trace(5))
+        g = [Recorded(stream, lambda: trace(i)) for i in (3, 11)]
+        big = Recorded(stream, lambda: trace(7, 64))  # its tables outgrow the block of those before
+        g.append(Recorded(stream, lambda: trace(23)))
+        for i in range(30):  # past every slot of the ring twice
+            assert np.array_equal(fresh(lambda: trace(i)), eager[i]), f"eager call {i} after the recording"
+        for rep in range(3):
+            for graph, i in zip(g + [big], (3, 11, 23, 7)):
+                assert np.array_equal(fresh(graph.replay), eager[i]), f"replay {rep} of call {i}"
+            for i in range(rep, 30, 2):
+                assert np.array_equal(fresh(lambda: trace(i)), eager[i]), f"eager call {i} after replay {rep}"
+        for graph in g + [big, never]:
+            graph.release()
+    finally:
+        sc.release()
+        ctx.stream_destroy(stream)
+
+
+def test_recorded_trace_on_a_fresh_stream(ctx):
+    """The first call that a stream sees may be a recorded one."""
+    print("case recorded trace, fresh stream", flush=True)
+    vgi = _vgi()
+    w = sg.random_soup(ntri=2000, n=32, levels=5, width=48, height=40)
+    sc, gb, out, mesh = _trace_setup(ctx, w, None)
+    cones = vgi.make_cones(**w.cones)
+    sc.trace(gb, cones, out[0], out[1])
+    ctx.sync()
+    want = [o.numpy() for o in out]
+    stream = ctx.stream_create()
+    try:
+        g = Recorded(stream, lambda: sc.trace(gb, cones, out[0], out[1], stream))
+        for _ in range(3):
+            for o in out:
+                o.zero()
+            g.replay()
+            ctx.sync(stream)
+            assert all(np.array_equal(o.numpy(), v) for o, v in zip(out, want))
+        g.release()
+    finally:
+        sc.release()
+        ctx.stream_destroy(stream)
