@@ -950,8 +950,8 @@ int mips_batch(vgi_context* ctx, const vgi_mips_item* items, uint32_t count, uin
   size_t total_lights = 0;
   // Builds with shadow-casting lights: where every scene has at most 32 and there is memory
   // for an answer byte a voxel per eight of them, k_visibility walks before the injecting
-  // launch; otherwise (or when that memory is missing under stream capture) that launch walks
-  // by itself.
+  // launch; otherwise that launch walks by itself. So it does in a build recorded in a graph,
+  // which may run when a larger build has replaced the stream's answer bytes.
   bool shadow = false, vis = true;
   size_t vis_need = 0;
   std::vector<size_t> vis_off(count);
@@ -968,13 +968,12 @@ int mips_batch(vgi_context* ctx, const vgi_mips_item* items, uint32_t count, uin
     vis_off[i] = vis_need;
     vis_need += align_up(n * n * n * ((ns + 7) / 8), 256) + (ns ? align_up(n * n * n / kVisVoxels * sizeof(uint32_t), 256) : 0);
   }
-  vis = vis && shadow;
   bool captured = false;
   TRY(stream_capturing(st, &captured));
+  vis = vis && shadow && !captured;
   if (vis && w->vis_bytes < vis_need) {
-    vis = !captured;
-    if (vis) HIP_TRY(hipStreamSynchronize(st));
-    vis = vis && grow_bytes(&w->vis, &w->vis_bytes, vis_need, "visibility") == VGI_OK;
+    HIP_TRY(hipStreamSynchronize(st));
+    vis = grow_bytes(&w->vis, &w->vis_bytes, vis_need, "visibility") == VGI_OK;
   }
   Carve cv;
   const size_t o_scenes = cv.take((size_t)count * sizeof(MipScene));

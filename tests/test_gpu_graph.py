@@ -184,3 +184,39 @@ def test_recorded_trace_on_a_fresh_stream(ctx):
     finally:
         sc.release()
         ctx.stream_destroy(stream)
+
+
+def test_recorded_build_with_shadow_lights(ctx):
+    """A recorded build with shadow-casting lights holds nothing of the stream's scratch: an
+    eager build of a larger grid replaces that scratch between the replays."""
+    vgi = _vgi()
+    print("case recorded mips with shadow-casting lights", flush=True)
+    small, large = (sg.room(ntri=3000, n=n, levels=5, width=32, height=18) for n in (32, 128))
+    lights = [dict(l, shadow=True) for l in small.lights]
+    ref = orc.inject_mips(orc.voxelize(small.positions, small.grid, albedo=small.albedo)[0], small.grid, lights, "fp32")
+    stream, scs = ctx.stream_create(), [ctx.scene(), ctx.scene()]
+    try:
+        meshes = [vgi.MeshData(ctx, w.positions.reshape(-1, 3), albedo=w.albedo) for w in (small, large)]
+        for sc, m, w in zip(scs, meshes, (small, large)):
+            sc.voxelize([m], vgi.make_grid(**w.grid), stream)
+
+        def build():
+            scs[0].build_mips(vgi.make_lights(lights), vgi.PREC_FP32, stream)
+
+        build()
+        g = Recorded(stream, build)
+        g.replay()
+        ctx.sync(stream)
+        _assert_levels(scs[0], ref, "replay")
+        before = ctx.workspace_bytes()
+        scs[1].build_mips(vgi.make_lights(lights), vgi.PREC_FP32, stream)
+        assert ctx.workspace_bytes() > before
+        for what, run in (("replay", g.replay), ("replay", g.replay), ("eager", build)):
+            run()
+            ctx.sync(stream)
+            _assert_levels(scs[0], ref, f"{what} after a larger build")
+        g.release()
+    finally:
+        for sc in scs:
+            sc.release()
+        ctx.stream_destroy(stream)
