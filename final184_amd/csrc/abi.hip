@@ -1278,7 +1278,12 @@ int trace_batch(vgi_context* ctx, const vgi_trace_item* items, uint32_t count, v
   if (!items) return fail(VGI_E_INVALID, "items is NULL");
   for (uint32_t i = 0; i < count; i++) TRY(check_trace_item(ctx, items[i], i));
   const vgi_tuning tn = tuning_of(ctx);
-  const bool morton = tn.pixel_order == VGI_ORDER_MORTON;
+  const hipStream_t st = pick(ctx, stream);
+  bool captured = false;
+  TRY(stream_capturing(st, &captured));
+  // A recorded call traces in tile order, with the same results: the sort's scratch may be
+  // replaced before the graph runs, and its library records memory-set nodes.
+  const bool morton = tn.pixel_order == VGI_ORDER_MORTON && !captured;
   // one launch per storage precision
   constexpr uint32_t kPrecisions = VGI_PREC_FP16X2 + 1;
   std::vector<uint32_t> group[kPrecisions];
@@ -1335,7 +1340,6 @@ int trace_batch(vgi_context* ctx, const vgi_trace_item* items, uint32_t count, v
     launches.push_back(L);
   }
   HIP_TRY(hipSetDevice(ctx->device));
-  const hipStream_t st = pick(ctx, stream);
   vgi_workspace* w = workspace(ctx, st);
   if (!w) return fail(VGI_E_HIP, "workspace creation failed");
   std::lock_guard<std::mutex> wl(w->mu);

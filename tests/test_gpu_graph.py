@@ -220,3 +220,39 @@ def test_recorded_build_with_shadow_lights(ctx):
         for sc in scs:
             sc.release()
         ctx.stream_destroy(stream)
+
+
+def test_recorded_trace_in_morton_order(ctx):
+    """A recorded call of a stream tuned to Morton order holds none of the sort's scratch, which
+    an eager call over more pixels replaces between the replays; the pixels' results are those
+    of either order."""
+    print("case recorded trace, Morton order", flush=True)
+    vgi = _vgi()
+    w = sg.random_soup(ntri=2000, n=32, levels=5, width=70, height=40)
+    stream = ctx.stream_create()
+    sc, gb, out, mesh = _trace_setup(ctx, w, stream)
+    cones = vgi.make_cones(**w.cones)
+    try:
+        ctx.set_tuning(pixel_order=vgi.ORDER_MORTON)
+
+        def trace(n=1):
+            ctx.trace_batch([(sc, gb, cones, out[0], out[1])] * n, stream)
+
+        trace()
+        ctx.sync(stream)
+        want = [o.numpy() for o in out]
+        g = Recorded(stream, trace)
+        for n in (0, 0, 8, 64, 0):
+            if n:
+                trace(n)
+                ctx.sync(stream)
+            for o in out:
+                o.zero()
+            g.replay()
+            ctx.sync(stream)
+            assert all(np.array_equal(o.numpy(), v) for o, v in zip(out, want)), f"replay after a batch of {n}"
+        g.release()
+    finally:
+        ctx.set_tuning()
+        sc.release()
+        ctx.stream_destroy(stream)
