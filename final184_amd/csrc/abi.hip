@@ -33,6 +33,7 @@
 #include <vector>
 
 #include "gltf.hpp"
+#include "scratch.hpp"
 #include "vgi_internal.hpp"
 
 using namespace vgi;
@@ -66,6 +67,10 @@ int fail(int code, const char* fmt, ...) {
   } while (0)
 
 bool is_pow2(uint32_t v) { return v && !(v & (v - 1)); }
+// Most answer bytes of visibility walks that a stream keeps: one scene of 512^3 with up to 16
+// shadow-casting lights (285 MB), or nine of 256^3 with 16.
+constexpr size_t kMaxVisBytes = 320u << 20;
+
 // A scene's mip tile state (vgi_scene::live): ten words per 16^3 tile, 64 of counts, and a bit
 // per bin of 8^3 voxels.
 uint64_t tile_state_bytes(uint64_t n) {
@@ -179,8 +184,7 @@ struct vgi_workspace {
   size_t sort_pix_bytes = 0;
   void* sort_tmp = nullptr;
   size_t sort_tmp_bytes = 0;
-  void* vis = nullptr;        // mip builds with shadow-casting lights: vis bytes (MipScene)
-  size_t vis_bytes = 0;
+  OptionalScratch vis{kMaxVisBytes};  // mip builds with shadow-casting lights: vis bytes (MipScene)
   // the descriptor tables of calls recorded in graphs, and the smaller blocks it replaced,
   // to which recorded graphs still write
   void* recorded = nullptr;
@@ -196,7 +200,7 @@ struct vgi_workspace {
   size_t device_bytes() const {
     size_t b = tris_bytes + tritex_bytes + tri_slot_bytes + big_list_bytes + zeroed_bytes + zero_list_bytes +
                scan_bytes + work_bytes + pairs_bytes + scan_tmp_bytes + sort_keys_bytes + sort_pix_bytes +
-               sort_tmp_bytes + vis_bytes + recorded_bytes + replaced_bytes;
+               sort_tmp_bytes + vis.bytes() + recorded_bytes + replaced_bytes;
     for (const Slot& s : slot) b += s.cap;
     return b;
   }
@@ -276,7 +280,7 @@ size_t scene_device_bytes(const vgi_scene* s) {
 void free_workspace(vgi_workspace* w) {
   void* dev[] = {w->tris,     w->tritex,   w->tri_slot, w->big_list, w->zeroed,    w->zero_list, w->scan_all,
                  w->work_map, w->pairs,    w->scan_tmp, w->sort_keys, w->sort_pix, w->sort_tmp,
-                 w->vis,      w->recorded};
+                 w->vis.data(), w->recorded};
   for (void* p : dev)
     if (p) (void)hipFree(p);
   for (void* p : w->replaced) (void)hipFree(p);
@@ -948,9 +952,9 @@ int mips_batch(vgi_context* ctx, const vgi_mips_item* items, uint32_t count, uin
   size_t nblocks = 0;
   for (const auto& v : stages) nblocks += v.size();
   size_t total_lights = 0;
-  // Builds with shadow-casting lights: where every scene has at most 32 and there is memory
-  // for an answer byte a voxel per eight of them, k_visibility walks before the injecting
-  // launch; otherwise that launch walks by itself. So it does in a build recorded in a graph,
+  // Builds with shadow-casting lights: where every scene has at most 32 and the stream holds
+  // or can get an answer byte a voxel per eight of them, up to kMaxVisBytes, k_visibility walks
+  // before the injecting launch; otherwise that launch walks by itself. So it does in a build recorded in a graph,
   // which may run when a larger build has replaced the stream's answer bytes.
   bool shadow = false, vis = true;
   size_t vis_need = 0;
@@ -971,10 +975,15 @@ int mips_batch(vgi_context* ctx, const vgi_mips_item* items, uint32_t count, uin
   bool captured = false;
   TRY(stream_capturing(st, &captured));
   vis = vis && shadow && !captured;
-  if (vis && w->vis_bytes < vis_need) {
-    HIP_TRY(hipStreamSynchronize(st));
-    vis = grow_bytes(&w->vis, &w->vis_bytes, vis_need, "visibility") == VGI_OK;
-  }
+  vis = vis && w->vis.reserve(
+                   vis_need,
+                   [](size_t bytes) {
+                     void* p = nullptr;
+                     if (hipMalloc(&p, bytes) == hipSuccess) return p;
+                     (void)hipGetLastError();
+                     return (void*)nullptr;
+                   },
+                   [st] { return hipStreamSynchronize(st) == hipSuccess; }, [](void* p) { (void)hipFree(p); });
   Carve cv;
   const size_t o_scenes = cv.take((size_t)count * sizeof(MipScene));
   const size_t o_blocks = cv.take(table ? nblocks * sizeof(MipBlock) : 0);
@@ -1017,7 +1026,7 @@ int mips_batch(vgi_context* ctx, const vgi_mips_item* items, uint32_t count, uin
       if (D.shadow) D.shadow = ++ns;
     }
     lbase += P.nlights;
-    P.vis = vis && ns ? (uint8_t*)w->vis + vis_off[i] : nullptr;
+    P.vis = vis && ns ? (uint8_t*)w->vis.data() + vis_off[i] : nullptr;
     P.vis_planes = P.vis ? (ns + 7) / 8 : 0;
     const size_t n3 = (size_t)g.n * g.n * g.n;
     P.vis_units = P.vis ? (uint32_t*)(P.vis + align_up(n3 * P.vis_planes, 256)) : nullptr;

@@ -276,7 +276,8 @@ int vgi_scene_get_stats(const vgi_scene* scene, vgi_scene_stats* out);
 /* Device bytes a scene of this grid and precision holds while resident: accumulator,
  * occupancy mask, bin table and mip levels (admission control). The voxelize scratch
  * (about 112 bytes per triangle, 4 per bin pair and 44 per bin) belongs to the stream
- * the call runs on and is reported by vgi_workspace_bytes. num_triangles is unused. */
+ * the call runs on and is reported by vgi_workspace_bytes, as is what a build with
+ * shadow-casting lights takes (vgi_build_mips). num_triangles is unused. */
 uint64_t vgi_scene_bytes_estimate(const vgi_grid* grid, uint32_t precision, uint64_t num_triangles);
 
 /* Clear + voxelize all meshes into the scene's accumulator (one frame's voxelize pass).
@@ -314,7 +315,10 @@ int vgi_voxelize_noalloc(vgi_context* ctx, vgi_scene* scene, const vgi_mesh* mes
                          const vgi_grid* grid, void* stream);
 
 /* Inject direct light into level 0 and build the 2x2x2 box mip chain in the given
- * precision. No reference code (planned in docs/index.md:36). */
+ * precision. No reference code (planned in docs/index.md:36). With shadow-casting lights the
+ * stream keeps up to 320 MiB of scratch for the visibility walks' answers (a byte a voxel per
+ * eight of them and n^3 / 8 bytes, summed over a batch; reported by vgi_workspace_bytes);
+ * without it, as in calls that need more, the levels are the same and take longer. */
 int vgi_build_mips(vgi_context* ctx, vgi_scene* scene, const vgi_lights* lights,
                    uint32_t precision, void* stream);
 

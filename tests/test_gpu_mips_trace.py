@@ -562,6 +562,37 @@ def test_shadow_walks_at_512(ctx):
         sc.release()
 
 
+def test_shadow_walks_beyond_the_scratch_limit(ctx):
+    """Five scenes of 256^3 with 32 shadow-casting lights need 346 MB for their walks' answers,
+    more than a stream keeps: the batch's launch walks by itself, with the levels that one
+    scene gets from the answers, and no scratch is added."""
+    vgi = _vgi()
+    print("case shadow walks beyond the scratch limit", flush=True)
+    w = sg.room(ntri=10_000, n=256, levels=6, width=32, height=18)
+    base = _shadow_lights(w)
+    lights = vgi.make_lights([base[i % len(base)] for i in range(32)])
+    mesh = vgi.MeshData(ctx, w.positions.reshape(-1, 3), albedo=w.albedo)
+    stream, scs = ctx.stream_create(), [ctx.scene() for _ in range(5)]
+    try:
+        ctx.voxelize_batch([(sc, [mesh], vgi.make_grid(**w.grid)) for sc in scs], stream)
+        empty = ctx.workspace_bytes()
+        scs[0].build_mips(lights, vgi.PREC_FP16, stream)
+        one = ctx.workspace_bytes()
+        assert one - empty >= 4 * 256 ** 3
+        ctx.sync(stream)
+        want = [scs[0].read_level(k) for k in (1, 3, 5)]
+        for _ in range(2):
+            ctx.build_mips_batch([(sc, lights) for sc in scs], vgi.PREC_FP16, stream)
+            ctx.sync(stream)
+            assert ctx.workspace_bytes() - one < 1 << 22  # (the batch's tables)
+            for sc in scs:
+                assert all(np.array_equal(sc.read_level(k), v) for k, v in zip((1, 3, 5), want))
+    finally:
+        for sc in scs:
+            sc.release()
+        ctx.stream_destroy(stream)
+
+
 def test_shadowed_and_plain_scenes_in_one_batch(ctx, soup):
     """One mip batch with a shadowed-light scene and a plain-light scene: the launch walks for
     the batch, and each scene still equals the oracle under its own lights."""
