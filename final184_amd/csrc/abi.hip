@@ -822,8 +822,7 @@ int voxelize_batch(vgi_context* ctx, const vgi_voxelize_item* items, uint32_t co
   // voxelize work units (one per workgroup), large triangles (4 per workgroup, one per
   // wavefront) and split bins (one per workgroup); kernels loop over any excess
   const uint64_t cus = (uint64_t)ctx->num_cus;
-  const uint64_t grid_want = w->hist_units ? w->hist_units + w->hist_units / 8 + 64 : cus * 8;
-  const uint32_t grid_blocks = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(grid_want, work_cap));
+  const uint32_t grid_blocks = voxelize_workgroups(w->hist_units, work_cap, cus);
   const uint32_t big_blocks =
       (uint32_t)std::min<uint64_t>(cus * 4, w->hist_big ? (w->hist_big + w->hist_big / 4 + 3) / 4 + 1 : cus);
   const uint32_t zero_blocks = (uint32_t)std::min<uint64_t>(
@@ -1781,8 +1780,8 @@ int vgi_voxelize_noalloc(vgi_context* ctx, vgi_scene* sc, const vgi_mesh* meshes
   B.nscenes = 1;
   B.total_bins = (uint32_t)nbins;
   B.textured = textured ? 1u : 0u;
-  const uint32_t grid_blocks = (uint32_t)std::min<uint64_t>((uint64_t)ctx->num_cus * 8, work_cap64);
   const uint32_t cus = (uint32_t)ctx->num_cus;
+  const uint32_t grid_blocks = voxelize_workgroups(0, work_cap64, cus);
   TRY(launch_voxelize_kernels(ctx, B, StageArgs{}, zb, zeroed_bytes, ceil_div(ntri, kBlockTris),
                               ceil_div(nbins, kBlockBins), ts, grid_blocks, cus,
                               (uint32_t)std::min<uint64_t>(cus / 4, nbins), &sc, 1, st, false));

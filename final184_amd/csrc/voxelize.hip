@@ -1094,13 +1094,26 @@ __device__ __forceinline__ bool tex_albedo(const TexCoef& T, int64_t e0, int64_t
   return true;
 }
 
+// UNIFORM: t is the wavefront's, and its records come through the scalar cache.
+template <bool UNIFORM>
 __device__ __forceinline__ void load_texcoef(const VoxScene& P, uint32_t t, TexCoef& C) {
-  const TriTex X = gld_rec(P.tritex + t);
+  TriTex X;
+  if constexpr (UNIFORM) X = sld_rec(P.tritex + t);
+  else X = gld_rec(P.tritex + t);
   C.textured = X.textured;
   if (!X.textured) return;
 #pragma unroll
   for (int i = 0; i < 6; i++) C.uv[i] = X.uv[i];
   const MeshDev* M = P.meshes + X.mesh;
+  if constexpr (UNIFORM) {
+    const MeshDev D = sld_rec(M);
+    C.tex = D.tex;
+    C.tw = D.tw;
+    C.th = D.th;
+#pragma unroll
+    for (int i = 0; i < 4; i++) C.factor[i] = D.factor[i];
+    return;
+  }
   C.tex = (const uint32_t*)gld((const unsigned long long*)&M->tex);
   C.tw = gld(&M->tw);
   C.th = gld(&M->th);
@@ -1293,25 +1306,35 @@ struct TileLayout {
 // four 64-bit atomics (exact with fewer than 2^21 triangles per voxel: no 32-bit word's total
 // reaches 2^32), and set the voxel's occupancy bit. Integer sums do not depend on order, so
 // the accumulator is the same as the binned path's.
+//
+// The wavefront's triangle stays in scalar registers, its edges are formed from it for every
+// 64 voxels: 4000 grid-wide triangles at 256^3, bound by their atomics (about 32 G/s), 20.2 ms;
+// 22.0 with a copy in every lane, which at k_voxelize's registers spills; 19.4 in a launch of
+// its own, and with the edges kept in scalar registers, which then spill into the binned path's
+// (16 soups 387 -> 407 us).
 template <bool TEX>
 __device__ __forceinline__ void fallback_pass(const VoxBatch& B, const VoxScene* __restrict__ scenes, uint32_t nwg) {
   const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t wave = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6), nwaves = nwg * (blockDim.x >> 6);
+  const uint32_t wave = blockIdx.x * (blockDim.x >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t nwaves = nwg * (blockDim.x >> 6);
   for (uint32_t sc = 0; sc < B.nscenes; sc++) {
     const VoxScene& P = scenes[sc];
     const uint32_t nbr = P.n >> 3;
     for (uint32_t t = wave; t < P.ntri; t += nwaves) {
-      const TriRec R = gld_rec(P.tris + t);
+      const TriRec R = sld_rec(P.tris + t);  // the wavefront's: it and what follows from it stay scalar
       if (!tri_ok(R)) continue;
-      int64_t q[3][3], N[3];
-      load_q(R, q, N);
+      int64_t N[3];
+      {
+        int64_t q[3][3];
+        load_q(R, q, N);
+      }
       const int nx = R.hi[0] - R.lo[0] + 1, ny = R.hi[1] - R.lo[1] + 1, nz = R.hi[2] - R.lo[2] + 1;
       const uint32_t r = R.rgb & 0xFFu, g = (R.rgb >> 8) & 0xFFu, b = (R.rgb >> 16) & 0xFFu;
       unsigned long long i0 = (unsigned long long)r | ((unsigned long long)g << 32);
       unsigned long long i1 = (unsigned long long)b | (1ull << 32);
       TexCoef X;
       X.textured = 0;
-      if constexpr (TEX) load_texcoef(P, t, X);
+      if constexpr (TEX) load_texcoef<true>(P, t, X);
       const unsigned long long i2 = (unsigned long long)(uint32_t)(R.nq[0] + kNormalBias) |
                                     ((unsigned long long)(uint32_t)(R.nq[1] + kNormalBias) << 32);
       const unsigned long long i3 = (unsigned long long)(uint32_t)(R.nq[2] + kNormalBias);
@@ -1320,6 +1343,13 @@ __device__ __forceinline__ void fallback_pass(const VoxBatch& B, const VoxScene*
         const int x = R.lo[0] + (int)(j % (uint32_t)nx), y = R.lo[1] + (int)((j / (uint32_t)nx) % (uint32_t)ny),
                   z = R.lo[2] + (int)(j / ((uint32_t)nx * (uint32_t)ny));
         const int32_t bb[3] = {x << VGI_FIXED_BITS, y << VGI_FIXED_BITS, z << VGI_FIXED_BITS};
+        int64_t q[3][3];
+#pragma unroll
+        for (int i = 0; i < 9; i++) {  // (the edges anew each time: kept, they would take more scalar registers than there are)
+          int32_t v = R.q[i];
+          asm volatile("" : "+s"(v));
+          q[i / 3][i % 3] = v;
+        }
         if (!sat_box(q, N, bb, VGI_FIXED_BITS)) continue;
         if constexpr (TEX) {
           if (X.textured) {
@@ -1351,11 +1381,10 @@ __device__ __forceinline__ void load_unit(const VoxBatch& B, uint32_t w, uint32_
 }
 
 // Registers: the 8^3 tile's unit accumulators (14 per thread) are held at 6 waves per SIMD
-// (80 VGPRs; 6 resident workgroups per CU, as many as LDS allows at 25.5 KB each), which
-// keeps the binned path in registers (only the fallback pass spills: as a launch of its own
-// it cost every call about 3 us to find nothing to do). The kernel is
-// latency-bound (dependent loads and barriers per chunk), so resident workgroups count:
-// 6 instead of 5 took the room's launch from 80 to 75 us.
+// (80 VGPRs; 6 resident workgroups per CU, as many as LDS allows at 25.5 KB each), the fallback
+// pass within them (as a launch of its own it cost every call about 3 us to find nothing to
+// do). The kernel is latency-bound (dependent loads and barriers per chunk), so resident
+// workgroups count: 6 instead of 5 took the room's launch from 80 to 75 us.
 // TEX: the batch has a textured mesh; each triangle's texture inputs sit beside its
 // coefficients and a textured triangle samples its albedo per column (kept apart so that
 // untextured batches run the kernel without the sampler's registers and LDS).
@@ -1417,12 +1446,15 @@ void k_voxelize(VoxBatch Bt, const VoxScene* __restrict__ scenes) {
     for (uint32_t at = 0; at < npairs; at += P.chunk) {
       const uint32_t first = base + at;
       const uint32_t cnt = min(P.chunk, npairs - at);
-      if ((tid & 63u) < cnt) {  // triangle tid % 64, coefficient part tid / 64
-        const uint32_t t = gld(Bt.pairs_all + first + (tid & 63u));
+      uint32_t v = tid;  // (hidden: else its addresses are kept across the chunks, and a sum is spilled for them)
+      asm volatile("" : "+v"(v));
+      const uint32_t q = v & 63u;
+      if (q < cnt) {  // triangle tid % 64, coefficient part tid / 64
+        const uint32_t t = gld(Bt.pairs_all + first + q);
         const TriRec R = gld_rec(P.tris + t);
-        make_coef(R, s_tri[tid & 63u], tid >> 6);
+        make_coef(R, s_tri[q], v >> 6);
         if constexpr (TEX)
-          if ((tid >> 6) == 3u) load_texcoef(P, t, s_tex[tid & 63u]);
+          if ((v >> 6) == 3u) load_texcoef<false>(P, t, s_tex[q]);
       }
 
       for (uint32_t st = 0; st < sub * sub * sub; st++) {

@@ -37,6 +37,15 @@ int main() {
   CHECK(trace_wavefronts(1u << 24, 10, 9, true, VGI_PREC_FP16) == 3);
   CHECK(trace_wavefronts((1u << 26) - 1, 10, 9, true, VGI_PREC_FP16) == 1);
   CHECK(trace_wavefronts(0, 10, 9, false, VGI_PREC_FP32) >= 1);
+  // the overflow path, which runs on the same workgroups, has at least one a CU
+  for (uint64_t seen : {0ull, 1ull, 8ull, 100ull, 171ull, 172ull, 5000ull, 1ull << 30})
+    for (uint64_t cap : {1ull, 65ull, 1100ull, 1ull << 31}) {
+      const uint32_t g = voxelize_workgroups(seen, cap, 256);
+      CHECK(g >= 256);
+      CHECK(g <= 256 || g <= cap);
+      if (seen && seen <= cap) CHECK(g >= seen);
+    }
+  CHECK(voxelize_workgroups(0, 1ull << 20, 256) == 2048 && voxelize_workgroups(800, 1ull << 20, 256) == 964);
   std::printf("LAUNCH RULES OK\n");
   return 0;
 }

@@ -268,6 +268,42 @@ def test_pair_overflow_takes_exact_fallback(ctx):
         ctx.stream_destroy(st_b)
 
 
+@pytest.mark.parametrize("textured", [False, True])
+def test_pair_overflow_after_small_scenes(ctx, textured):
+    """The overflow path runs on workgroups counted from the stream's earlier calls: after
+    scenes of a few work units it still covers every triangle of the one call that overflows."""
+    vgi = _vgi()
+    print(f"case pair-list overflow after small scenes, textured {textured}", flush=True)
+    n = 256
+    grid_d = dict(origin=(0.0, 0.0, 0.0), extent=1.0, n=n, levels=8)
+    grid = vgi.make_grid(**grid_d)
+    pos, alb = _planes(80, n, 5)
+    small = sg.random_soup(ntri=12, n=n).positions
+    stream, sc = ctx.stream_create(), ctx.scene()
+    try:
+        ms = vgi.MeshData(ctx, small.reshape(-1, 3))
+        for _ in range(3):
+            sc.voxelize([ms], grid, stream=stream)
+            ctx.sync(stream)
+            assert sc.stats().work_items < 100
+        if textured:
+            uv = np.random.default_rng(3).uniform(0, 1, (pos.size // 3, 2)).astype(np.float32)
+            tex = np.random.default_rng(4).integers(0, 256, (8, 8, 4), dtype=np.uint8)
+            mesh = vgi.MeshData(ctx, pos.reshape(-1, 3), texcoords=uv, texture=tex)
+            ref, _ = orc.voxelize_textured(pos, grid_d, uv, tex)
+        else:
+            mesh = vgi.MeshData(ctx, pos.reshape(-1, 3), albedo=alb)
+            ref, _ = orc.voxelize(pos, grid_d, albedo=alb)
+        sc.voxelize([mesh], grid, stream=stream)
+        ctx.sync(stream)
+        assert sc.stats().voxelize_fallback == 1
+        acc = sc.read_voxels()
+        assert np.array_equal(acc, ref), _diff_msg(acc, ref)
+    finally:
+        sc.release()
+        ctx.stream_destroy(stream)
+
+
 def test_voxelize_returns_without_waiting(ctx):
     """vgi_voxelize enqueues its kernels and returns: queued behind about 40 cone traces on
     the same stream, the call comes back while the stream is still busy and in a small
