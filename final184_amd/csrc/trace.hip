@@ -558,6 +558,7 @@ __device__ __forceinline__ float4 cone_march_shared(const TraceParams& P, bool f
   const float uoz = cone_origin(oz, P.origin[2], P.inv_h), udz = dz * P.inv_h;
   const float h = P.h, inv_h = P.inv_h, step = P.step, cutoff = P.cutoff, max_dist = P.max_dist;
   const uint32_t n = fixed ? __builtin_amdgcn_readfirstlane(P.sched_len[1]) : (uint32_t)VGI_MAX_MARCH_STEPS;
+  if (n == 0u) return make_float4(0.f, 0.f, 0.f, 0.f);  // no entry to load (the same in every wavefront)
   for (uint32_t it = 0, half = 0;; it += nw, half ^= nw) {
     bool in = alive && it + wave < n;
     uint32_t taken = 0;

@@ -675,6 +675,31 @@ def test_cone_counts_vs_fp64(ctx, soup, num_diffuse, specular):
     f.release()
 
 
+@pytest.mark.parametrize("batch", [1, 3])
+@pytest.mark.parametrize("prec", ["fp32", "fp16x2"])
+def test_cones_that_start_past_their_end(ctx, soup, prec, batch):
+    """Cones whose first sample lies beyond the maximum distance have no schedule entry: a
+    launch of few blocks, whose wavefronts march the specular cone together, gives what a
+    large one does, nothing gathered and full visibility."""
+    vgi = _vgi()
+    w = soup["w"]
+    print(f"case empty schedules {prec} x{batch}", flush=True)
+    f = Frame(ctx, w, prec)
+    h = w.grid["extent"] / w.grid["n"]
+    cones = vgi.make_cones(**dict(w.cones, start_offset=3.0, max_distance=2.0 * h))
+    n = 61 * 13
+    gb = vgi.GBufferData(ctx, w.gb_pos[:n], w.gb_nrm[:n], 61, 13)
+    outs = [(vgi.DeviceArray.empty(ctx, (n, 4), np.float32), vgi.DeviceArray.empty(ctx, (n, 4), np.float32))
+            for _ in range(batch)]
+    ctx.trace_batch([(f.scene, gb, cones, od, os) for od, os in outs])
+    f.scene.trace(f.gb, cones, f.od, f.os)
+    want_d, want_s = f.od.numpy()[:n], f.os.numpy()[:n]
+    assert not want_s.any() and not want_d[:, :3].any() and (want_d[:, 3] == 1.0).all()
+    for od, os in outs:
+        assert np.array_equal(od.numpy(), want_d) and np.array_equal(os.numpy(), want_s)
+    f.release()
+
+
 @pytest.mark.parametrize("meshes", [1, 120])
 def test_queued_calls_keep_their_descriptors(ctx, soup, meshes):
     """Thirty frames queued without waiting, each with its own lights, eye and mesh split (more
