@@ -420,9 +420,7 @@ int recorded_room(vgi_workspace* w, size_t bytes) {
 // them to the stream's recorded block each time it runs, so that graphs recorded on one stream
 // share that block (their runs have to be ordered) and none outlives its tables.
 template <class F, class L>
-int stage_descriptors(vgi_workspace* w, UploadSite site, size_t bytes, F&& fill, L&& launch) {
-  bool captured = false;
-  TRY(stream_capturing(w->stream, &captured));
+int stage_descriptors(vgi_workspace* w, bool captured, UploadSite site, size_t bytes, F&& fill, L&& launch) {
   if (captured) {
     TRY(recorded_room(w, bytes));
     Slot s;
@@ -684,6 +682,8 @@ int voxelize_batch(vgi_context* ctx, const vgi_voxelize_item* items, uint32_t co
   vgi_workspace* w = workspace(ctx, st);
   if (!w) return fail(VGI_E_HIP, "workspace creation failed");
   std::lock_guard<std::mutex> wl(w->mu);
+  bool captured = false;
+  TRY(stream_capturing(st, &captured));
 
   for (VoxPlan& p : plan) {
     p.s->has_voxels = false;
@@ -834,7 +834,7 @@ int voxelize_batch(vgi_context* ctx, const vgi_voxelize_item* items, uint32_t co
     return launch_voxelize_kernels(ctx, B, stage, zb, zeroed_need, nblk_t, nblk_b, ts, grid_blocks, big_blocks,
                                    zero_blocks, scs.data(), count, st, ctx->profiling != 0);
   };
-  TRY(stage_descriptors(w, kSiteVoxelize, cv.off, fill, launch));
+  TRY(stage_descriptors(w, captured, kSiteVoxelize, cv.off, fill, launch));
   for (uint32_t i = 0; i < count; i++) {
     vgi_scene* s = plan[i].s;
     s->grid = items[i].grid;
@@ -1097,7 +1097,7 @@ int mips_batch(vgi_context* ctx, const vgi_mips_item* items, uint32_t count, uin
     }
     return VGI_OK;
   };
-  TRY(stage_descriptors(w, kSiteMips, cv.off, fill, launch));
+  TRY(stage_descriptors(w, captured, kSiteMips, cv.off, fill, launch));
   for (uint32_t i = 0; i < count; i++) {
     items[i].scene->prec = precision;
     items[i].scene->has_mips = true;
@@ -1391,7 +1391,7 @@ int trace_batch(vgi_context* ctx, const vgi_trace_item* items, uint32_t count, v
     }
     return VGI_OK;
   };
-  TRY(stage_descriptors(w, kSiteTrace, cv.off, fill, launch));
+  TRY(stage_descriptors(w, captured, kSiteTrace, cv.off, fill, launch));
   return VGI_OK;
 }
 
