@@ -557,10 +557,11 @@ def _counter_rows(outdir):
 # take the launches of that precision; the voxelize-front-end keys take the last frame
 # (FP32), whose front end is identical to the FP16 frame's.
 COUNTER_KERNELS = [
-    ("trace_fp16", r"k_trace<1\b"), ("trace_fp32", r"k_trace<0\b"), ("trace_fp16x2", r"k_trace<3\b"),
-    ("mips_fp16_first", r"k_mips<1, true, false>"), ("mips_fp16_rest", r"k_mips<1, false, false>"),
-    ("mips_fp32_first", r"k_mips<0, true, false>"), ("mips_fp32_rest", r"k_mips<0, false, false>"),
-    ("mips_fp16x2_first", r"k_mips<3, true, false>"), ("mips_fp16x2_rest", r"k_mips<3, false, false>"),
+    ("trace_fp16", r"k_trace(_one)?<1\b"), ("trace_fp32", r"k_trace(_one)?<0\b"),
+    ("trace_fp16x2", r"k_trace(_one)?<3\b"),
+    ("mips_fp16_first", r"k_mips<1, true, 0>"), ("mips_fp16_rest", r"k_mips<1, false, 0>"),
+    ("mips_fp32_first", r"k_mips<0, true, 0>"), ("mips_fp32_rest", r"k_mips<0, false, 0>"),
+    ("mips_fp16x2_first", r"k_mips<3, true, 0>"), ("mips_fp16x2_rest", r"k_mips<3, false, 0>"),
     ("setup", r"k_setup\b"), ("voxelize", r"k_voxelize<8, false>"),
     ("probe_fma", r"k_probe_fma"), ("probe_int", r"k_probe_int"), ("probe_atomic_ret", r"k_probe_atomic<true>"),
     ("probe_atomic_noret", r"k_probe_atomic<false>"), ("copy", r"k_copy\b"),
