@@ -800,7 +800,7 @@ def main() -> int:
         "shadowed_mips": {"lights": f"the workload's {len(w.lights)} lights casting shadows",
                           "mip_storage": head["prec"], "mips_ms": shadow_ms["shadowed"],
                           "plain_mips_ms": shadow_ms["plain"],
-                          "note": "visibility walks through the level-0 occupancy inside the injecting launch"},
+                          "note": "visibility walks through the level-0 occupancy in a launch of their own before the injecting one"},
         "trilinear_per_pixel": head["trilinear"] / px,
         "tuning": tuned.as_dict() if tuned is not None else
                   {"bin_size": args.bin, "schedule": args.order if args.order == "morton" else args.tile},

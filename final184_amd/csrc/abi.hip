@@ -623,7 +623,7 @@ int launch_voxelize_kernels(vgi_context* ctx, const VoxBatch& B, const StageArgs
   HIP_TRY(launch_big_count(B, persistent, st));
   if (prof) HIP_TRY(hipEventRecord(ctx->ev[1], st));
   HIP_TRY(launch_bins(B, (uint32_t)nblk_b, st));
-  for (uint32_t i = 0; i < count; i++) scenes[i]->vox_seq = B.seq;  // k_scatter stores it
+  for (uint32_t i = 0; i < count; i++) scenes[i]->vox_seq = B.seq;  // k_voxelize's last workgroup stores it
   if (prof) HIP_TRY(hipEventRecord(ctx->ev[2], st));
   HIP_TRY(launch_scatter(B, (uint32_t)nblk_b, (uint32_t)nblk_t, big_blocks, zero_blocks, st));
   if (prof) HIP_TRY(hipEventRecord(ctx->ev[3], st));

@@ -27,8 +27,10 @@ namespace vgi {
 // scattered pixels in tile order (room and soup, 1636 x 1504, 4 + 1 cones, one / two
 // wavefronts: BF16 618 / 628 us and 4.62 / 4.93 ms, FP16 601 / 599 and 4.60 / 4.77, x-pair
 // 500 / 509 and 4.82 / 5.14; room, 1920 x 1080, 9 + 1: 910 / 905, 891 / 874, 726 / 720),
-// while at 1280 x 720 it is worth 5% (BF16 454 / 433). FP32 gains at every size (room at
-// 1080p 878 / 818).
+// while at 1280 x 720 it is worth 5% (BF16 454 / 433). FP32 gains more by it (whole calls, a
+// room at 1080p, 9 + 1 cones, 892 / 802; 1636 x 1504, 4 + 1, 606 / 561), and loses up to 6% on
+// scattered pixels (soup, 256^3, 1636 x 1504, 4 + 1 cones, 2000 triangles 7.05 / 7.45 ms, 20000
+// 10.45 / 10.69; 9 + 1, 20000, 16.73 / 16.68): what kind a G-buffer is the launch does not know.
 constexpr uint64_t kOneTraceBlocks = 24000;
 constexpr uint64_t kManyTraceBlocks = 12000;
 // From here a launch fills the chip (k_trace's registers: trace_waves).

@@ -248,8 +248,8 @@ __global__ __launch_bounds__(256) void k_blur(vgi_blur_params p, uint32_t ntx, u
 
   // All of a thread's loads are issued before the first is waited for: one round trip to
   // memory a workgroup instead of eight along y, three along x (with the
-  // exp2 above, all four screen passes: 1080p FP16 71.9 -> 68.1 us, 4K 265 -> 247, 643 x 361
-  // FP32 22.4 -> 20.4).
+  // exp2 above, all four screen passes: 1080p FP16 72.0 -> 68.5 us, 4K 265 -> 247; at 643 x 361
+  // FP32, 22 us, no more than two runs differ by).
   constexpr int kStage = (T::LX * T::LY + 255) / 256;
   typename Raw<IN_HALF>::type raw[kStage];
   float depth[kStage];

@@ -726,7 +726,7 @@ constexpr int trace_waves(int prec, bool full) { return prec == VGI_PREC_FP32 &&
 // launch (96 x 54 pixels, 9 + 1 cones: 104 us, 47 with three wavefronts), and of a large
 // launch keeps twice the blocks resident per CU, whose footprints share its L1 (1280 x 720:
 // FP32 439 -> 388 us, FP16 436 -> 410, BF16 470 -> 427, FP16 x-pair 364 -> 341).
-// SHARED (a launch of few blocks): all wavefronts, up to sixteen, first march the specular
+// SHARED (a launch of few blocks): all wavefronts, twelve at most, first march the specular
 // cone together (cone_march_shared), whose chain of samples sets the length of such a
 // launch, then take the diffuse cones as above.
 template <int PREC, bool BUF, bool SORTED, bool FULL, bool SHARED>
@@ -820,7 +820,7 @@ void k_trace(TraceBatch Bt, const TraceParams* __restrict__ scenes, const uint2*
 
 // A wavefront for each 8x8 block, marching every cone in turn with the block's frames in
 // registers: for launches of many blocks, where sharing gains a camera's G-buffer little
-// and costs scattered ones 3-7% (the host's kOneTraceBlocks).
+// and costs scattered ones 3-7% (kOneTraceBlocks).
 template <int PREC>
 __global__ __launch_bounds__(64) void k_trace_one(TraceBatch Bt, const TraceParams* __restrict__ scenes,
                                                   const uint2* __restrict__ blocks) {
