@@ -186,6 +186,45 @@ def test_recorded_trace_on_a_fresh_stream(ctx):
         ctx.stream_destroy(stream)
 
 
+def test_recorded_batch_build_replays(ctx):
+    """A recorded batch of builds carries its block tables too: three scenes, one of them with a
+    shadow-casting light, of which eager single builds run between the replays."""
+    vgi = _vgi()
+    print("case recorded batch of mips", flush=True)
+    soups = Soups(ctx, 64, 7)
+    w = soups.w
+    lights = [w.lights, [dict(w.lights[0], shadow=True)], w.lights]
+    ref = [[orc.inject_mips(a, w.grid, ls, "fp16") for ls in lights] for a in soups.acc]
+    stream, scs = ctx.stream_create(), [ctx.scene() for _ in lights]
+    try:
+        jobs = [(sc, vgi.make_lights(ls)) for sc, ls in zip(scs, lights)]
+        for sc in scs:
+            sc.voxelize([soups.mesh], soups.grid, stream)
+        ctx.build_mips_batch(jobs, vgi.PREC_FP16, stream)
+
+        def voxels():
+            for sc in scs:
+                sc.voxelize_noalloc([soups.mesh], soups.grid, stream)
+
+        g = Recorded(stream, lambda: (voxels(), ctx.build_mips_batch(jobs, vgi.PREC_FP16, stream)))
+        for step, (i, eager) in enumerate(((0, 0), (0, 0), (1, 0), (2, 1), (0, 0), (1, 1), (2, 0))):
+            soups.put(ctx, i)
+            if eager:
+                voxels()
+                for sc, ls in jobs:
+                    sc.build_mips(ls, vgi.PREC_FP16, stream)
+            else:
+                g.replay()
+            ctx.sync(stream)
+            for k, sc in enumerate(scs):
+                _assert_levels(sc, ref[i][k], f"step {step}, {'eager' if eager else 'replay'}, soup {i}, scene {k}")
+        g.release()
+    finally:
+        for sc in scs:
+            sc.release()
+        ctx.stream_destroy(stream)
+
+
 def test_recorded_build_with_shadow_lights(ctx):
     """A recorded build with shadow-casting lights holds nothing of the stream's scratch: an
     eager build of a larger grid replaces that scratch between the replays."""
