@@ -68,6 +68,7 @@ int fail(int code, const char* fmt, ...) {
   } while (0)
 
 bool is_pow2(uint32_t v) { return v && !(v & (v - 1)); }
+
 // Most answer bytes of visibility walks that a stream keeps: one scene of 512^3 with up to 16
 // shadow-casting lights (285 MB), or nine of 256^3 with 16.
 constexpr size_t kMaxVisBytes = 320u << 20;
@@ -954,8 +955,9 @@ int mips_batch(vgi_context* ctx, const vgi_mips_item* items, uint32_t count, uin
   size_t total_lights = 0;
   // Builds with shadow-casting lights: where every scene has at most 32 and the stream holds
   // or can get an answer byte a voxel per eight of them, up to kMaxVisBytes, k_visibility walks
-  // before the injecting launch; otherwise that launch walks by itself. So it does in a build recorded in a graph,
-  // which may run when a larger build has replaced the stream's answer bytes.
+  // before the injecting launch; otherwise that launch walks by itself. So it does in a build
+  // recorded in a graph, which may run when a larger build has replaced the stream's answer
+  // bytes.
   bool shadow = false, vis = true;
   size_t vis_need = 0;
   std::vector<size_t> vis_off(count);
